@@ -102,6 +102,11 @@ struct GroupDev {
     // frame data, frameH x fframeW column-contiguous
     const void *img;
     int imgType, vec;
+    // A thread's run of rows is the L lines of one image column of an affine
+    // block, in whole aligned chunks of 8, the gradients are derived or BF16,
+    // and 32-bit byte offsets address the template: the pixel kernels' loops
+    // without per-pixel geometry, tails or 64-bit addresses.
+    int fast;
     const int *minPts;
     // state
     double *p, *pLast, *p0, *d0, *deltaP, *errval;

@@ -764,6 +764,10 @@ ss_status setup_group(ss_handle *h, Plan &P, char *D, char *HS, ss::GroupDev &g,
     }
     // chunks of rows start 16-byte aligned when the columns do
     g.vec = ((fh % 8) == 0 && (g.runLen % 8) == 0 && ((uintptr_t)g.img % 16) == 0) ? 1 : 0;
+    g.fast = (g.vec && g.affine && g.runLen == g.L && g.tw < (1 << 20) && g.th < (1 << 20) &&
+              (size_t)g.th * g.tw * sizeof(double2) < ((size_t)1 << 32))
+                 ? 1
+                 : 0;
     // min points (first n_blocks entries are read: minPointsPerBlock[c % frameW])
     HIPCHK(up(P.oMin, in.min_points, nb * sizeof(int)));
     g.minPts = (const int *)dptr(P.oMin);

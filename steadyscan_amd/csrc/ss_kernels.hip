@@ -13,13 +13,22 @@
 // and end the groups that stopped.
 //
 // Pixel work: one workgroup (4 wave64) per line-block column (frame f,
-// block b = column c = f * nb + b of the block matrix).  The column is cut
-// into chunks of 8 rows dealt round-robin to the threads, so a wave reads
-// 64 consecutive chunks (fully coalesced 16-byte loads) and, since a block
-// lists its pixels column by column, neighbouring lanes sit on neighbouring
-// scan-line pixels: a wave's template gathers touch a few cache lines.  Per-column partial sums are reduced in registers, then
-// across waves through LDS in FP64.  No floating-point atomics: every result
-// is run-to-run deterministic.
+// block b = column c = f * nb + b of the block matrix).  A thread walks runs
+// of rows, the lines of one image column of the block, so that neighbouring
+// lanes sit on neighbouring scan-line pixels and a wave's template gathers
+// touch a few cache lines; frame values come 8 rows at a time in 16-byte
+// loads.  A chunk of rows computes its coordinates, issues all its gathers,
+// and only then does the arithmetic (sched_fence, pin): left to itself the
+// compiler put every sample's gathers under the branch that discards
+// unmasked samples, with a wait each.  Per-column partial sums are reduced
+// in registers, then across waves through LDS in FP64.  No floating-point
+// atomics: every result is run-to-run deterministic.
+// What bounds them (1000 x 512x512 uint16, FP64): VALU issue, 67-82% of the
+// cycles, next to the L1's 64 bytes a cycle for the gathers.  Global instead
+// of flat loads, batched gathers, scalar loads of the group's description,
+// line-constant geometry and lane-swap reductions took the full batch's
+// first assembly launch from 1269 to 729 us, a line-search launch from 342
+// to 193 us and a correlation launch from 624 to 325 us on average.
 #include "ss_device.h"
 #include "ss_tuning.h"
 
@@ -31,6 +40,16 @@ constexpr int kWG = 256;       // pixel kernels
 constexpr int kSolveWG = 256;  // per-group kernels
 constexpr int kCH = 8;         // pixels per unrolled chunk
 
+// Everything a group points to is device memory.  Saying so (address space
+// 1) makes the pixel loads global loads; through the generic pointers of
+// GroupDev they would be flat loads, which also wait for LDS and cannot be
+// counted apart, so that every use waits for all loads in flight.  What no
+// kernel of the launch writes (address space 4) is read by scalar loads.
+#define SS_GLOBAL __attribute__((address_space(1)))
+#define SS_CONST __attribute__((address_space(4)))
+// a group's description in the pixel kernels, which do not write it
+using GroupRef = const SS_CONST GroupDev &;
+
 // ---------------------------------------------------------------------------
 // precision: pixel arithmetic in R = float (precision 'S') or double ('D');
 // every reduction is FP64 in both
@@ -39,25 +58,21 @@ template <typename R>
 struct Prec;
 template <>
 struct Prec<float> {
-    using V2 = float2;
-    using V4 = float4;
-    static __device__ __forceinline__ const AffineGeo<float> &aff(const GroupDev &g) { return g.afF; }
-    static __device__ __forceinline__ const float4 *geo(const GroupDev &g) { return g.geo; }
-    static __device__ __forceinline__ const float *fnext(const GroupDev &g) { return g.fnext; }
-    static __device__ __forceinline__ const float2 *tp(const GroupDev &g) { return g.tp; }
-    static __device__ __forceinline__ const float2 *gxv(const GroupDev &g) { return g.gxv; }
-    static __device__ __forceinline__ const float2 *gyh(const GroupDev &g) { return g.gyh; }
+    static __device__ __forceinline__ const SS_CONST AffineGeo<float> &aff(GroupRef g) { return g.afF; }
+    static __device__ __forceinline__ const float4 *geo(GroupRef g) { return g.geo; }
+    static __device__ __forceinline__ const float *fnext(GroupRef g) { return g.fnext; }
+    static __device__ __forceinline__ const float2 *tp(GroupRef g) { return g.tp; }
+    static __device__ __forceinline__ const float2 *gxv(GroupRef g) { return g.gxv; }
+    static __device__ __forceinline__ const float2 *gyh(GroupRef g) { return g.gyh; }
 };
 template <>
 struct Prec<double> {
-    using V2 = double2;
-    using V4 = double4;
-    static __device__ __forceinline__ const AffineGeo<double> &aff(const GroupDev &g) { return g.afD; }
-    static __device__ __forceinline__ const double4 *geo(const GroupDev &g) { return g.geoD; }
-    static __device__ __forceinline__ const double *fnext(const GroupDev &g) { return g.fnextD; }
-    static __device__ __forceinline__ const double2 *tp(const GroupDev &g) { return g.tpD; }
-    static __device__ __forceinline__ const double2 *gxv(const GroupDev &g) { return g.gxvD; }
-    static __device__ __forceinline__ const double2 *gyh(const GroupDev &g) { return g.gyhD; }
+    static __device__ __forceinline__ const SS_CONST AffineGeo<double> &aff(GroupRef g) { return g.afD; }
+    static __device__ __forceinline__ const double4 *geo(GroupRef g) { return g.geoD; }
+    static __device__ __forceinline__ const double *fnext(GroupRef g) { return g.fnextD; }
+    static __device__ __forceinline__ const double2 *tp(GroupRef g) { return g.tpD; }
+    static __device__ __forceinline__ const double2 *gxv(GroupRef g) { return g.gxvD; }
+    static __device__ __forceinline__ const double2 *gyh(GroupRef g) { return g.gyhD; }
 };
 
 __device__ __forceinline__ float mad(float a, float b, float c) { return fmaf(a, b, c); }
@@ -72,95 +87,105 @@ __host__ __device__ constexpr int img_type() {
 }
 // true when group g runs in the instantiation <TI, R>
 template <typename TI, typename R>
-__device__ __forceinline__ bool runs_here(const GroupDev &g) {
+__device__ __forceinline__ bool runs_here(GroupRef g) {
     return g.imgType == img_type<TI>() && g.fp64 == (sizeof(R) == 8 ? 1 : 0);
 }
 
 // ---------------------------------------------------------------------------
 // helpers
 // ---------------------------------------------------------------------------
-template <typename R>
-__device__ __forceinline__ void load8(const float *p, bool vec, int n, R (&v)[kCH]) {
-    if (vec && n >= kCH) {
-        const float4 a = *reinterpret_cast<const float4 *>(p);
-        const float4 b = *reinterpret_cast<const float4 *>(p + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-#pragma unroll
-        for (int i = 0; i < kCH; i++) v[i] = i < n ? (R)p[i] : (R)0;
-    }
+template <typename T>
+__device__ __forceinline__ const SS_GLOBAL T *as_global(const T *p) {
+    return (const SS_GLOBAL T *)p;
 }
-template <typename R>
-__device__ __forceinline__ void load8(const double *p, bool vec, int n, R (&v)[kCH]) {
-    if (vec && n >= kCH) {
-#pragma unroll
-        for (int i = 0; i < kCH / 2; i++) {
-            const double2 a = *reinterpret_cast<const double2 *>(p + 2 * i);
-            v[2 * i] = (R)a.x;
-            v[2 * i + 1] = (R)a.y;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kCH; i++) v[i] = i < n ? (R)p[i] : (R)0;
-    }
+template <typename T>
+__device__ __forceinline__ const SS_CONST T *as_const(const T *p) {
+    return (const SS_CONST T *)p;
 }
+__device__ __forceinline__ GroupRef group_of(const Batch &B, int gi) { return as_const(B.groups)[gi]; }
+
+// native vectors: their loads keep the pointer's address space
+using f2v = float __attribute__((ext_vector_type(2)));
+using f4v = float __attribute__((ext_vector_type(4)));
+using d2v = double __attribute__((ext_vector_type(2)));
+using d4v = double __attribute__((ext_vector_type(4)));
+using u4v = uint32_t __attribute__((ext_vector_type(4)));
 template <typename R>
-__device__ __forceinline__ void load8(const uint16_t *p, bool vec, int n, R (&v)[kCH]) {
-    if (vec && n >= kCH) {
-        const uint4 a = *reinterpret_cast<const uint4 *>(p);
-        const unsigned w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            v[2 * i] = (R)(w[i] & 0xffffu);
-            v[2 * i + 1] = (R)(w[i] >> 16);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kCH; i++) v[i] = i < n ? (R)p[i] : (R)0;
-    }
+struct Nat {
+    using V2 = f2v;
+    using V4 = f4v;
+};
+template <>
+struct Nat<double> {
+    using V2 = d2v;
+    using V4 = d4v;
+};
+
+// The scheduler moves nothing across: the loads of a chunk stay ahead of
+// the arithmetic that uses them.
+__device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
+// A value the compiler must have at this point: an expression that is only
+// selected afterwards (cond ? v : 0) is otherwise moved under a branch
+// together with its loads, one wait per sample.
+__device__ __forceinline__ void pin(float &v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void pin(double &v) { asm volatile("" : "+v"(v)); }
+// A wave-uniform value kept in scalar registers.
+__device__ __forceinline__ float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
-template <typename R>
-__device__ __forceinline__ void load8(const int16_t *p, bool vec, int n, R (&v)[kCH]) {
-    if (vec && n >= kCH) {
-        const uint4 a = *reinterpret_cast<const uint4 *>(p);
-        const unsigned w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            v[2 * i] = (R)(int16_t)(w[i] & 0xffffu);
-            v[2 * i + 1] = (R)((int)w[i] >> 16);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kCH; i++) v[i] = i < n ? (R)p[i] : (R)0;
-    }
+__device__ __forceinline__ double uniform(double v) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// CH consecutive frame values from p (16-byte loads when the chunk is
-// aligned, i.e. vec and a full chunk); values past n read as 0.
-template <int CH, typename TI>
-struct alignas(CH * sizeof(TI) >= 16 ? 16 : CH * sizeof(TI)) Pack {
-    TI v[CH];
-};
-template <int CH, typename TI, typename R>
-__device__ __forceinline__ void load_chunk(const TI *p, bool vec, int n, R (&v)[CH]) {
-    if constexpr (CH == kCH) {
-        load8(p, vec, n, v);
-    } else {
-        if (vec && n >= CH) {
-            constexpr int per = (CH * (int)sizeof(TI) <= 16) ? CH : 16 / (int)sizeof(TI);
+// Truncation towards zero, saturated at the int range, 0 for NaN (the
+// instruction's own behaviour; the C conversion leaves these undefined).
+__device__ __forceinline__ int trunc_int(float v) {
+    int r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+__device__ __forceinline__ int trunc_int(double v) {
+    int r;
+    asm("v_cvt_i32_f64 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+__device__ __forceinline__ float fraction(float v) { return __builtin_amdgcn_fractf(v); }
+__device__ __forceinline__ double fraction(double v) { return __builtin_amdgcn_fract(v); }
+
+// kCH consecutive frame values: in raw form (16-byte loads, four registers
+// for 16-bit frames) when the rows are aligned, converted when used.
+template <typename TI>
+struct Rows8 {
+    static constexpr int kVec = kCH * (int)sizeof(TI) / 16;
+    u4v q[kVec];
+    __device__ __forceinline__ void load(const SS_GLOBAL TI *p) {
+        const SS_GLOBAL u4v *v = (const SS_GLOBAL u4v *)p;
 #pragma unroll
-            for (int j = 0; j < CH / per; j++) {
-                const Pack<per, TI> q = *reinterpret_cast<const Pack<per, TI> *>(p + j * per);
+        for (int i = 0; i < kVec; i++) q[i] = v[i];
+    }
+    // rows past n read as 0
+    __device__ __forceinline__ void load_ragged(const SS_GLOBAL TI *p, int n) {
+        TI v[kCH];
 #pragma unroll
-                for (int i = 0; i < per; i++) v[j * per + i] = (R)q.v[i];
-            }
+        for (int i = 0; i < kCH; i++) v[i] = i < n ? p[i] : (TI)0;
+        __builtin_memcpy(q, v, sizeof(q));
+    }
+    template <typename R>
+    __device__ __forceinline__ R at(int i) const {
+        if constexpr (sizeof(TI) == 2) {
+            const uint32_t w = q[0][i >> 1];
+            if constexpr (std::is_same<TI, uint16_t>::value) return (R)((i & 1) ? w >> 16 : w & 0xffffu);
+            else return (R)((i & 1) ? (int)w >> 16 : (int)(int16_t)(w & 0xffffu));
+        } else if constexpr (sizeof(TI) == 4) {
+            return (R)__uint_as_float(q[i >> 2][i & 3]);
         } else {
-#pragma unroll
-            for (int i = 0; i < CH; i++) v[i] = i < n ? (R)p[i] : (R)0;
+            const uint32_t lo = q[i >> 1][2 * (i & 1)], hi = q[i >> 1][2 * (i & 1) + 1];
+            return (R)__longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
         }
     }
-}
+};
 
 // Rows per chunk: enough independent template gathers per wave to hide
 // their latency, few enough that the unrolled chunk stays in registers
@@ -171,22 +196,58 @@ __host__ __device__ constexpr int chunk_rows(int samplesPerRow, int budget) {
     return c < 1 ? 1 : (c > kCH ? kCH : c);
 }
 
+// Wave sums of NV per-thread doubles without LDS: two lane-swap steps that
+// each add the halves of two values at once (lanes 32 apart, then 16 apart),
+// then DPP row shifts by 8, 4, 2, 1.  Every value is added in the order
+// ((l + l+32) + (l+16 + l+48)) ..., as a shuffle-down tree adds it; value i's
+// sum ends in lane 16 * row(i & 3) of register i >> 2, rows 0 2 1 3.  (A
+// column's 19 assembly sums were 228 LDS shuffles a wave and a chain of six
+// LDS round trips.)
+__device__ __forceinline__ void swap_add(double a, double b, double &out, bool half) {
+    const long long ba = __double_as_longlong(a), bb = __double_as_longlong(b);
+    const auto lo = half ? __builtin_amdgcn_permlane32_swap((int)ba, (int)bb, false, false)
+                         : __builtin_amdgcn_permlane16_swap((int)ba, (int)bb, false, false);
+    const auto hi = half ? __builtin_amdgcn_permlane32_swap((int)(ba >> 32), (int)(bb >> 32), false, false)
+                         : __builtin_amdgcn_permlane16_swap((int)(ba >> 32), (int)(bb >> 32), false, false);
+    const double x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+    const double y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+    out = x + y;
+}
+template <int CTRL>
+__device__ __forceinline__ double row_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return v + __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+template <int NV>
+__device__ __forceinline__ void wave_sums(const double (&v)[NV], double (&q)[(NV + 3) / 4]) {
+    constexpr int N2 = (NV + 1) / 2, N4 = (NV + 3) / 4;
+    double h[N2];
+#pragma unroll
+    for (int i = 0; i < N2; i++) swap_add(v[2 * i], 2 * i + 1 < NV ? v[2 * i + 1] : 0.0, h[i], true);
+#pragma unroll
+    for (int i = 0; i < N4; i++) {
+        swap_add(h[2 * i], 2 * i + 1 < N2 ? h[2 * i + 1] : 0.0, q[i], false);
+        q[i] = row_add<0x108>(q[i]);  // row_shl:8: lane l adds lane l + 8 of its row
+        q[i] = row_add<0x104>(q[i]);
+        q[i] = row_add<0x102>(q[i]);
+        q[i] = row_add<0x101>(q[i]);
+    }
+}
+
 // Sum over the workgroup of NV per-thread doubles; thread i < NV gets sum i
 // in out (LDS-backed, returns after a barrier).
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double *out) {
-    __shared__ double sh[kWG / 64][NV];
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-        double x = v[i];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-        v[i] = x;
-    }
+    __shared__ double sh[kWG / 64][(NV + 3) / 4 * 4];
+    double q[(NV + 3) / 4];
+    wave_sums<NV>(v, q);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) {
+    if ((lane & 15) == 0) {
+        const int row = lane >> 4, which = ((row & 1) << 1) | (row >> 1);
 #pragma unroll
-        for (int i = 0; i < NV; i++) sh[wave][i] = v[i];
+        for (int i = 0; i < (NV + 3) / 4; i++) sh[wave][4 * i + which] = q[i];
     }
     __syncthreads();
     if (threadIdx.x < NV) {
@@ -217,135 +278,195 @@ __device__ __forceinline__ double reduce_pow(double v, double r, int k) {
     return v;
 }
 
-// Geometry of the pixels of one thread segment: affine in the block's
+// Geometry of the pixels of one thread's run of rows: affine in the block's
 // (column j, line i) coordinates -- the block matrix lists a block's pixels
 // column-major, row r = j * L + i -- or read from the per-pixel table.
-template <typename R>
-struct GeoIter {
-    R fj, fi, Lf, byb;
-    __device__ __forceinline__ void start(const GroupDev &g, int b, int r0) {
-        if (g.affine) {
-            const AffineGeo<R> &a = Prec<R>::aff(g);
-            const int j = r0 / g.L;
-            fj = (R)j;
-            fi = (R)(r0 - j * g.L);
-            Lf = (R)g.L;
-            byb = a.gy0 + a.gyb * (R)b;
+// FAST (see GroupDev::fast): a run is one image column's L lines, so j is
+// fixed and i counts the rows.
+template <typename R, bool FAST>
+struct GeoRun {
+    const SS_CONST AffineGeo<R> &a;
+    R byb, fj, fi, Lf, f0, x0, y0;
+    int affine, L;
+    const SS_GLOBAL typename Nat<R>::V4 *tab;
+    __device__ __forceinline__ GeoRun(GroupRef g, int b) : a(Prec<R>::aff(g)) {
+        affine = FAST ? 1 : g.affine;
+        L = g.L;
+        byb = a.gy0 + a.gyb * (R)b;
+        if constexpr (!FAST) {
+            tab = (const SS_GLOBAL typename Nat<R>::V4 *)Prec<R>::geo(g) + (size_t)b * g.frameH;
+            Lf = (R)L;
         }
     }
-    __device__ __forceinline__ void at(const GroupDev &g, const typename Prec<R>::V4 *geo, int r, R &bx,
-                                       R &by, R &f, bool &m) const {
-        if (g.affine) {
-            const AffineGeo<R> &a = Prec<R>::aff(g);
-            f = mad(a.fi, fi, mad(a.fj, fj, a.f0));
-            bx = mad(a.gxi, fi, mad(a.gxj, fj, a.gx0));
-            by = mad(a.gyi, fi, mad(a.gyj, fj, byb));
-            m = true;
+    __device__ __forceinline__ void start(int run, int r0) {
+        fi = (R)0;
+        if constexpr (FAST) {
+            set_column((R)run);
+        } else if (affine) {
+            const int j = r0 / L;
+            fi = (R)(r0 - j * L);
+            set_column((R)j);
+        }
+    }
+    __device__ __forceinline__ void set_column(R j) {
+        fj = j;
+        f0 = mad(a.fj, fj, a.f0);
+        x0 = mad(a.gxj, fj, a.gx0);
+        y0 = mad(a.gyj, fj, byb);
+    }
+    // the next CH rows, from row r on (rows past last repeat it)
+    template <int CH>
+    __device__ __forceinline__ void rows(int r, int last, R (&bx)[CH], R (&by)[CH], R (&f)[CH], bool (&m)[CH]) {
+        if (FAST || affine) {
+#pragma unroll
+            for (int k = 0; k < CH; k++) {
+                f[k] = mad(a.fi, fi, f0);
+                bx[k] = mad(a.gxi, fi, x0);
+                by[k] = mad(a.gyi, fi, y0);
+                m[k] = true;
+                fi += (R)1;
+                if constexpr (!FAST) {
+                    if (fi == Lf) {
+                        fi = (R)0;
+                        set_column(fj + (R)1);
+                    }
+                }
+            }
         } else {
-            const typename Prec<R>::V4 q = geo[r];
-            bx = q.x;
-            by = q.y;
-            f = q.z;
-            m = q.w != (R)0;
-        }
-    }
-    __device__ __forceinline__ void next() {
-        fi += (R)1;
-        if (fi == Lf) {
-            fi = (R)0;
-            fj += (R)1;
+#pragma unroll
+            for (int k = 0; k < CH; k++) {
+                const typename Nat<R>::V4 q = tab[min(r + k, last)];
+                bx[k] = q.x;
+                by[k] = q.y;
+                f[k] = q.z;
+                m[k] = q.w != (R)0;
+            }
         }
     }
 };
-
-template <typename R>
-__device__ __forceinline__ bool in_bounds(const GroupDev &g, R x, R y) {
-    // non-short-circuit: four compares combined without branches
-    return (x >= (R)0) & (x < (R)g.xmax) & (y >= (R)0) & (y < (R)g.ymax);
-}
 
 // Two BF16 values packed in 32 bits (low half first) as a float pair.
 __device__ __forceinline__ float2 bf16_pair(uint32_t u) {
     return make_float2(__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u));
 }
 
-// Bilinear template sample at (x, y) (task_differenceimage.cuh:13-32) from
-// the paired layout.  Branch-free: a point outside the mask reads cell 0 (the
-// caller discards the value), so a wave can issue all gathers of a chunk
-// before waiting on any.
+// Bilinear template samples (task_differenceimage.cuh:13-32) from the paired
+// layout.  A point outside the mask reads the nearest cell (the caller
+// discards the value), so a wave issues all gathers of a chunk before it
+// waits on any.  FAST addresses the template by 32-bit byte offsets.
 template <typename R>
-struct Cell {
+struct Tap {
     R fx, fy;
-    typename Prec<R>::V2 top, bot;
-    int t;
+    typename Nat<R>::V2 top, bot;
+    unsigned t;
 };
-template <typename R>
-__device__ __forceinline__ R sample(const GroupDev &g, R x, R y, bool valid, Cell<R> &cl) {
-    const R xs = valid ? x : (R)0, ys = valid ? y : (R)0;
-    const int ix = (int)xs, iy = (int)ys;
-    cl.fx = xs - (R)ix;
-    cl.fy = ys - (R)iy;
-    cl.t = iy * g.tw + ix;
-    const typename Prec<R>::V2 *tp = Prec<R>::tp(g);
-    cl.top = tp[cl.t];
-    cl.bot = tp[cl.t + g.tw];
-    const R a = mad(cl.fx, cl.top.y - cl.top.x, cl.top.x);
-    const R b = mad(cl.fx, cl.bot.y - cl.bot.x, cl.bot.x);
-    return mad(cl.fy, b - a, a);
-}
-
-// Template gradients at the sample of cl (task_updategradients.cu): from
-// the BF16 gradient pairs in mixed precision, else derived from the cell
-// corners when they are forward differences, else from the gradient pairs.
-template <typename R>
-__device__ __forceinline__ void gradients(const GroupDev &g, const Cell<R> &cl, R &wx, R &wy) {
-    if constexpr (sizeof(R) == 4) {
-        if (g.gradBF16) {  // pairs (G[t], G[t + step]) as two BF16 values
-            const float2 gx = bf16_pair(g.gxvB[cl.t]), gy = bf16_pair(g.gyhB[cl.t]);
-            wx = mad(cl.fy, gx.y - gx.x, gx.x);
-            wy = mad(cl.fx, gy.y - gy.x, gy.x);
-            return;
+template <typename R, bool FAST>
+struct Template {
+    const SS_GLOBAL char *row0, *row1;
+    int tw, xl, yl;
+    R xmax, ymax;
+    __device__ __forceinline__ explicit Template(GroupRef g) {
+        tw = g.tw;
+        xl = g.tw - 2;
+        yl = g.th - 2;
+        xmax = (R)g.xmax;
+        ymax = (R)g.ymax;
+        row0 = (const SS_GLOBAL char *)Prec<R>::tp(g);
+        row1 = row0 + (size_t)tw * sizeof(typename Nat<R>::V2);
+    }
+    __device__ __forceinline__ bool inside(R x, R y) const {
+        // non-short-circuit: four compares combined without branches
+        return (x >= (R)0) & (x < xmax) & (y >= (R)0) & (y < ymax);
+    }
+    __device__ __forceinline__ void fetch(R x, R y, Tap<R> &c) const {
+        using V2 = typename Nat<R>::V2;
+        const int ix = min(max(trunc_int(x), 0), xl), iy = min(max(trunc_int(y), 0), yl);
+        c.fx = fraction(x);
+        c.fy = fraction(y);
+        c.t = __umul24(iy, tw) + ix;
+        if constexpr (FAST) {
+            const unsigned o = c.t * (unsigned)sizeof(V2);
+            c.top = *(const SS_GLOBAL V2 *)(row0 + o);
+            c.bot = *(const SS_GLOBAL V2 *)(row1 + o);
+        } else {
+            const size_t o = (size_t)((long long)iy * tw + ix) * sizeof(V2);
+            c.t = (unsigned)(iy * tw + ix);
+            c.top = *(const SS_GLOBAL V2 *)(row0 + o);
+            c.bot = *(const SS_GLOBAL V2 *)(row1 + o);
         }
     }
-    if (g.gradFD) {
-        wx = mad(cl.fy, (cl.bot.y - cl.bot.x) - (cl.top.y - cl.top.x), cl.top.y - cl.top.x);
-        wy = mad(cl.fx, (cl.bot.y - cl.top.y) - (cl.bot.x - cl.top.x), cl.bot.x - cl.top.x);
-        return;
-    }
-    const typename Prec<R>::V2 gx = Prec<R>::gxv(g)[cl.t], gy = Prec<R>::gyh(g)[cl.t];
-    wx = mad(cl.fy, gx.y - gx.x, gx.x);
-    wy = mad(cl.fx, gy.y - gy.x, gy.x);
+};
+template <typename R>
+__device__ __forceinline__ R bilinear(const Tap<R> &c) {
+    const R a = mad(c.fx, c.top.y - c.top.x, c.top.x);
+    const R b = mad(c.fx, c.bot.y - c.bot.x, c.bot.x);
+    return mad(c.fy, b - a, a);
 }
+
+// Template gradients at a sample (task_updategradients.cu): derived from the
+// cell corners when they are forward differences, from the BF16 gradient
+// pairs in mixed precision, else from the gradient pairs.
+enum GradForm { GRAD_FD = 0, GRAD_PAIRS = 1, GRAD_BF16 = 2 };
+template <typename R, int GRAD>
+struct Grads {
+    typename Nat<R>::V2 gx, gy;
+    __device__ __forceinline__ void fetch(GroupRef g, const Tap<R> &c) {
+        if constexpr (GRAD == GRAD_PAIRS) {
+            gx = ((const SS_GLOBAL typename Nat<R>::V2 *)Prec<R>::gxv(g))[(size_t)c.t];
+            gy = ((const SS_GLOBAL typename Nat<R>::V2 *)Prec<R>::gyh(g))[(size_t)c.t];
+        }
+        if constexpr (GRAD == GRAD_BF16) {  // pairs (G[t], G[t + step]) as two BF16 values
+            gx.x = __uint_as_float(as_global(g.gxvB)[(size_t)c.t]);
+            gy.x = __uint_as_float(as_global(g.gyhB)[(size_t)c.t]);
+        }
+    }
+    __device__ __forceinline__ void eval(const Tap<R> &c, R &wx, R &wy) const {
+        if constexpr (GRAD == GRAD_FD) {
+            wx = mad(c.fy, (c.bot.y - c.bot.x) - (c.top.y - c.top.x), c.top.y - c.top.x);
+            wy = mad(c.fx, (c.bot.y - c.top.y) - (c.bot.x - c.top.x), c.bot.x - c.top.x);
+        } else if constexpr (GRAD == GRAD_BF16) {
+            const float2 p = bf16_pair(__float_as_uint(gx.x)), q = bf16_pair(__float_as_uint(gy.x));
+            wx = mad(c.fy, p.y - p.x, p.x);
+            wy = mad(c.fx, q.y - q.x, q.x);
+        } else {
+            wx = mad(c.fy, gx.y - gx.x, gx.x);
+            wy = mad(c.fx, gy.y - gy.x, gy.x);
+        }
+    }
+};
 
 // Knots of a column for candidate k of the line search (or the half-
 // iteration start state for k < 0), as x = base_x + a + d * frac.
 template <typename R>
 struct ColKnots {
     R ax, dx, ay, dy;
+    __device__ __forceinline__ R x(R bx, R f) const { return mad(dx, f, bx + ax); }
+    __device__ __forceinline__ R y(R by, R f) const { return mad(dy, f, by + ay); }
 };
 template <typename R>
 __device__ __forceinline__ ColKnots<R> make_knots(double lx, double rx, double ly, double ry) {
-    return ColKnots<R>{(R)lx, (R)(rx - lx), (R)ly, (R)(ry - ly)};
+    return ColKnots<R>{uniform((R)lx), uniform((R)(rx - lx)), uniform((R)ly), uniform((R)(ry - ly))};
 }
 template <typename R>
-__device__ __forceinline__ ColKnots<R> state_knots(const GroupDev &g, int c, int k) {
+__device__ __forceinline__ ColKnots<R> state_knots(GroupRef g, int c, int k) {
     const int N = g.N;
+    const SS_CONST double *p0 = as_const(g.p0), *d0 = as_const(g.d0);
     double lx, ly, rx, ry;
     if (k < 0) {  // half-iteration start: p0 with the real right knot
-        lx = g.p0[c];
-        ly = g.p0[c + N];
-        rx = g.p0[c + 1];
-        ry = g.p0[c + 1 + N];
+        lx = p0[c];
+        ly = p0[c + N];
+        rx = p0[c + 1];
+        ry = p0[c + 1 + N];
     } else {
         const double r = g.rmult;
-        lx = g.p0[c] + reduce_pow(g.d0[c], r, k);
-        ly = g.p0[c + N] + reduce_pow(g.d0[c + N], r, k);
+        lx = p0[c] + reduce_pow(d0[c], r, k);
+        ly = p0[c + N] + reduce_pow(d0[c + N], r, k);
         if (c + 1 == g.fframeW) {  // pnew of the group's last knot is never written
             rx = 1e6;
             ry = 1e6;
         } else {
-            rx = g.p0[c + 1] + reduce_pow(g.d0[c + 1], r, k);
-            ry = g.p0[c + 1 + N] + reduce_pow(g.d0[c + 1 + N], r, k);
+            rx = p0[c + 1] + reduce_pow(d0[c + 1], r, k);
+            ry = p0[c + 1 + N] + reduce_pow(d0[c + 1 + N], r, k);
         }
     }
     return make_knots<R>(lx, rx, ly, ry);
@@ -353,14 +474,37 @@ __device__ __forceinline__ ColKnots<R> state_knots(const GroupDev &g, int c, int
 
 // Knots of column c from the current parameter vector p (applyParameters on p).
 template <typename R>
-__device__ __forceinline__ ColKnots<R> current_knots(const GroupDev &g, int c) {
+__device__ __forceinline__ ColKnots<R> current_knots(GroupRef g, int c) {
     const int N = g.N;
-    return make_knots<R>(g.p[c], g.p[c + 1], g.p[c + N], g.p[c + 1 + N]);
+    const SS_CONST double *p = as_const(g.p);
+    return make_knots<R>(p[c], p[c + 1], p[c + N], p[c + 1 + N]);
 }
 
 template <typename TI>
-__device__ __forceinline__ const TI *column_ptr(const GroupDev &g, int c) {
-    return reinterpret_cast<const TI *>(g.img) + (size_t)c * g.frameH;
+__device__ __forceinline__ const SS_GLOBAL TI *column_ptr(GroupRef g, int c) {
+    return (const SS_GLOBAL TI *)g.img + (size_t)c * g.frameH;
+}
+
+// Walks a thread's rows of a column in chunks of CH: body(r, n, I, off) gets
+// the first row, the rows of the chunk inside the run (CH when FAST) and
+// the frame values (chunk row k is I.at(off + k)).
+template <int CH, bool FAST, typename TI, typename Start, typename Body>
+__device__ __forceinline__ void walk_rows(GroupRef g, const SS_GLOBAL TI *img, Start &&start, Body &&body) {
+    const int L = g.runLen, H = g.frameH;
+    for (int run = threadIdx.x; run * L < H; run += kWG) {
+        const int rend = min(run * L + L, H);
+        start(run, run * L);
+        for (int r0 = run * L; r0 < rend; r0 += kCH) {
+            Rows8<TI> I;
+            if (FAST || (g.vec && rend - r0 >= kCH)) I.load(img + r0);
+            else I.load_ragged(img + r0, rend - r0);
+#pragma unroll
+            for (int q = 0; q < kCH; q += CH) {
+                if (!FAST && r0 + q >= rend) break;
+                body(r0 + q, FAST ? CH : min(CH, rend - r0 - q), I, q);
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -368,13 +512,14 @@ __device__ __forceinline__ const TI *column_ptr(const GroupDev &g, int c) {
 // (d_applyParameters, d_createDifferenceImage, d_calcBaseErrval,
 //  d_updateGradients, d_fillDiagonals, d_fillJTr in one pass)
 // ---------------------------------------------------------------------------
-template <typename TI, typename R, int V>
-__device__ void assemble_column(const GroupDev &g, int c) {
+template <typename TI, typename R, int V, bool FAST, int GRAD>
+__device__ __forceinline__ void assemble_column_t(GroupRef g, int c) {
     const int b = c % g.nb;
     const ColKnots<R> kn = current_knots<R>(g, c);
-    const TI *img = column_ptr<TI>(g, c);
-    const typename Prec<R>::V4 *geo = Prec<R>::geo(g) ? Prec<R>::geo(g) + (size_t)b * g.frameH : nullptr;
-    const R *fnx = g.fracUniform ? nullptr : Prec<R>::fnext(g) + (size_t)b * g.frameH;
+    const Template<R, FAST> T(g);
+    GeoRun<R, FAST> geo(g, b);
+    const SS_GLOBAL R *fnx = FAST || g.fracUniform ? nullptr : as_global(Prec<R>::fnext(g)) + (size_t)b * g.frameH;
+    const int last = g.frameH - 1;
     // h[1] = sum I, h[i - 1] = column sum i for i >= CS_AXX; the errval term
     // is accumulated in FP64 per pixel: it decides line-search acceptance
     // against near-equal candidates
@@ -384,37 +529,40 @@ __device__ void assemble_column(const GroupDev &g, int c) {
     for (int i = 0; i < CS_N - 1; i++) h[i] = (R)0;
     int cnt = 0;
     constexpr int CH = chunk_rows<R>(2, tune_variant<TK_ASSEMBLE, R, V>().samples);
-    for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
-        const int rend = min(run * g.runLen + g.runLen, g.frameH);
-        GeoIter<R> it;
-        it.start(g, b, run * g.runLen);
-        for (int r0 = run * g.runLen; r0 < rend; r0 += CH) {
-            const int n = min(CH, rend - r0);
-            R I[CH];
-            load_chunk<CH>(img + r0, g.vec, n, I);
+    walk_rows<CH, FAST>(
+        g, column_ptr<TI>(g, c), [&](int run, int r0) { geo.start(run, r0); },
+        [&](int r, int n, const Rows8<TI> &I, int off) {
+            R bx[CH], by[CH], f[CH];
+            bool ok[CH];
+            Tap<R> tap[CH];
+            Grads<R, GRAD> gr[CH];
+            geo.template rows<CH>(r, last, bx, by, f, ok);
 #pragma unroll
             for (int k = 0; k < CH; k++) {
-                const int rr = min(r0 + k, g.frameH - 1);
-                R bx, by, f;
-                bool m;
-                it.at(g, geo, rr, bx, by, f, m);
-                it.next();
-                h[CS_SUMI] += I[k];
-                const R x = mad(kn.dx, f, bx + kn.ax);
-                const R y = mad(kn.dy, f, by + kn.ay);
-                const bool ok = k < n && m && in_bounds(g, x, y);
-                Cell<R> cl;
-                const R s = sample(g, x, y, ok, cl);
-                R wx, wy;
-                gradients(g, cl, wx, wy);
+                const R x = kn.x(bx[k], f[k]), y = kn.y(by[k], f[k]);
+                ok[k] = (FAST || (k < n && ok[k])) && T.inside(x, y);
+                T.fetch(x, y, tap[k]);
+                gr[k].fetch(g, tap[k]);
+            }
+            sched_fence();
+#pragma unroll
+            for (int k = 0; k < CH; k++) {
+                const R Ik = I.template at<R>(off + k);
+                h[CS_SUMI] += Ik;
+                R d = Ik - bilinear(tap[k]), wx, wy;
+                gr[k].eval(tap[k], wx, wy);
+                pin(d);
+                pin(wx);
+                pin(wy);
                 // outside the mask every term below is zero
-                const R d = ok ? I[k] - s : (R)0;
-                wx = ok ? wx : (R)0;
-                wy = ok ? wy : (R)0;
-                const R cf = (R)1 - f;
+                d = ok[k] ? d : (R)0;
+                wx = ok[k] ? wx : (R)0;
+                wy = ok[k] ? wy : (R)0;
+                const R fk = f[k];
+                const R cf = (R)1 - fk;
                 const R xx = wx * wx, yy = wy * wy, xy = wx * wy;
-                const R c2 = cf * cf, f2 = f * f, fc = f - f2;
-                cnt += ok ? 1 : 0;
+                const R c2 = cf * cf, f2 = fk * fk, fc = fk - f2;
+                cnt += ok[k] ? 1 : 0;
                 d2 = fma((double)d, (double)d, d2);
                 h[CS_AXX - 1] = mad(xx, c2, h[CS_AXX - 1]);
                 h[CS_AYY - 1] = mad(yy, c2, h[CS_AYY - 1]);
@@ -425,21 +573,20 @@ __device__ void assemble_column(const GroupDev &g, int c) {
                 h[CS_CXX - 1] = mad(xx, fc, h[CS_CXX - 1]);
                 h[CS_CYY - 1] = mad(yy, fc, h[CS_CYY - 1]);
                 h[CS_CXY - 1] = mad(xy, fc, h[CS_CXY - 1]);
-                const R dc = d * cf, df = d * f;
+                const R dc = d * cf, df = d * fk;
                 h[CS_JXA - 1] = mad(dc, wx, h[CS_JXA - 1]);
                 h[CS_JYA - 1] = mad(dc, wy, h[CS_JYA - 1]);
                 h[CS_JXB - 1] = mad(df, wx, h[CS_JXB - 1]);
                 h[CS_JYB - 1] = mad(df, wy, h[CS_JYB - 1]);
-                if (fnx) {
-                    const R fn = fnx[rr];
+                if (!FAST && fnx) {
+                    const R fn = fnx[min(r + k, last)];
                     const R n2 = fn * fn;
                     h[CS_QXX - 1] = mad(xx, n2, h[CS_QXX - 1]);
                     h[CS_QYY - 1] = mad(yy, n2, h[CS_QYY - 1]);
                     h[CS_QXY - 1] = mad(xy, n2, h[CS_QXY - 1]);
                 }
             }
-        }
-    }
+        });
     double v[CS_N];
     v[CS_D2] = d2;
     v[CS_SUMI] = (double)h[CS_SUMI];
@@ -451,18 +598,32 @@ __device__ void assemble_column(const GroupDev &g, int c) {
     if (threadIdx.x < CS_N) g.colsum[(size_t)c * CS_N + threadIdx.x] = out[threadIdx.x];
 }
 
+template <typename TI, typename R, int V>
+__device__ __forceinline__ void assemble_column(GroupRef g, int c) {
+    if constexpr (sizeof(R) == 4) {
+        if (g.gradBF16) {
+            if (g.fast) assemble_column_t<TI, R, V, true, GRAD_BF16>(g, c);
+            else assemble_column_t<TI, R, V, false, GRAD_BF16>(g, c);
+            return;
+        }
+    }
+    if (!g.gradFD) assemble_column_t<TI, R, V, false, GRAD_PAIRS>(g, c);
+    else if (g.fast) assemble_column_t<TI, R, V, true, GRAD_FD>(g, c);
+    else assemble_column_t<TI, R, V, false, GRAD_FD>(g, c);
+}
+
 template <typename TI, typename R>
-__device__ __forceinline__ void final_column(const GroupDev &g, int c);
+__device__ __forceinline__ void final_column(GroupRef g, int c);
 
 // The assembly launch also runs the final pass of the groups that stopped
 // in the previous tick (phase PH_FINAL), for a tick without final stages.
 template <typename TI, typename R, int V>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(tune_variant<TK_ASSEMBLE, R, V>().waves))) void k_assemble(Batch B) {
     for (int item = blockIdx.x; item < B.nItems; item += gridDim.x) {
-        const int gi = B.itemGroup[item];
-        const int phase = B.ctl[gi].phase;
+        const int gi = as_const(B.itemGroup)[item];
+        const int phase = as_const(B.ctl)[gi].phase;
         if (phase != PH_ASSEMBLE && phase != PH_FINAL) continue;
-        const GroupDev &g = B.groups[gi];
+        GroupRef g = group_of(B, gi);
         if (!runs_here<TI, R>(g) || g.var[TK_ASSEMBLE] != V) continue;
         if (phase == PH_FINAL) {
             final_column<TI, R>(g, item - g.itemStart);
@@ -1240,25 +1401,28 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
 // candidates in slot 0 (K1 after the solve, Kn when the line search goes on
 // from the previous slots) and Kn after it; no round runs past maxRounds.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ bool ls_round_runs(const GroupDev &g, const GroupCtl &ctl, int slot) {
+template <typename G, typename C>
+__device__ __forceinline__ bool ls_round_runs(G &g, C &ctl, int slot) {
     return ctl.roundsThisLS + slot < g.maxRounds;
 }
-__device__ __forceinline__ int ls_round_k(const GroupDev &g, const GroupCtl &ctl, int slot) {
+template <typename G, typename C>
+__device__ __forceinline__ int ls_round_k(G &g, C &ctl, int slot) {
     return slot == 0 ? ctl.K : g.Kn;
 }
 
 // Candidates k0 .. k0 + K - 1 of column c; their sums go to the column's
 // candidate slots slot0 .. slot0 + K - 1.
-template <typename TI, typename R, int V, int K>
-__device__ void ls_column(const GroupDev &g, int c, int b, int k0, int slot0) {
+template <typename TI, typename R, int V, int K, bool FAST>
+__device__ __forceinline__ void ls_column_t(GroupRef g, int c, int b, int k0, int slot0) {
     ColKnots<R> kn[K];
     {
         const int N = g.N;
         const double r = g.rmult;
-        double dlx = reduce_pow(g.d0[c], r, k0), dly = reduce_pow(g.d0[c + N], r, k0);
-        double drx = reduce_pow(g.d0[c + 1], r, k0), dry = reduce_pow(g.d0[c + 1 + N], r, k0);
+        const SS_CONST double *p0 = as_const(g.p0), *d0 = as_const(g.d0);
+        double dlx = reduce_pow(d0[c], r, k0), dly = reduce_pow(d0[c + N], r, k0);
+        double drx = reduce_pow(d0[c + 1], r, k0), dry = reduce_pow(d0[c + 1 + N], r, k0);
         const bool lastKnot = (c + 1 == g.fframeW);
-        const double plx = g.p0[c], ply = g.p0[c + N], prx = g.p0[c + 1], pry = g.p0[c + 1 + N];
+        const double plx = p0[c], ply = p0[c + N], prx = p0[c + 1], pry = p0[c + 1 + N];
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const double lx = plx + dlx, ly = ply + dly;
@@ -1270,8 +1434,9 @@ __device__ void ls_column(const GroupDev &g, int c, int b, int k0, int slot0) {
             dry *= r;
         }
     }
-    const TI *img = column_ptr<TI>(g, c);
-    const typename Prec<R>::V4 *geo = Prec<R>::geo(g) ? Prec<R>::geo(g) + (size_t)b * g.frameH : nullptr;
+    const Template<R, FAST> T(g);
+    GeoRun<R, FAST> geo(g, b);
+    const int last = g.frameH - 1;
     double e2[K];  // FP64: compared against the half-iteration's errval
     int cnt[K];
 #pragma unroll
@@ -1280,35 +1445,35 @@ __device__ void ls_column(const GroupDev &g, int c, int b, int k0, int slot0) {
         cnt[k] = 0;
     }
     constexpr int CH = chunk_rows<R>(K, tune_variant<TK_LS, R, V>().samples);
-    for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
-        const int rend = min(run * g.runLen + g.runLen, g.frameH);
-        GeoIter<R> it;
-        it.start(g, b, run * g.runLen);
-        for (int r0 = run * g.runLen; r0 < rend; r0 += CH) {
-            const int n = min(CH, rend - r0);
-            R I[CH];
-            load_chunk<CH>(img + r0, g.vec, n, I);
+    walk_rows<CH, FAST>(
+        g, column_ptr<TI>(g, c), [&](int run, int r0) { geo.start(run, r0); },
+        [&](int r, int n, const Rows8<TI> &I, int off) {
+            R bx[CH], by[CH], f[CH];
+            bool m[CH], ok[CH][K];
+            Tap<R> tap[CH][K];
+            geo.template rows<CH>(r, last, bx, by, f, m);
 #pragma unroll
-            for (int q = 0; q < CH; q++) {
-                R bx, by, f;
-                bool m;
-                it.at(g, geo, min(r0 + q, g.frameH - 1), bx, by, f, m);
-                it.next();
-                m = m && q < n;
+            for (int q = 0; q < CH; q++)
 #pragma unroll
                 for (int k = 0; k < K; k++) {
-                    const R x = mad(kn[k].dx, f, bx + kn[k].ax);
-                    const R y = mad(kn[k].dy, f, by + kn[k].ay);
-                    const bool ok = m && in_bounds(g, x, y);
-                    Cell<R> cl;
-                    const R s = sample(g, x, y, ok, cl);
-                    const R d = ok ? I[q] - s : (R)0;
+                    const R x = kn[k].x(bx[q], f[q]), y = kn[k].y(by[q], f[q]);
+                    ok[q][k] = (FAST || (q < n && m[q])) && T.inside(x, y);
+                    T.fetch(x, y, tap[q][k]);
+                }
+            sched_fence();
+#pragma unroll
+            for (int q = 0; q < CH; q++) {
+                const R Iq = I.template at<R>(off + q);
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+                    R d = Iq - bilinear(tap[q][k]);
+                    pin(d);
+                    d = ok[q][k] ? d : (R)0;
                     e2[k] = fma((double)d, (double)d, e2[k]);
-                    cnt[k] += ok ? 1 : 0;
+                    cnt[k] += ok[q][k] ? 1 : 0;
                 }
             }
-        }
-    }
+        });
     double v[2 * K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
@@ -1320,6 +1485,12 @@ __device__ void ls_column(const GroupDev &g, int c, int b, int k0, int slot0) {
     if (threadIdx.x < 2 * K) g.lssum[(size_t)c * 2 * kMaxCand + 2 * slot0 + threadIdx.x] = out[threadIdx.x];
 }
 
+template <typename TI, typename R, int V, int K>
+__device__ __forceinline__ void ls_column(GroupRef g, int c, int b, int k0, int slot0) {
+    if (g.fast) ls_column_t<TI, R, V, K, true>(g, c, b, k0, slot0);
+    else ls_column_t<TI, R, V, K, false>(g, c, b, k0, slot0);
+}
+
 // split = 2: work item w covers column w % nItems and, of a round of four
 // candidates, the two of half w / nItems (each candidate's sums are the
 // same whichever workgroup computes them); other rounds run in half 0.
@@ -1328,14 +1499,14 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(tune_varian
     const int nWork = B.nItems * split;
     for (int w = blockIdx.x; w < nWork; w += gridDim.x) {
         const int half = w >= B.nItems ? 1 : 0, item = w - half * B.nItems;
-        const int gi = B.itemGroup[item];
-        const GroupCtl &ctl = B.ctl[gi];
+        const int gi = as_const(B.itemGroup)[item];
+        const SS_CONST GroupCtl &ctl = as_const(B.ctl)[gi];
         if (ctl.phase != PH_LS) continue;
-        const GroupDev &g = B.groups[gi];
+        GroupRef g = group_of(B, gi);
         if (!runs_here<TI, R>(g) || g.var[TK_LS] != V || !ls_round_runs(g, ctl, slot)) continue;
         const int c = item - g.itemStart, f = c / g.nb, b = c % g.nb;
-        if (!g.lsActive[f]) continue;
-        int K = ls_round_k(g, ctl, slot), k0 = g.lsNextK[f], slot0 = 0;
+        if (!as_const(g.lsActive)[f]) continue;
+        int K = ls_round_k(g, ctl, slot), k0 = as_const(g.lsNextK)[f], slot0 = 0;
         if (split == 2 && K == 4) {
             K = 2;
             k0 += 2 * half;
@@ -1534,34 +1705,32 @@ __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
 // task_correlation.cu:63-99) of every frame's last-tried state; the
 // statistic of a column covers its leading run of masked rows only.
 // ---------------------------------------------------------------------------
-template <typename TI, typename R, int V>
-__device__ void corr_column(const GroupDev &g, int c) {
+template <typename TI, typename R, int V, bool FAST>
+__device__ __forceinline__ void corr_column_t(GroupRef g, int c) {
     const int f = c / g.nb, b = c % g.nb;
-    const int mk = g.lsMk[f], dk = g.lsDk[f];
+    const int mk = as_const(g.lsMk)[f], dk = as_const(g.lsDk)[f];
     const bool same = (mk == dk);
     const ColKnots<R> km = state_knots<R>(g, c, mk);
     const ColKnots<R> kd = state_knots<R>(g, c, dk);
-    const TI *img = column_ptr<TI>(g, c);
-    const typename Prec<R>::V4 *geo = Prec<R>::geo(g) ? Prec<R>::geo(g) + (size_t)b * g.frameH : nullptr;
+    const SS_GLOBAL TI *img = column_ptr<TI>(g, c);
+    const Template<R, FAST> T(g);
+    GeoRun<R, FAST> geo(g, b);
+    const int last = g.frameH - 1;
     // first row outside the mask of the last-tried state: the moments cover
     // the rows before it
     int firstOut = g.frameH;
     constexpr int CH = chunk_rows<R>(1, tune_variant<TK_CORR, R, V>().samples);
     for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
         const int rend = min(run * g.runLen + g.runLen, g.frameH);
-        GeoIter<R> it;
-        it.start(g, b, run * g.runLen);
+        geo.start(run, run * g.runLen);
         for (int r0 = run * g.runLen; r0 < rend && r0 < firstOut; r0 += CH) {
-            const int n = min(CH, rend - r0);
+            R bx[CH], by[CH], f1[CH];
+            bool m[CH];
+            geo.template rows<CH>(r0, last, bx, by, f1, m);
 #pragma unroll
             for (int q = 0; q < CH; q++) {
-                R bx, by, f1;
-                bool m;
-                it.at(g, geo, min(r0 + q, g.frameH - 1), bx, by, f1, m);
-                it.next();
-                const R x = mad(km.dx, f1, bx + km.ax);
-                const R y = mad(km.dy, f1, by + km.ay);
-                if (q < n && !(m && in_bounds(g, x, y))) firstOut = min(firstOut, r0 + q);
+                const R x = km.x(bx[q], f1[q]), y = km.y(by[q], f1[q]);
+                if ((FAST || r0 + q < rend) && !(m[q] && T.inside(x, y))) firstOut = min(firstOut, r0 + q);
             }
         }
     }
@@ -1569,60 +1738,70 @@ __device__ void corr_column(const GroupDev &g, int c) {
     double v[CR_N];
 #pragma unroll
     for (int i = 0; i < CR_N; i++) v[i] = 0.0;
-    for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
-        const int rend = min(run * g.runLen + g.runLen, g.frameH);
-        GeoIter<R> it;
-        it.start(g, b, run * g.runLen);
-        for (int r0 = run * g.runLen; r0 < rend; r0 += CH) {
-            const int n = min(CH, rend - r0);
-            R I[CH];
-            load_chunk<CH>(img + r0, g.vec, n, I);
+    walk_rows<CH, FAST>(
+        g, img, [&](int run, int r0) { geo.start(run, r0); },
+        [&](int r, int n, const Rows8<TI> &I, int off) {
+            R bx[CH], by[CH], f1[CH];
+            bool m[CH], mm[CH], okd[CH];
+            Tap<R> tap[CH];
+            geo.template rows<CH>(r, last, bx, by, f1, m);
+            R xd[CH], yd[CH];
 #pragma unroll
             for (int q = 0; q < CH; q++) {
-                R bx, by, f1;
-                bool m;
-                it.at(g, geo, min(r0 + q, g.frameH - 1), bx, by, f1, m);
-                it.next();
-                m = m && q < n;
-                const R x = mad(km.dx, f1, bx + km.ax);
-                const R y = mad(km.dy, f1, by + km.ay);
-                const bool mm = m && in_bounds(g, x, y);
-                // the difference image holds the last-decided state's residual
-                R xd = x, yd = y;
-                bool okd = mm;
-                if (!same) {
-                    xd = mad(kd.dx, f1, bx + kd.ax);
-                    yd = mad(kd.dy, f1, by + kd.ay);
-                    okd = m && in_bounds(g, xd, yd);
+                m[q] = FAST || (q < n && m[q]);
+                xd[q] = km.x(bx[q], f1[q]);
+                yd[q] = km.y(by[q], f1[q]);
+                okd[q] = mm[q] = m[q] && T.inside(xd[q], yd[q]);
+            }
+            // the difference image holds the last-decided state's residual
+            if (!same) {
+#pragma unroll
+                for (int q = 0; q < CH; q++) {
+                    xd[q] = kd.x(bx[q], f1[q]);
+                    yd[q] = kd.y(by[q], f1[q]);
+                    okd[q] = m[q] && T.inside(xd[q], yd[q]);
                 }
-                Cell<R> cl;
-                const R s = sample(g, xd, yd, okd, cl);
-                const R dbuf = okd ? I[q] - s : (R)0;
-                const double Iq = q < n ? (double)I[q] : 0.0;
-                v[CR_SUMD] += mm ? (double)(I[q] - dbuf) : (double)dbuf;
-                v[CR_NMASK] += mm ? 1.0 : 0.0;
-                const bool run = r0 + q < firstOut;  // rows before it are all inside the mask
-                const double a = run ? (double)(I[q] - dbuf) : 0.0, bb = run ? Iq : 0.0;
+            }
+#pragma unroll
+            for (int q = 0; q < CH; q++) T.fetch(xd[q], yd[q], tap[q]);
+            sched_fence();
+#pragma unroll
+            for (int q = 0; q < CH; q++) {
+                const R Iq = I.template at<R>(off + q);
+                R d = Iq - bilinear(tap[q]);
+                pin(d);
+                const R dbuf = okd[q] ? d : (R)0;
+                const R w = Iq - dbuf;
+                const double Id = FAST || q < n ? (double)Iq : 0.0;
+                v[CR_SUMD] += (double)(mm[q] ? w : dbuf);
+                v[CR_NMASK] += mm[q] ? 1.0 : 0.0;
+                const bool lead = r + q < firstOut;  // rows before it are all inside the mask
+                const double a = lead ? (double)w : 0.0, bb = lead ? Id : 0.0;
                 v[CR_SA] += a;
                 v[CR_SAA] += a * a;
                 v[CR_SB] += bb;
                 v[CR_SBB] += bb * bb;
                 v[CR_SAB] += a * bb;
-                v[CR_NS] += run ? 1.0 : 0.0;
+                v[CR_NS] += lead ? 1.0 : 0.0;
             }
-        }
-    }
+        });
     __shared__ double out[CR_N];
     block_sum<CR_N>(v, out);
     if (threadIdx.x < CR_N) g.corrsum[(size_t)c * CR_N + threadIdx.x] = out[threadIdx.x];
 }
 
 template <typename TI, typename R, int V>
+__device__ __forceinline__ void corr_column(GroupRef g, int c) {
+    if (g.fast) corr_column_t<TI, R, V, true>(g, c);
+    else corr_column_t<TI, R, V, false>(g, c);
+}
+
+template <typename TI, typename R, int V>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(tune_variant<TK_CORR, R, V>().waves))) void k_corr(Batch B) {
     for (int item = blockIdx.x; item < B.nItems; item += gridDim.x) {
-        const int gi = B.itemGroup[item];
-        if (B.ctl[gi].phase != PH_CORR) continue;
-        const GroupDev &g = B.groups[gi];
+        const int gi = as_const(B.itemGroup)[item];
+        if (as_const(B.ctl)[gi].phase != PH_CORR) continue;
+        GroupRef g = group_of(B, gi);
         if (!runs_here<TI, R>(g) || g.var[TK_CORR] != V) continue;
         corr_column<TI, R, V>(g, item - g.itemStart);
     }
@@ -1638,49 +1817,43 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(tune_varian
 // own, launched only for batches that ask for it, so that the correlation
 // kernel's register allocation does not carry it.
 template <typename TI, typename R>
-__device__ void frame_corr_column(const GroupDev &g, int c) {
+__device__ void frame_corr_column(GroupRef g, int c) {
     const int f = c / g.nb, b = c % g.nb;
-    const int mk = g.lsMk[f], dk = g.lsDk[f];
+    const int mk = as_const(g.lsMk)[f], dk = as_const(g.lsDk)[f];
     const bool same = (mk == dk);
     const ColKnots<R> km = state_knots<R>(g, c, mk);
     const ColKnots<R> kd = state_knots<R>(g, c, dk);
-    const TI *img = column_ptr<TI>(g, c);
-    const typename Prec<R>::V4 *geo = Prec<R>::geo(g) ? Prec<R>::geo(g) + (size_t)b * g.frameH : nullptr;
+    const Template<R, false> T(g);
+    GeoRun<R, false> geo(g, b);
+    const int last = g.frameH - 1;
     constexpr int CH = chunk_rows<R>(1, sizeof(R) == 8 ? kFinalSamplesF64 : kFinalSamplesF32);
     const long long swapBack = min((long long)((g.fframeW + 255) / 256) * 256, (long long)g.frameH * g.fframeW);
     double w[FC_N];
 #pragma unroll
     for (int i = 0; i < FC_N; i++) w[i] = 0.0;
-    for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
-        const int rend = min(run * g.runLen + g.runLen, g.frameH);
-        GeoIter<R> it;
-        it.start(g, b, run * g.runLen);
-        for (int r0 = run * g.runLen; r0 < rend; r0 += CH) {
-            const int n = min(CH, rend - r0);
-            R I[CH];
-            load_chunk<CH>(img + r0, g.vec, n, I);
+    walk_rows<CH, false>(
+        g, column_ptr<TI>(g, c), [&](int run, int r0) { geo.start(run, r0); },
+        [&](int r, int n, const Rows8<TI> &I, int off) {
+            R bx[CH], by[CH], f1[CH];
+            bool m[CH];
+            geo.template rows<CH>(r, last, bx, by, f1, m);
 #pragma unroll
             for (int q = 0; q < CH; q++) {
-                R bx, by, f1;
-                bool m;
-                it.at(g, geo, min(r0 + q, g.frameH - 1), bx, by, f1, m);
-                it.next();
-                m = m && q < n;
-                const R x = mad(km.dx, f1, bx + km.ax);
-                const R y = mad(km.dy, f1, by + km.ay);
-                const bool mm = m && in_bounds(g, x, y);
-                R xd = x, yd = y;
+                const bool in = q < n && m[q];
+                R xd = km.x(bx[q], f1[q]), yd = km.y(by[q], f1[q]);
+                const bool mm = in && T.inside(xd, yd);
                 bool okd = mm;
                 if (!same) {
-                    xd = mad(kd.dx, f1, bx + kd.ax);
-                    yd = mad(kd.dy, f1, by + kd.ay);
-                    okd = m && in_bounds(g, xd, yd);
+                    xd = kd.x(bx[q], f1[q]);
+                    yd = kd.y(by[q], f1[q]);
+                    okd = in && T.inside(xd, yd);
                 }
-                Cell<R> cl;
-                const R smp = sample(g, xd, yd, okd, cl);
-                const R Ir = q < n ? I[q] : (R)0;
+                Tap<R> tap;
+                T.fetch(xd, yd, tap);
+                const R smp = bilinear(tap);
+                const R Ir = q < n ? I.template at<R>(off + q) : (R)0;
                 const R dbuf = okd ? Ir - smp : (R)0;
-                const bool pre = (long long)(r0 + q) * g.fframeW + c < swapBack;
+                const bool pre = (long long)(r + q) * g.fframeW + c < swapBack;
                 const R d1 = Ir - dbuf;           // the global correlation's swap
                 const R d2 = pre ? Ir - d1 : d1;  // its partial swap-back
                 const R d3 = mm ? Ir - d2 : dbuf; // the frame correlation's swap
@@ -1695,8 +1868,7 @@ __device__ void frame_corr_column(const GroupDev &g, int c) {
                 w[FC_SBB] += mm ? bb * bb : zb * zb;
                 w[FC_SAB] += a * bb;
             }
-        }
-    }
+        });
     __shared__ double outF[FC_N];
     block_sum<FC_N>(w, outF);
     if (threadIdx.x < FC_N) g.finalsum[(size_t)c * FS_N + threadIdx.x] = outF[threadIdx.x];
@@ -1705,9 +1877,9 @@ __device__ void frame_corr_column(const GroupDev &g, int c) {
 template <typename TI, typename R>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k_corr_frames(Batch B) {
     for (int item = blockIdx.x; item < B.nItems; item += gridDim.x) {
-        const int gi = B.itemGroup[item];
-        if (B.ctl[gi].phase != PH_CORR) continue;
-        const GroupDev &g = B.groups[gi];
+        const int gi = as_const(B.itemGroup)[item];
+        if (as_const(B.ctl)[gi].phase != PH_CORR) continue;
+        GroupRef g = group_of(B, gi);
         if (!g.fcIter || !runs_here<TI, R>(g)) continue;
         frame_corr_column<TI, R>(g, item - g.itemStart);
     }
@@ -1817,60 +1989,69 @@ __global__ __launch_bounds__(kSolveWG) void k_corr_finish(Batch B) {
 // final state: errvals, frame correlations and mask of the last-tried state
 // (hd_calculateGroupErrvals(0) + hd_frameCorrelation, task.cpp:389-405)
 // ---------------------------------------------------------------------------
-template <typename TI, typename R>
-__device__ __forceinline__ void final_column(const GroupDev &g, int c) {
+template <typename TI, typename R, bool FAST>
+__device__ __forceinline__ void final_column_t(GroupRef g, int c) {
     const int f = c / g.nb, b = c % g.nb;
-    const ColKnots<R> kn = state_knots<R>(g, c, g.lsMk[f]);
-    const TI *img = column_ptr<TI>(g, c);
-    const typename Prec<R>::V4 *geo = Prec<R>::geo(g) ? Prec<R>::geo(g) + (size_t)b * g.frameH : nullptr;
-    uint8_t *mo = g.maskOut ? g.maskOut + (size_t)c * g.frameH : nullptr;
+    const ColKnots<R> kn = state_knots<R>(g, c, as_const(g.lsMk)[f]);
+    const Template<R, FAST> T(g);
+    GeoRun<R, FAST> geo(g, b);
+    const int last = g.frameH - 1;
+    SS_GLOBAL uint8_t *mo = g.maskOut ? (SS_GLOBAL uint8_t *)g.maskOut + (size_t)c * g.frameH : nullptr;
     double v[FS_N];
 #pragma unroll
     for (int i = 0; i < FS_N; i++) v[i] = 0.0;
     constexpr int CH = chunk_rows<R>(1, sizeof(R) == 8 ? kFinalSamplesF64 : kFinalSamplesF32);
-    for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
-        const int rend = min(run * g.runLen + g.runLen, g.frameH);
-        GeoIter<R> it;
-        it.start(g, b, run * g.runLen);
-        for (int r0 = run * g.runLen; r0 < rend; r0 += CH) {
-            const int n = min(CH, rend - r0);
-            R I[CH];
-            load_chunk<CH>(img + r0, g.vec, n, I);
+    walk_rows<CH, FAST>(
+        g, column_ptr<TI>(g, c), [&](int run, int r0) { geo.start(run, r0); },
+        [&](int r, int n, const Rows8<TI> &I, int off) {
+            R bx[CH], by[CH], f1[CH];
+            bool mm[CH];
+            Tap<R> tap[CH];
+            geo.template rows<CH>(r, last, bx, by, f1, mm);
 #pragma unroll
             for (int q = 0; q < CH; q++) {
-                R bx, by, f1;
-                bool m;
-                it.at(g, geo, min(r0 + q, g.frameH - 1), bx, by, f1, m);
-                it.next();
-                const R x = mad(kn.dx, f1, bx + kn.ax);
-                const R y = mad(kn.dy, f1, by + kn.ay);
-                const bool mm = q < n && m && in_bounds(g, x, y);
-                if (mo && q < n) mo[r0 + q] = mm ? 1 : 0;
-                Cell<R> cl;
-                const R s = sample(g, x, y, mm, cl);
-                const double wI = mm ? (double)s : 0.0, Iq = mm ? (double)I[q] : 0.0;
+                const R x = kn.x(bx[q], f1[q]), y = kn.y(by[q], f1[q]);
+                mm[q] = (FAST || (q < n && mm[q])) && T.inside(x, y);
+                T.fetch(x, y, tap[q]);
+            }
+            sched_fence();
+            if (mo) {
+#pragma unroll
+                for (int q = 0; q < CH; q++)
+                    if (FAST || q < n) mo[r + q] = mm[q] ? 1 : 0;
+            }
+#pragma unroll
+            for (int q = 0; q < CH; q++) {
+                double s = (double)bilinear(tap[q]);
+                pin(s);
+                const double wI = mm[q] ? s : 0.0, Iq = mm[q] ? (double)I.template at<R>(off + q) : 0.0;
                 const double d = Iq - wI;
                 v[FS_D2] += d * d;
-                v[FS_CNT] += mm ? 1.0 : 0.0;
+                v[FS_CNT] += mm[q] ? 1.0 : 0.0;
                 v[FS_SA] += wI;
                 v[FS_SAA] += wI * wI;
                 v[FS_SB] += Iq;
                 v[FS_SBB] += Iq * Iq;
                 v[FS_SAB] += wI * Iq;
             }
-        }
-    }
+        });
     __shared__ double out[FS_N];
     block_sum<FS_N>(v, out);
     if (threadIdx.x < FS_N) g.finalsum[(size_t)c * FS_N + threadIdx.x] = out[threadIdx.x];
 }
 
 template <typename TI, typename R>
+__device__ __forceinline__ void final_column(GroupRef g, int c) {
+    if (g.fast) final_column_t<TI, R, true>(g, c);
+    else final_column_t<TI, R, false>(g, c);
+}
+
+template <typename TI, typename R>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? kFinalWavesF64 : kFinalWavesF32))) void k_final(Batch B) {
     for (int item = blockIdx.x; item < B.nItems; item += gridDim.x) {
-        const int gi = B.itemGroup[item];
-        if (B.ctl[gi].phase != PH_FINAL) continue;
-        const GroupDev &g = B.groups[gi];
+        const int gi = as_const(B.itemGroup)[item];
+        if (as_const(B.ctl)[gi].phase != PH_FINAL) continue;
+        GroupRef g = group_of(B, gi);
         if (!runs_here<TI, R>(g)) continue;
         final_column<TI, R>(g, item - g.itemStart);
     }

@@ -7,15 +7,15 @@
 //   waves:   minimum waves per SIMD that the kernel's register allocation
 //            must allow (more waves hide more gather latency; fewer
 //            registers limit how many gathers a wave keeps in flight).
-// Variant 0 is the default for batches that fill the chip: the values
-// measured fastest on MI355X for batches of 512x512 groups (the headline
-// workload); in FP32 the assembly and line search take 4 samples, which
-// measure as fast as 8 without spilling registers.  A batch of at most 8
-// block columns per CU (one 512x512 group of 50 frames has 1600) runs too
-// few workgroups to fill the chip, and there kSmallBatchVariant picks the
-// variants measured fastest there: FP64 assembly and correlation at 4 waves
-// per SIMD (one 512x512 group's first tick 142 and 72 us against 154 and 75)
-// and the FP32 line search with 8 samples in flight (131 against 141 us).
+// Variant 0 is the default: the values measured fastest on MI355X for batches
+// of 512x512 groups (1000 x 512x512 uint16 in FP64: line search 36.6 ms with
+// 4 samples at 5 waves against 46.0 at 4 waves and 40.0 with 8 samples at 3;
+// correlation 10.4 against 11.8 with 8 samples at 3 waves; assembly 20.6
+// against 21.2 at 3 waves.  24 uneven groups in FP32: line search 36.3 ms with
+// 4 samples at 5 waves against 37.9 with 8 at 4, correlation 8.7 against 9.4).
+// One 512x512 group of 50 frames measures the same order, so a batch of at
+// most 8 block columns per CU, whose group does not fill the chip, runs them
+// too (kSmallBatchVariant).
 // The engine's autotuner (off unless asked for) times all variants on a
 // group shape's first tick and keeps the fastest per kernel.
 // A variant only changes how many rows a thread unrolls and how registers
@@ -35,15 +35,15 @@ struct TuneVariant {
 // [kernel][fp64][variant]
 constexpr TuneVariant kTuneTable[TK_COUNT][2][kVariants] = {
     // assembly: FP32, FP64
-    {{{4, 4}, {8, 4}, {8, 3}}, {{4, 2}, {2, 3}, {2, 4}}},
+    {{{8, 4}, {4, 4}, {4, 5}}, {{4, 4}, {4, 3}, {2, 4}}},
     // line search
-    {{{4, 4}, {8, 4}, {8, 3}}, {{4, 4}, {2, 4}, {8, 3}}},
+    {{{4, 5}, {8, 4}, {4, 4}}, {{4, 5}, {8, 3}, {4, 4}}},
     // correlation (one sample per row; a chunk holds at most 8 rows)
-    {{{8, 4}, {4, 4}, {2, 4}}, {{8, 2}, {4, 3}, {2, 3}}},
+    {{{4, 5}, {8, 4}, {4, 6}}, {{4, 4}, {8, 3}, {2, 4}}},
 };
 
 // [kernel][fp64]: the variant of batches of at most 8 block columns per CU
-constexpr int kSmallBatchVariant[TK_COUNT][2] = {{0, 2}, {1, 0}, {0, 2}};
+constexpr int kSmallBatchVariant[TK_COUNT][2] = {{0, 0}, {0, 0}, {0, 0}};
 
 template <int KERNEL, typename R, int V>
 __host__ __device__ constexpr TuneVariant tune_variant() {
