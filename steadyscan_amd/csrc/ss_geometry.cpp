@@ -35,21 +35,17 @@ bool scan_setup(const ss_geometry_desc &g, ScanParams &s, double *kt) {
         // (steady_scan.m:801-804)
         const int L = (int)lines_per_knot;
         for (int k = 0; k + 1 < nknots; k++) {
-            double mn = scan_pixel_time(s, k * L, 0);
-            for (int j = 1; j < s.W; j++) mn = std::fmin(mn, scan_pixel_time(s, k * L, j));
+            // a line's times are monotone in the column
+            const double mn = std::fmin(scan_pixel_time(s, k * L, 0), scan_pixel_time(s, k * L, s.W - 1));
             kt[k] = mn - dwell / 2;
         }
         kt[nknots - 1] = 1;
         kt[0] = 0;
     } else {
         // equal spacing over the cropped scan (steady_scan.m:805-811)
-        double lo = scan_cropped_time(s, 0, 0), hi = lo;
-        for (int i = 0; i < s.Hc; i++)
-            for (int j = 0; j < s.Wc; j++) {
-                const double t = scan_cropped_time(s, i, j);
-                lo = std::fmin(lo, t);
-                hi = std::fmax(hi, t);
-            }
+        // the scan's times increase from line to line and are monotone in a line
+        const double lo = std::fmin(scan_cropped_time(s, 0, 0), scan_cropped_time(s, 0, s.Wc - 1));
+        const double hi = std::fmax(scan_cropped_time(s, s.Hc - 1, 0), scan_cropped_time(s, s.Hc - 1, s.Wc - 1));
         for (int k = 0; k < nknots; k++) kt[k] = matlab_linspace(lo - dwell / 2, hi + dwell / 2, nknots, k);
         kt[0] = 0;
         kt[nknots - 1] = 1;
