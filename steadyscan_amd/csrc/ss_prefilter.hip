@@ -72,6 +72,8 @@ constexpr int kBlurRowLoads = (kBlurRows + 2 * kBlurRadius + 63) / 64;
 
 // the taps, which no kernel writes, come by scalar loads
 #define SS_CONST __attribute__((address_space(4)))
+// device memory behind a pointer of a struct: global instead of flat loads
+#define SS_GLOBAL __attribute__((address_space(1)))
 
 // One axis: the tap at distance d (dlo <= d <= dhi, every residue mod S at
 // most once) is g[d - dlo + kBlurOut - 1]; kBlurOut - 1 zeros stand on both
@@ -384,26 +386,67 @@ __global__ __launch_bounds__(1024) void k_median_divide(T *__restrict__ data, in
 // ---------------------------------------------------------------------------
 struct FillChunk {
     int th, tw, np;
-    const double *a;       // B x np input (NaN = missing)
-    double *out;           // B x np
     int *list;             // B x np: missing pixels, ascending
+    int *map;              // B x np: compact index of each missing pixel
     int *nmiss;            // B
-    double *x, *r, *ap;    // B x np (first nmiss used)
-    double *pfull;         // B x np: search direction on the image grid, 0 at known pixels
-                           // (k_fill_cg); compact index of each missing pixel (k_fill_cg_lds)
-    double *b;             // B x np: right-hand side
+    uint2 *code;           // B x np (the first nmiss used, as below): an entry's W and E neighbours,
+    uint8_t *meta;         // its degree and whether N and S are missing
+    double *x, *r, *p;     // solution, residual and search direction of the entries past the LDS
     int *status;           // B: iterations, or -1 if not converged
     int maxit;
 };
 
+// A missing pixel's system: the sum of its known neighbours and its degree
+// (in-image neighbours), W N S E (ascending index), the compact indices of
+// missing W and E neighbours and whether N and S are missing (entries m - 1
+// and m + 1).
+constexpr unsigned kAbsent = ~0u;
+struct FillEntry {
+    double known;
+    unsigned deg, w, e;
+    bool n, s;
+};
+template <typename T>
+__device__ __forceinline__ FillEntry fill_entry(const T *a, const int *map, int i, int th, int tw) {
+#pragma clang fp contract(off)
+    FillEntry q{0.0, 0, kAbsent, kAbsent, false, false};
+    const int col = i / th, row = i - col * th;
+    if (col > 0) {
+        const double v = (double)a[i - th];
+        q.deg++;
+        if (isnan(v)) q.w = (unsigned)map[i - th];
+        else q.known += v;
+    }
+    if (row > 0) {
+        const double v = (double)a[i - 1];
+        q.deg++;
+        q.n = isnan(v);
+        if (!q.n) q.known += v;
+    }
+    if (row + 1 < th) {
+        const double v = (double)a[i + 1];
+        q.deg++;
+        q.s = isnan(v);
+        if (!q.s) q.known += v;
+    }
+    if (col + 1 < tw) {
+        const double v = (double)a[i + th];
+        q.deg++;
+        if (isnan(v)) q.e = (unsigned)map[i + th];
+        else q.known += v;
+    }
+    return q;
+}
+
 // The missing (NaN) pixels of a frame in ascending order, and their count:
 // tiles of 4 * kCgThreads pixels, 4 consecutive ones per thread, a wave
 // scan by shuffles and the wave totals through LDS.
-__global__ __launch_bounds__(kCgThreads) void k_fill_list(FillChunk C) {
+template <typename T>
+__global__ __launch_bounds__(kCgThreads) void k_fill_list(FillChunk C, const T *__restrict__ data) {
     constexpr int kW = kCgThreads / 64;
     __shared__ int wsum[kW];
     const int f = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const double *a = C.a + (size_t)f * C.np;
+    const T *a = data + (size_t)f * C.np;
     int *list = C.list + (size_t)f * C.np;
     const int np = C.np;
     int carry = 0;
@@ -438,200 +481,237 @@ __global__ __launch_bounds__(kCgThreads) void k_fill_list(FillChunk C) {
 }
 
 // Sum over the workgroup of one value per thread: a butterfly in each wave,
-// then the 16 wave sums in order.
-__device__ double block_sum(double v, double *sp) {
+// then the 16 wave sums in order.  sp alternates between two buffers from
+// call to call, so that one barrier a call is enough.
+__device__ __forceinline__ double block_sum(double v, double *sp) {
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
     if ((threadIdx.x & 63) == 0) sp[threadIdx.x >> 6] = v;
     __syncthreads();
     double r = 0.0;
+#pragma unroll
     for (int w = 0; w < kCgThreads / 64; w++) r += sp[w];
-    __syncthreads();
     return r;
 }
 
-// Conjugate gradients for a frame with at most kFillLds missing pixels, in
-// compact form (entry m = the m-th missing pixel): the search direction p
-// and the residual r live in LDS, the solution x in global memory, and
-// thread t keeps, for its entries t, t + 1024, ..., only the degree and the
-// compact indices of the missing W N S E neighbours (14 bits each).  Same
-// algebra and dot-product order as k_fill_cg; a neighbour's term enters Ap
-// only when it is missing (a known neighbour's direction is zero).
-constexpr int kFillK = 8;
+// Conjugate gradients of a frame in compact form (entry m = the m-th missing
+// pixel), one workgroup per frame.  The search direction p takes the
+// workgroup's LDS, and thread t keeps the solution and the residual of its
+// entries t, t + 1024, ... in registers.  A missing N or S neighbour is entry
+// m - 1 or m + 1; the compact indices of W and E (15 bits each) and the two
+// flags fill one word.  An absent neighbour reads the zero after the last
+// entry, and entries past n hold zeros.  Dot products add every thread's
+// entries in order, then the threads as block_sum does.
+// Bound by the 10 LDS reads per entry and iteration and by the barriers of
+// the two reductions.  128 x 512x512 frames with up to 18300 missing pixels
+// and 546 iterations take 5.8 ms; with the residual in LDS too, which held
+// 8192 entries and left larger frames to a kernel in global memory, 25 ms.
+constexpr int kFillK = 19;
 constexpr int kFillLds = kFillK * kCgThreads;
-constexpr unsigned kNoNbr = 0x3fffu;
+constexpr unsigned kNoNbr = 0x7fffu, kHasN = 1u << 30, kHasS = 1u << 31;
+static_assert(kFillLds < (int)kNoNbr, "compact indices take 15 bits");
 
-__global__ __launch_bounds__(kCgThreads) void k_fill_cg_lds(FillChunk C) {
+// The entries of frame f: neighbours and right-hand side (put(m, known) takes
+// the latter); returns the thread's part of its square.
+template <typename T, typename Put>
+__device__ __forceinline__ double fill_setup(const FillChunk &C, const T *a, size_t fo, int n, Put &&put) {
 #pragma clang fp contract(off)
-    __shared__ double sp[kCgThreads / 64];
-    __shared__ double lp[kFillLds], lr[kFillLds];
-    const int f = blockIdx.x, t = threadIdx.x;
-    const int th = C.th, tw = C.tw, np = C.np;
-    const size_t fo = (size_t)f * np;
-    const double *a = C.a + fo;
-    double *out = C.out + fo, *x = C.x + fo;
-    const int *list = C.list + fo;
-    int *map = (int *)(C.pfull + fo);  // compact index of each missing pixel
-    const int n = C.nmiss[f];
-    if (n > kFillLds) return;  // k_fill_cg takes this frame
-    for (int i = t; i < np; i += kCgThreads) out[i] = a[i];
-    if (n == 0 || n == np) {  // nothing to fill, or no known pixel (left as NaN)
-        if (t == 0) C.status[f] = 0;
-        return;
-    }
-    for (int k = 0; k < kFillK; k++) {
-        const int m = t + k * kCgThreads;
-        if (m < n) map[list[m]] = m;
-    }
+    const SS_GLOBAL int *list = (const SS_GLOBAL int *)C.list + fo;
+    int *map = C.map + fo;
+    SS_GLOBAL uint32_t *code = (SS_GLOBAL uint32_t *)(C.code + fo);
+    SS_GLOBAL uint8_t *meta = (SS_GLOBAL uint8_t *)C.meta + fo;
+    for (int m = threadIdx.x; m < n; m += kCgThreads) map[list[m]] = m;
     __syncthreads();
-    unsigned nb01[kFillK], nb23[kFillK];  // id0 | id1 << 14 | degree << 28, id2 | id3 << 14
     double part = 0.0;
+    for (int m = threadIdx.x; m < n; m += kCgThreads) {
+        const FillEntry q = fill_entry(a, map, list[m], C.th, C.tw);
+        code[2 * (size_t)m] = q.w;
+        code[2 * (size_t)m + 1] = q.e;
+        meta[m] = (uint8_t)(q.deg | (q.n ? 8 : 0) | (q.s ? 16 : 0));
+        put(m, q.known);
+        part += q.known * q.known;
+    }
+    return part;
+}
+
+using Partials = double[kCgThreads / 64];
+
+template <typename T>
+__device__ __forceinline__ void fill_cg_lds(const FillChunk &C, T *__restrict__ data, Partials *sp, double *lp) {
+#pragma clang fp contract(off)
+    const int f = blockIdx.x, t = threadIdx.x, np = C.np;
+    const size_t fo = (size_t)f * np;
+    T *a = data + fo;
+    const SS_GLOBAL int *list = (const SS_GLOBAL int *)C.list + fo;
+    const int n = C.nmiss[f];
+    const int nk = (n + kCgThreads - 1) / kCgThreads;
+    for (int m = n + t; m < nk * kCgThreads; m += kCgThreads) lp[m] = 0.0;
+    if (t == 0) lp[kFillLds] = 0.0;
+    double part = fill_setup(C, a, fo, n, [&](int m, double known) { lp[m] = known; });
+    const SS_GLOBAL uint32_t *code = (const SS_GLOBAL uint32_t *)(C.code + fo);
+    const SS_GLOBAL uint8_t *meta = (const SS_GLOBAL uint8_t *)C.meta + fo;
+    double r[kFillK], x[kFillK];
+    unsigned nb[kFillK], deg[2] = {0, 0};  // deg: 3 bits per entry
+#pragma unroll
     for (int k = 0; k < kFillK; k++) {
         const int m = t + k * kCgThreads;
-        nb01[k] = nb23[k] = kNoNbr | (kNoNbr << 14);
-        if (m >= n) continue;
-        const int i = list[m], row = i % th, col = i / th;
-        // right-hand side: the known neighbours, W N S E (ascending index)
-        double s = 0.0;
-        unsigned d = 0, id[4] = {kNoNbr, kNoNbr, kNoNbr, kNoNbr};
-        const bool in[4] = {col > 0, row > 0, row + 1 < th, col + 1 < tw};
-        const int j[4] = {i - th, i - 1, i + 1, i + th};
-        for (int q = 0; q < 4; q++) {
-            if (!in[q]) continue;
-            d++;
-            const double v = a[j[q]];
-            if (isnan(v)) id[q] = (unsigned)map[j[q]];
-            else s += v;
+        x[k] = r[k] = 0.0;
+        nb[k] = kNoNbr | (kNoNbr << 15);
+        if (m < n) {
+            r[k] = lp[m];
+            const unsigned w = code[2 * (size_t)m], e = code[2 * (size_t)m + 1], q = meta[m];
+            nb[k] = min(w, kNoNbr) | (min(e, kNoNbr) << 15) | ((q & 8) ? kHasN : 0) | ((q & 16) ? kHasS : 0);
+            deg[k / 10] |= (q & 7) << (3 * (k % 10));
         }
-        nb01[k] = id[0] | (id[1] << 14) | (d << 28);
-        nb23[k] = id[2] | (id[3] << 14);
-        lr[m] = s;
-        lp[m] = s;
-        x[m] = 0.0;
-        part += s * s;
     }
-    // (A p)_m from the direction in LDS
-    auto apply = [&](int k, int m) {
-        const unsigned id[4] = {nb01[k] & kNoNbr, (nb01[k] >> 14) & kNoNbr, nb23[k] & kNoNbr,
-                                (nb23[k] >> 14) & kNoNbr};
+    // (A p)_m of entry k, p_m in p.  The word is opaque here: unpacked ahead
+    // of the loop its indices would take four registers per entry.
+    auto apply = [&](int k, double &p) {
+        const int m = t + k * kCgThreads;
+        unsigned c = nb[k], d = deg[k / 10];
+        asm volatile("" : "+v"(c), "+v"(d));
+        const unsigned w = min(c & kNoNbr, (unsigned)kFillLds), e = min((c >> 15) & kNoNbr, (unsigned)kFillLds);
+        const unsigned no = (c & kHasN) ? m - 1 : kFillLds, so = (c & kHasS) ? m + 1 : kFillLds;
+        p = lp[m];
         double s = 0.0;
-        for (int q = 0; q < 4; q++)
-            if (id[q] != kNoNbr) s += lp[id[q]];
-        return (double)(nb01[k] >> 28) * lp[m] - s;
+        s += lp[w];
+        s += lp[no];
+        s += lp[so];
+        s += lp[e];
+        return (double)((d >> (3 * (k % 10))) & 7u) * p - s;
     };
-    double rr_ = block_sum(part, sp);  // also orders the LDS writes before the reads
+    double rr_ = block_sum(part, sp[0]);  // also orders the direction's writes before the reads
     const double tol2 = 1e-26 * rr_;
     int it = 0;
     bool ok = rr_ <= tol2;
     while (!ok && it < C.maxit) {
         it++;
         part = 0.0;
+#pragma unroll
         for (int k = 0; k < kFillK; k++) {
-            const int m = t + k * kCgThreads;
-            if (m >= n) break;
-            part += lp[m] * apply(k, m);
+            if (k < nk) {
+                double p;
+                const double ap = apply(k, p);
+                part += p * ap;
+            }
         }
-        const double pap = block_sum(part, sp);
+        const double pap = block_sum(part, sp[1]);
         const double alpha = rr_ / pap;
         part = 0.0;
+#pragma unroll
         for (int k = 0; k < kFillK; k++) {
-            const int m = t + k * kCgThreads;
-            if (m >= n) break;
-            x[m] += alpha * lp[m];
-            const double rm = lr[m] - alpha * apply(k, m);
-            lr[m] = rm;
-            part += rm * rm;
+            if (k < nk) {
+                double p;
+                const double ap = apply(k, p);
+                x[k] += alpha * p;
+                r[k] -= alpha * ap;
+                part += r[k] * r[k];
+            }
         }
-        const double rn = block_sum(part, sp);
+        const double rn = block_sum(part, sp[0]);  // also orders these reads of p before its writes
         if (rn <= tol2) {
             ok = true;
             break;
         }
         const double beta = rn / rr_;
         rr_ = rn;
+#pragma unroll
         for (int k = 0; k < kFillK; k++) {
-            const int m = t + k * kCgThreads;
-            if (m >= n) break;
-            lp[m] = lr[m] + beta * lp[m];
+            if (k < nk) {
+                const int m = t + k * kCgThreads;
+                lp[m] = r[k] + beta * lp[m];
+            }
         }
         __syncthreads();
     }
+#pragma unroll
     for (int k = 0; k < kFillK; k++) {
         const int m = t + k * kCgThreads;
-        if (m < n) out[list[m]] = x[m];
+        if (m < n) a[list[m]] = to_class<T>(x[k]);
     }
     if (t == 0) C.status[f] = ok ? it : -1;
 }
 
-__global__ __launch_bounds__(kCgThreads) void k_fill_cg(FillChunk C) {
+// The same for larger regions: p of the first kFillLds entries in LDS, the
+// rest of it and the other vectors in global memory (57 bytes per entry and
+// iteration, at one CU's latency and bandwidth).  128 frames of which the
+// largest misses 20400 pixels take 14 ms; 29 ms through generic pointers with
+// p on the image grid.
+template <typename T>
+__device__ __forceinline__ void fill_cg_stream(const FillChunk &C, T *__restrict__ data, Partials *sp, double *lp) {
 #pragma clang fp contract(off)
-    __shared__ double sp[kCgThreads / 64];
-    const int f = blockIdx.x;
-    const int th = C.th, tw = C.tw, np = C.np;
+    const int f = blockIdx.x, t = threadIdx.x, np = C.np;
     const size_t fo = (size_t)f * np;
-    const double *a = C.a + fo;
-    double *out = C.out + fo;
-    const int *list = C.list + fo;
-    double *__restrict__ x = C.x + fo, *__restrict__ r = C.r + fo, *__restrict__ ap = C.ap + fo,
-                         *__restrict__ p = C.pfull + fo, *__restrict__ b = C.b + fo;
+    T *a = data + fo;
+    const SS_GLOBAL int *list = (const SS_GLOBAL int *)C.list + fo;
     const int n = C.nmiss[f];
-    if (n <= kFillLds) return;  // k_fill_cg_lds takes this frame
-    for (int i = threadIdx.x; i < np; i += kCgThreads) {
-        out[i] = a[i];
-        p[i] = 0.0;
-    }
-    __syncthreads();
-    if (n == 0 || n == np) {  // nothing to fill, or no known pixel (left as NaN)
-        if (threadIdx.x == 0) C.status[f] = 0;
-        return;
-    }
-    // right-hand side: the known neighbours, W N S E (ascending index)
-    double part = 0.0;
-    for (int m = threadIdx.x; m < n; m += kCgThreads) {
-        const int i = list[m], rr = i % th, cc = i / th;
-        double s = 0.0;
-        if (cc > 0 && !isnan(a[i - th])) s += a[i - th];
-        if (rr > 0 && !isnan(a[i - 1])) s += a[i - 1];
-        if (rr + 1 < th && !isnan(a[i + 1])) s += a[i + 1];
-        if (cc + 1 < tw && !isnan(a[i + th])) s += a[i + th];
-        b[m] = s;
+    const SS_GLOBAL uint32_t *code = (const SS_GLOBAL uint32_t *)(C.code + fo);
+    const SS_GLOBAL uint8_t *meta = (const SS_GLOBAL uint8_t *)C.meta + fo;
+    SS_GLOBAL double *x = (SS_GLOBAL double *)C.x + fo, *r = (SS_GLOBAL double *)C.r + fo,
+                     *gp = (SS_GLOBAL double *)C.p + fo;
+    double part = fill_setup(C, a, fo, n, [&](int m, double known) {
         x[m] = 0.0;
-        r[m] = s;
-        p[i] = s;
-        part += s * s;
-    }
-    double rr_ = block_sum(part, sp);  // also orders p's writes before the reads
+        r[m] = known;
+        if (m < kFillLds) lp[m] = known;
+        else gp[m] = known;
+    });
+    // Entries [m0, m1) of this thread, four at a time: all loads of the four
+    // first, p from LDS where the index lies there.
+    auto near = [&](unsigned i) { return lp[min(i, (unsigned)kFillLds - 1)]; };
+    auto passes = [&](auto &&body) {
+        for (int m0 = t; m0 < n; m0 += 4 * kCgThreads) {
+            unsigned w[4], e[4], q[4];
+            double p[4], vw[4], vn[4], vs[4], ve[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int m = min(m0 + u * kCgThreads, n - 1);
+                w[u] = code[2 * (size_t)m];
+                e[u] = code[2 * (size_t)m + 1];
+                q[u] = meta[m];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const unsigned m = min(m0 + u * kCgThreads, n - 1);
+                p[u] = near(m);
+                vw[u] = near(w[u]);
+                vn[u] = near(m - 1);
+                vs[u] = near(m + 1);
+                ve[u] = near(e[u]);
+                if (m >= (unsigned)kFillLds) p[u] = gp[m];
+                if (m > (unsigned)kFillLds) vn[u] = gp[m - 1];
+                if (m + 1 >= (unsigned)kFillLds) vs[u] = gp[min(m + 1, (unsigned)n - 1)];
+                if (w[u] != kAbsent && w[u] >= (unsigned)kFillLds) vw[u] = gp[w[u]];
+                if (e[u] != kAbsent && e[u] >= (unsigned)kFillLds) ve[u] = gp[e[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int m = m0 + u * kCgThreads;
+                double s = 0.0;
+                s += w[u] != kAbsent ? vw[u] : 0.0;
+                s += (q[u] & 8) ? vn[u] : 0.0;
+                s += (q[u] & 16) ? vs[u] : 0.0;
+                s += e[u] != kAbsent ? ve[u] : 0.0;
+                if (m < n) body(m, p[u], (double)(q[u] & 7u) * p[u] - s);
+            }
+        }
+    };
+    double rr_ = block_sum(part, sp[0]);  // also orders the direction's writes before the reads
     const double tol2 = 1e-26 * rr_;
     int it = 0;
     bool ok = rr_ <= tol2;
-    // Each pass is unrolled by 4 so that a thread has several entries' loads
-    // in flight; the partial sums still run over m = t, t + 1024, ... in order.
     while (!ok && it < C.maxit) {
         it++;
         part = 0.0;
-#pragma unroll 4
-        for (int m = threadIdx.x; m < n; m += kCgThreads) {
-            const int i = list[m], row = i % th, col = i / th;
-            double deg = 0.0, s = 0.0;
-            if (col > 0) { deg += 1.0; s += p[i - th]; }
-            if (row > 0) { deg += 1.0; s += p[i - 1]; }
-            if (row + 1 < th) { deg += 1.0; s += p[i + 1]; }
-            if (col + 1 < tw) { deg += 1.0; s += p[i + th]; }
-            const double pi = p[i], api = deg * pi - s;
-            ap[m] = api;
-            b[m] = pi;
-            part += pi * api;
-        }
-        const double pap = block_sum(part, sp);
+        passes([&](int, double p, double ap) { part += p * ap; });
+        const double pap = block_sum(part, sp[1]);
         const double alpha = rr_ / pap;
         part = 0.0;
-#pragma unroll 4
-        for (int m = threadIdx.x; m < n; m += kCgThreads) {
-            x[m] += alpha * b[m];
-            const double rm = r[m] - alpha * ap[m];
+        passes([&](int m, double p, double ap) {
+            x[m] += alpha * p;
+            const double rm = r[m] - alpha * ap;
             r[m] = rm;
             part += rm * rm;
-        }
-        const double rn = block_sum(part, sp);
+        });
+        const double rn = block_sum(part, sp[0]);
         if (rn <= tol2) {
             ok = true;
             break;
@@ -639,11 +719,27 @@ __global__ __launch_bounds__(kCgThreads) void k_fill_cg(FillChunk C) {
         const double beta = rn / rr_;
         rr_ = rn;
 #pragma unroll 4
-        for (int m = threadIdx.x; m < n; m += kCgThreads) p[list[m]] = r[m] + beta * b[m];
+        for (int m = t; m < kFillLds; m += kCgThreads) lp[m] = r[m] + beta * lp[m];
+#pragma unroll 4
+        for (int m = kFillLds + t; m < n; m += kCgThreads) gp[m] = r[m] + beta * gp[m];
         __syncthreads();
     }
-    for (int m = threadIdx.x; m < n; m += kCgThreads) out[list[m]] = x[m];
-    if (threadIdx.x == 0) C.status[f] = ok ? it : -1;
+    for (int m = t; m < n; m += kCgThreads) a[list[m]] = to_class<T>(x[m]);
+    if (t == 0) C.status[f] = ok ? it : -1;
+}
+
+template <typename T>
+__global__ __launch_bounds__(kCgThreads) void k_fill_cg(FillChunk C, T *__restrict__ data) {
+    __shared__ Partials sp[2];
+    __shared__ double lp[kFillLds + 1];
+    const int n = C.nmiss[blockIdx.x];
+    if (n == 0 || n == C.np) {  // nothing to fill, or no known pixel (left as NaN)
+        if (threadIdx.x == 0) C.status[blockIdx.x] = 0;
+    } else if (n <= kFillLds) {
+        fill_cg_lds(C, data, sp, lp);
+    } else {
+        fill_cg_stream(C, data, sp, lp);
+    }
 }
 
 size_t esize(ss_dtype t) { return t == SS_F64 ? 8 : t == SS_F32 ? 4 : 2; }
@@ -843,7 +939,7 @@ extern "C" ss_status ss_fill_gaps(ss_handle *h, ss_dtype type, const void *in, v
         return ss::handle_fail(h, SS_ERR_INVALID_ARGUMENT, "fill_gaps: frame too large");
     const int H = height, W = width;
     const size_t np = (size_t)H * W, es = esize(type);
-    const size_t perFrame = align256(np * 8) * 7 + align256(np * 4) + align256(8) * 2 +
+    const size_t perFrame = align256(np * 8) * 4 + align256(np * 4) * 2 + align256(np) + align256(8) * 2 +
                             (on_device ? 0 : align256(np * es));
     // work memory: half of what is free on the device or already held by the handle
     PCHK(hipSetDevice(ss::handle_device(h)));
@@ -867,14 +963,12 @@ extern "C" ss_status ss_fill_gaps(ss_handle *h, ss_dtype type, const void *in, v
     C.tw = W;
     C.np = (int)np;
     C.maxit = 200000;
-    double *da = (double *)take(np * 8 * B);
-    C.a = da;
-    C.out = (double *)take(np * 8 * B);
     C.x = (double *)take(np * 8 * B);
     C.r = (double *)take(np * 8 * B);
-    C.ap = (double *)take(np * 8 * B);
-    C.pfull = (double *)take(np * 8 * B);
-    C.b = (double *)take(np * 8 * B);
+    C.p = (double *)take(np * 8 * B);
+    C.code = (uint2 *)take(np * 8 * B);
+    C.meta = (uint8_t *)take(np * B);
+    C.map = (int *)take(np * 4 * B);
     C.list = (int *)take(np * 4 * B);
     C.nmiss = (int *)take(4 * (size_t)B);
     C.status = (int *)take(4 * (size_t)B);
@@ -885,20 +979,17 @@ extern "C" ss_status ss_fill_gaps(ss_handle *h, ss_dtype type, const void *in, v
         const size_t cnt = np * nb;
         const char *src = (const char *)in + es * np * f0;
         char *dst = (char *)out + es * np * f0;
-        const char *work = src;
-        if (!on_device) {
-            PCHK(hipMemcpyAsync(dio, src, es * cnt, hipMemcpyHostToDevice, s));
-            work = dio;
-        }
-        const dim3 g1d((unsigned)((cnt + 255) / 256));
-        if (type == SS_F64) hipLaunchKernelGGL(k_to_double<double>, g1d, dim3(256), 0, s, (const double *)work, da, cnt);
-        else hipLaunchKernelGGL(k_to_double<float>, g1d, dim3(256), 0, s, (const float *)work, da, cnt);
-        hipLaunchKernelGGL(k_fill_list, dim3(nb), dim3(kCgThreads), 0, s, C);
-        hipLaunchKernelGGL(k_fill_cg_lds, dim3(nb), dim3(kCgThreads), 0, s, C);
-        hipLaunchKernelGGL(k_fill_cg, dim3(nb), dim3(kCgThreads), 0, s, C);
-        char *o = on_device ? dst : dio;
-        if (type == SS_F64) hipLaunchKernelGGL(k_from_double<double>, g1d, dim3(256), 0, s, C.out, (double *)o, cnt);
-        else hipLaunchKernelGGL(k_from_double<float>, g1d, dim3(256), 0, s, C.out, (float *)o, cnt);
+        // only the missing pixels are written: the frames are filled in place
+        char *work = on_device ? dst : dio;
+        if (!on_device) PCHK(hipMemcpyAsync(dio, src, es * cnt, hipMemcpyHostToDevice, s));
+        else if (src != dst) PCHK(hipMemcpyAsync(dst, src, es * cnt, hipMemcpyDeviceToDevice, s));
+        auto fill = [&](auto *frames) {
+            using T = std::remove_pointer_t<decltype(frames)>;
+            hipLaunchKernelGGL(k_fill_list<T>, dim3(nb), dim3(kCgThreads), 0, s, C, (const T *)frames);
+            hipLaunchKernelGGL(k_fill_cg<T>, dim3(nb), dim3(kCgThreads), 0, s, C, frames);
+        };
+        if (type == SS_F64) fill((double *)work);
+        else fill((float *)work);
         PCHK(hipGetLastError());
         PCHK(hipMemcpyAsync(status.data(), C.status, 4 * nb, hipMemcpyDeviceToHost, s));
         if (!on_device) PCHK(hipMemcpyAsync(dst, dio, es * cnt, hipMemcpyDeviceToHost, s));
