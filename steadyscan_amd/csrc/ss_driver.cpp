@@ -4,7 +4,8 @@
 //
 // The reference aligns its sets one after another; here every set of the
 // stack is one group of a single batched submission (ss_align_batch), with
-// the template and geometry resident.  The set partition, the +1-frame
+// the template and geometry resident; the raw frames go to the GPU once and are
+// filtered and packed there.  The set partition, the +1-frame
 // overlap, the prefiltering, the unpacking and the per-frame success tests
 // follow the reference line by line.
 #include <algorithm>
@@ -19,6 +20,7 @@
 #include <vector>
 
 #include "steadyscan.h"
+#include "ss_pack.h"
 #include "ss_pinned.h"
 
 namespace {
@@ -104,8 +106,8 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
     // geometry block matrices and the template gradients (steady_scan.m:166-179)
     std::vector<double> frac(nbm), bx(nbm), by(nbm);
     std::vector<uint8_t> bm(nbm);
-    std::vector<int32_t> minpts(nk);
-    st = ss_geometry_init(geom, nullptr, nullptr, nullptr, nullptr, frac.data(), bx.data(), by.data(), bm.data(),
+    std::vector<int32_t> minpts(nk), knot((size_t)Hc * Wc);
+    st = ss_geometry_init(geom, knot.data(), nullptr, nullptr, nullptr, frac.data(), bx.data(), by.data(), bm.data(),
                           minpts.data());
     if (st) return st;
     const double nan = std::numeric_limits<double>::quiet_NaN();
@@ -147,32 +149,59 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         zeros.assign((size_t)nk * n_frames, 0.0);
         est_dx = est_dy = zeros.data();
     }
-    const size_t esz = elem_size(type), rawFrame = (size_t)geom->nlines * geom->linewidth * esz;
-    // prefilter_foralignment of each set's (uncropped) frames (steady_scan.m:228);
-    // a frame's result does not depend on its set, so the stack is filtered once
-    std::vector<char> filtered;
-    if (ds->pregauss > 0 || ds->mednorm) {
-        filtered.resize(rawFrame * n_frames);
-        st = ss_prefilter(h, type, frames, filtered.data(), geom->nlines, geom->linewidth, n_frames, ds->pregauss,
-                          ds->mednorm, 0);
-        if (st) {
-            ss_release(h, tid);
-            ss_release(h, gid);
-            return st;
-        }
-        frames = filtered.data();
+    const size_t esz = elem_size(type), rawPix = (size_t)geom->nlines * geom->linewidth, rawFrame = rawPix * esz;
+    // the raw pixel of every block-matrix element: a block lists its pixels
+    // column by column (steady_scan.m:229-234, 601-613) of the cropped image
+    // (steady_scan.m:830-834)
+    if (rawPix >= ss::kNoPixel) return SS_ERR_INVALID_ARGUMENT;
+    std::vector<uint32_t> at(nbm, ss::kNoPixel);
+    {
+        std::vector<size_t> fill(nb, 0);
+        for (int j = 0; j < Wc; j++)
+            for (int i = 0; i < Hc; i++) {
+                const int b = knot[(size_t)j * Hc + i] - 1;
+                at[(size_t)b * fh + fill[b]++] = (uint32_t)((size_t)(j + geom->cropping[0]) * geom->nlines + (i + geom->cropping[2]));
+            }
     }
-    std::vector<std::vector<char>> packed(nsets);
+    // Device memory of the stack: the table, the used flags, the packed
+    // frames (a set's are consecutive, its last one the next set's first),
+    // the sets' masks, and a piece of raw frames to upload, filter and pack.
+    size_t cols = 0;
+    for (int n : nset) cols += (size_t)n * nb;
+    auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const int piece = (int)std::max<size_t>(1, std::min<size_t>(n_frames, ((size_t)256 << 20) / rawFrame));
+    const size_t oUsed = al(nbm * sizeof(uint32_t)), oPacked = oUsed + al(cols), oMask = oPacked + al(nbm * esz * n_frames),
+                 oRaw = oMask + al(cols * fh);
+    char *dev = (char *)ss::handle_stack(h, oRaw + rawFrame * piece, &st);
+    auto release = [&] {
+        ss_release(h, tid);
+        ss_release(h, gid);
+        return st;
+    };
+    if (st) return release();
+    void *stream = ss::handle_raw_stream(h);
+    st = ss::handle_upload(h, dev, at.data(), nbm * sizeof(uint32_t));
+    for (int f0 = 0; f0 < n_frames && !st; f0 += piece) {
+        const int n = std::min(piece, n_frames - f0);
+        st = ss::handle_upload(h, dev + oRaw, (const char *)frames + rawFrame * f0, rawFrame * n);
+        // prefilter_foralignment of each set's (uncropped) frames (steady_scan.m:228);
+        // a frame's result does not depend on its set, so the stack is filtered once
+        if (!st && (ds->pregauss > 0 || ds->mednorm))
+            st = ss_prefilter(h, type, dev + oRaw, dev + oRaw, geom->nlines, geom->linewidth, n, ds->pregauss, ds->mednorm, 1);
+        if (!st && ss::pack_frames(stream, (const uint32_t *)dev, (int)nbm, (int)esz, dev + oRaw, rawPix, n,
+                                   dev + oPacked + nbm * esz * f0))
+            st = SS_ERR_DEVICE;
+    }
+    if (st) return release();
     std::vector<ss_group_in> gin(nsets);
     std::vector<ss_settings> gs(nsets, *s);
     std::vector<ss_group_out> gout(nsets);
     std::vector<std::vector<double>> kx(nsets), ky(nsets), fc(nsets), rr(nsets);
-    std::vector<std::vector<uint8_t>> mk(nsets);
+    std::vector<size_t> col0(nsets);  // a set's first column of the masks and used flags
+    size_t col = 0;
     for (int i = 0; i < nsets; i++) {
         const int n = nset[i];
-        packed[i].resize(nbm * n * esz);
-        st = ss_pack_frames(geom, type, (const char *)frames + (size_t)start[i] * rawFrame, n, packed[i].data());
-        if (st) break;
+        col0[i] = col;
         ss_group_in &g = gin[i];
         std::memset(&g, 0, sizeof(g));
         g.frame_h = fh;
@@ -184,7 +213,8 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         g.template_id = tid;
         g.geometry_id = gid;
         g.data_type = type;
-        g.data = packed[i].data();
+        g.data = dev + oPacked + nbm * esz * start[i];
+        g.data_on_device = 1;
         g.init_x = est_dx;
         g.init_y = est_dy;
         g.min_points = minpts.data();
@@ -192,19 +222,21 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         ky[i].resize((size_t)nk * n);
         fc[i].resize(n);
         rr[i].resize(n);
-        mk[i].resize(nbm * n);
         ss_group_out &o = gout[i];
         std::memset(&o, 0, sizeof(o));
         o.knots_x = kx[i].data();
         o.knots_y = ky[i].data();
         o.frame_corr = fc[i].data();
         o.residrms = rr[i].data();
-        o.mask = mk[i].data();
+        o.mask = (uint8_t *)dev + oMask + col * fh;
+        o.mask_on_device = 1;
+        col += (size_t)n * nb;
     }
-    if (!st) st = ss_align_batch(h, nsets, gin.data(), gs.data(), gout.data());
-    ss_release(h, tid);
-    ss_release(h, gid);
-    if (st) return st;
+    st = ss_align_batch(h, nsets, gin.data(), gs.data(), gout.data());
+    std::vector<uint8_t> usedAll(cols);
+    if (!st && ss::used_blocks(stream, (const uint8_t *)dev + oMask, fh, (int)cols, (uint8_t *)dev + oUsed)) st = SS_ERR_DEVICE;
+    if (!st) st = ss::handle_download(h, usedAll.data(), dev + oUsed, cols);
+    if (release()) return st;
     // unpacking and success tests (steady_scan.m:246-284)
     for (int i = 0; i < nsets; i++) {
         for (int sj = 0; sj + 1 < nset[i]; sj++) {
@@ -216,13 +248,9 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
             if (out->iter_used) out->iter_used[j] = gout[i].iterations;
             if (out->residrms) out->residrms[j] = rr[i][sj];
             // blocks with at least one masked pixel
-            std::vector<uint8_t> used(nb, 0);
-            bool any = false;
-            for (int b = 0; b < nb; b++) {
-                const uint8_t *col = mk[i].data() + ((size_t)sj * nb + b) * fh;
-                for (int r = 0; r < fh && !used[b]; r++) used[b] = col[r] && bm[(size_t)b * fh + r];
-                any |= used[b] != 0;
-            }
+            const uint8_t *u = usedAll.data() + col0[i] + (size_t)sj * nb;
+            const std::vector<uint8_t> used(u, u + nb);
+            const bool any = std::find(u, u + nb, 1) != u + nb;
             if (!any) {
                 if (out->failed) out->failed[j] = 1;
                 if (out->corr) out->corr[j] = nan;

@@ -23,6 +23,7 @@
 
 #include "ss_device.h"
 #include "ss_host.h"
+#include "ss_pack.h"
 #include "ss_pinned.h"
 #include "steadyscan.h"
 
@@ -138,6 +139,8 @@ struct ss_handle {
     size_t harenaBytes = 0;
     void *scratch = nullptr;  // work memory of the reconstruction
     size_t scratchBytes = 0;
+    void *stack = nullptr;    // the driver's frame stack
+    size_t stackBytes = 0;
     Profile prof;
     // the tick's launches, captured once per group table and replayed
     bool useGraph = true;
@@ -605,6 +608,26 @@ void stage_frames(const Plan &P, char *HS, size_t b, size_t e) {
         const size_t es = img_size(P.imgType);
         std::memcpy(stage + b * es, (const char *)P.in->data + b * es, (e - b) * es);
     }
+}
+
+// body(b, e) over [0, n) in pieces of about `step` on up to 16 host threads;
+// pieces whose thread cannot be started run on the calling thread.
+template <typename Body>
+void parallel_pieces(size_t n, size_t step, Body &&body) {
+    const size_t pieces = (n + step - 1) / step;
+    const size_t nt = std::min<size_t>(pieces, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
+    auto run = [&](size_t t) {
+        for (size_t k = t; k < pieces; k += nt) body(k * step, std::min(n, (k + 1) * step));
+    };
+    std::vector<std::thread> pool;
+    size_t started = 1;
+    try {
+        for (; started < nt; started++) pool.emplace_back(run, started);
+    } catch (...) {  // no thread available: the rest runs here
+    }
+    run(0);
+    for (size_t t = started; t < nt; t++) run(t);
+    for (auto &th : pool) th.join();
 }
 
 // The host frames of all groups of a batch into their staging (group gi at
@@ -1657,6 +1680,57 @@ void *handle_scratch(ss_handle *h, size_t bytes, ss_status *st) {
 
 size_t handle_scratch_held(const ss_handle *h) { return h->scratchBytes; }
 
+void *handle_raw_stream(const ss_handle *h) { return (void *)h->stream; }
+
+void *handle_stack(ss_handle *h, size_t bytes, ss_status *st) {
+    *st = SS_OK;
+    if (h->stackBytes >= bytes) return h->stack;
+    (void)hipSetDevice(h->device);
+    if (h->stack) {
+        (void)hipStreamSynchronize(h->stream);
+        (void)hipFree(h->stack);
+        h->stack = nullptr;
+        h->stackBytes = 0;
+    }
+    if (hipMalloc(&h->stack, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        h->stack = nullptr;
+        *st = fail(h, SS_ERR_OUT_OF_MEMORY, "unable to allocate device memory for the frame stack");
+        return nullptr;
+    }
+    h->stackBytes = bytes;
+    return h->stack;
+}
+
+ss_status handle_upload(ss_handle *h, void *dst, const void *src, size_t bytes) {
+    HIPCHK(hipSetDevice(h->device));
+    // two halves of the staging: the host fills one while the other uploads
+    const size_t half = std::min(bytes, (size_t)32 << 20);
+    ss_status st = ensure_arena(h, 0, 2 * half);
+    if (st) return st;
+    for (int i = 0; i < 2; i++)
+        if (!h->tickDone[i]) HIPCHK(hipEventCreateWithFlags(&h->tickDone[i], hipEventDisableTiming));
+    int k = 0;
+    for (size_t o = 0; o < bytes; o += half, k++) {
+        const size_t n = std::min(half, bytes - o);
+        char *stage = (char *)h->harena + (k & 1) * half;
+        if (k >= 2) HIPCHK(hipEventSynchronize(h->tickDone[k & 1]));
+        const char *from = (const char *)src + o;
+        parallel_pieces(n, (size_t)4 << 20, [&](size_t b, size_t e) { std::memcpy(stage + b, from + b, e - b); });
+        HIPCHK(hipMemcpyAsync((char *)dst + o, stage, n, hipMemcpyHostToDevice, h->stream));
+        HIPCHK(hipEventRecord(h->tickDone[k & 1], h->stream));
+    }
+    HIPCHK(hipStreamSynchronize(h->stream));
+    return SS_OK;
+}
+
+ss_status handle_download(ss_handle *h, void *dst, const void *src, size_t bytes) {
+    HIPCHK(hipSetDevice(h->device));
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
+    return SS_OK;
+}
+
 void *pinned_alloc(size_t bytes) {
     void *p = nullptr;
     if (hipHostMalloc(&p, bytes, hipHostMallocPortable) != hipSuccess) {
@@ -1723,6 +1797,7 @@ void ss_destroy(ss_handle *h) {
     if (h->arena) e = hipFree(h->arena);
     if (h->harena) e = hipHostFree(h->harena);
     if (h->scratch) e = hipFree(h->scratch);
+    if (h->stack) e = hipFree(h->stack);
     if (h->trialTable) e = hipFree(h->trialTable);
     if (h->trialStage) e = hipHostFree(h->trialStage);
     if (h->stream) e = hipStreamDestroy(h->stream);
