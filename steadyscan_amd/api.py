@@ -351,7 +351,7 @@ def align_group_to_template(flags, template_image, xgrad, ygrad, tfrac, basex, b
     if "E" in opts:
         print(f"Execution terminated:{N.STOP_NAMES[go.stop_criterion]}\niterations: {go.iterations}")
     outs = [kx.reshape(-1, 1), ky.reshape(-1, 1), fc.reshape(-1, 1), np.int32(go.iterations),
-            None if mask is None else mask.astype(bool), rr.reshape(-1, 1), go.device_init_time,
+            None if mask is None else mask.view(bool), rr.reshape(-1, 1), go.device_init_time,
             icorr if (icorr is not None and "C" in opts) else np.zeros((0, 0))]
     empty = np.zeros((0, 0))
     # 9, 10 ('t'/'T'), 11 ('c'), 12 ('e'), 13 ('P'), 14
@@ -453,7 +453,7 @@ def _prepare_call(a, h, s, gi, go, with_mask, linesearch_candidates, keep):
 
 def _collect(r, go):
     if r["mask"] is not None:
-        r["mask"] = r["mask"].astype(bool)
+        r["mask"] = r["mask"].view(bool)  # the bytes are 0 and 1
     r.update(iterations=go.iterations, stop_criterion=N.STOP_NAMES[go.stop_criterion],
              half_iterations=go.half_iterations, linesearch_rounds=go.linesearch_rounds,
              linesearch_tries=go.linesearch_tries)

@@ -67,23 +67,28 @@ uint32_t to_bf16(double v) {
     return u >> 16;
 }
 
+// Row-major pairs of a column-major array, a tile at a time, so that both the
+// source's columns and the pairs' rows stay within a few cache lines.
+template <typename P, typename F>
+void fill_pairs(int th, int tw, std::vector<P> &out, F &&pair) {
+    constexpr int kTile = 16;
+    out.resize((size_t)th * tw);
+    for (int y0 = 0; y0 < th; y0 += kTile)
+        for (int x0 = 0; x0 < tw; x0 += kTile)
+            for (int iy = y0; iy < std::min(th, y0 + kTile); iy++)
+                for (int ix = x0; ix < std::min(tw, x0 + kTile); ix++) out[(size_t)iy * tw + ix] = pair(iy, ix);
+}
+
 // Gradient pairs as packed BF16 (the Jacobian factors of mixed precision):
 // gxv low half xgrad[iy][ix], high half xgrad[iy+1][ix]; gyh low half
 // ygrad[iy][ix], high half ygrad[iy][ix+1].  Always built, also when the
 // gradients are the template's forward differences.
 void gradient_pairs_bf16(int th, int tw, const double *xg, const double *yg, std::vector<uint32_t> &gxv,
                          std::vector<uint32_t> &gyh) {
-    const size_t n = (size_t)th * tw;
     auto at = [&](const double *a, int iy, int ix) { return a[(size_t)ix * th + iy]; };
     auto pack = [](double lo, double hi) { return to_bf16(lo) | (to_bf16(hi) << 16); };
-    gxv.assign(n, 0u);
-    gyh.assign(n, 0u);
-    for (int iy = 0; iy < th; iy++)
-        for (int ix = 0; ix < tw; ix++) {
-            const size_t o = (size_t)iy * tw + ix;
-            gxv[o] = pack(at(xg, iy, ix), iy + 1 < th ? at(xg, iy + 1, ix) : 0.0);
-            gyh[o] = pack(at(yg, iy, ix), ix + 1 < tw ? at(yg, iy, ix + 1) : 0.0);
-        }
+    fill_pairs(th, tw, gxv, [&](int iy, int ix) { return pack(at(xg, iy, ix), iy + 1 < th ? at(xg, iy + 1, ix) : 0.0); });
+    fill_pairs(th, tw, gyh, [&](int iy, int ix) { return pack(at(yg, iy, ix), ix + 1 < tw ? at(yg, iy, ix + 1) : 0.0); });
 }
 struct GeometryHost {
     std::vector<float4> tab;
@@ -275,46 +280,36 @@ ss_status ensure_arena(ss_handle *h, size_t bytes, size_t hostBytes) {
 template <typename P, typename S>
 void template_pairs(int th, int tw, const double *t, const double *xg, const double *yg, bool fd,
                     std::vector<P> &tp, std::vector<P> &gxv, std::vector<P> &gyh) {
-    const size_t n = (size_t)th * tw;
-    auto at = [&](const double *a, int iy, int ix) { return (S)a[(size_t)ix * th + iy]; };
-    tp.assign(n, P{});
-    for (int iy = 0; iy < th; iy++)
-        for (int ix = 0; ix < tw; ix++) {
-            P &q = tp[(size_t)iy * tw + ix];
-            q.x = at(t, iy, ix);
-            q.y = ix + 1 < tw ? at(t, iy, ix + 1) : (S)0;
-        }
+    auto pair = [](double x, double y) {
+        P q;
+        q.x = (S)x;
+        q.y = (S)y;
+        return q;
+    };
+    auto at = [&](const double *a, int iy, int ix) { return a[(size_t)ix * th + iy]; };
+    fill_pairs(th, tw, tp, [&](int iy, int ix) { return pair(at(t, iy, ix), ix + 1 < tw ? at(t, iy, ix + 1) : 0.0); });
     gxv.clear();
     gyh.clear();
     if (fd) return;
-    gxv.assign(n, P{});
-    gyh.assign(n, P{});
-    for (int iy = 0; iy < th; iy++)
-        for (int ix = 0; ix < tw; ix++) {
-            const size_t o = (size_t)iy * tw + ix;
-            gxv[o].x = at(xg, iy, ix);
-            gxv[o].y = iy + 1 < th ? at(xg, iy + 1, ix) : (S)0;
-            gyh[o].x = at(yg, iy, ix);
-            gyh[o].y = ix + 1 < tw ? at(yg, iy, ix + 1) : (S)0;
-        }
+    fill_pairs(th, tw, gxv, [&](int iy, int ix) { return pair(at(xg, iy, ix), iy + 1 < th ? at(xg, iy + 1, ix) : 0.0); });
+    fill_pairs(th, tw, gyh, [&](int iy, int ix) { return pair(at(yg, iy, ix), ix + 1 < tw ? at(yg, iy, ix + 1) : 0.0); });
 }
 
 void convert_template(int th, int tw, const double *t, const double *xg, const double *yg, bool wantF,
                       bool wantD, bool wantB, TemplateHost &out, int &gradFD) {
-    auto T = [&](int iy, int ix) { return t[(size_t)ix * th + iy]; };
-    auto GX = [&](int iy, int ix) { return xg[(size_t)ix * th + iy]; };
-    auto GY = [&](int iy, int ix) { return yg[(size_t)ix * th + iy]; };
     double tmax = 0;
     for (size_t i = 0; i < (size_t)th * tw; i++) tmax = std::max(tmax, std::fabs(t[i]));
-    // every gradient value the warp can read: xgrad(:, 1:end-1), ygrad(1:end-1, :)
-    bool fd = true;
+    // every gradient value the warp can read: xgrad(:, 1:end-1), ygrad(1:end-1, :),
+    // column by column as they lie in memory
+    int bad = 0;
     const double tol = 1e-12 * std::max(1.0, tmax);
-    for (int iy = 0; iy < th && fd; iy++)
-        for (int ix = 0; ix + 1 < tw; ix++)
-            if (!(std::fabs(GX(iy, ix) - (T(iy, ix + 1) - T(iy, ix))) <= tol)) { fd = false; break; }
-    for (int iy = 0; iy + 1 < th && fd; iy++)
-        for (int ix = 0; ix < tw; ix++)
-            if (!(std::fabs(GY(iy, ix) - (T(iy + 1, ix) - T(iy, ix))) <= tol)) { fd = false; break; }
+    for (int ix = 0; ix < tw && !bad; ix++) {
+        const double *c = t + (size_t)ix * th, *e = c + th, *gx = xg + (size_t)ix * th, *gy = yg + (size_t)ix * th;
+        if (ix + 1 < tw)
+            for (int iy = 0; iy < th; iy++) bad |= !(std::fabs(gx[iy] - (e[iy] - c[iy])) <= tol);
+        for (int iy = 0; iy + 1 < th; iy++) bad |= !(std::fabs(gy[iy] - (c[iy + 1] - c[iy])) <= tol);
+    }
+    const bool fd = !bad;
     gradFD = fd ? 1 : 0;
     if (wantF) template_pairs<float2, float>(th, tw, t, xg, yg, fd, out.tp, out.gxv, out.gyh);
     if (wantD) template_pairs<double2, double>(th, tw, t, xg, yg, fd, out.tpD, out.gxvD, out.gyhD);
@@ -330,12 +325,13 @@ void convert_geometry(int fh, int nb, const double *frac, const double *bx, cons
     const size_t n = (size_t)fh * nb;
     g.frameH = fh;
     g.nb = nb;
-    bool uniform = true, allMask = true;
-    for (int b = 0; b < nb && uniform; b++)
-        for (int r = 0; r < fh; r++)
-            if (frac[(size_t)b * fh + r] != frac[r]) { uniform = false; break; }
-    for (size_t i = 0; i < n; i++)
-        if (!bm[i]) { allMask = false; break; }
+    bool uniform = true;
+    for (int b = 0; b < nb && uniform; b++) {
+        int differ = 0;
+        for (int r = 0; r < fh; r++) differ |= frac[(size_t)b * fh + r] != frac[r];
+        uniform = !differ;
+    }
+    const bool allMask = !std::memchr(bm, 0, n);
     g.fracUniform = uniform ? 1 : 0;
     // affine detection: L = first row where base_x changes within block 0
     g.affine = 0;
@@ -352,16 +348,17 @@ void convert_geometry(int fh, int nb, const double *frac, const double *bx, cons
                          gyj = J > 1 ? at(by, 0, L) - gy0 : 0.0, gyb = nb > 1 ? at(by, 1, 0) - gy0 : 0.0;
             const double f0 = frac[0], fi = L > 1 ? frac[1] - f0 : 0.0, fj = J > 1 ? frac[L] - f0 : 0.0;
             bool ok = true;
-            const double tol = 1e-12;
+            const double tol = 1e-12, tolx = tol * std::max(1.0, std::fabs(gx0) + std::fabs(gxj) * J),
+                         toly = tol * std::max(1.0, std::fabs(gy0) + std::fabs(gyb) * nb);
             for (int b = 0; b < nb && ok; b++)
-                for (int r = 0; r < fh; r++) {
-                    const int j = r / L, i = r % L;
-                    if (std::fabs(at(bx, b, r) - (gx0 + gxj * j + gxi * i)) > tol * std::max(1.0, std::fabs(gx0) + std::fabs(gxj) * J) ||
-                        std::fabs(at(by, b, r) - (gy0 + gyb * b + gyj * j + gyi * i)) > tol * std::max(1.0, std::fabs(gy0) + std::fabs(gyb) * nb) ||
-                        std::fabs(at(frac, b, r) - (f0 + fj * j + fi * i)) > tol) {
-                        ok = false;
-                        break;
-                    }
+                for (int j = 0; j < J && ok; j++) {
+                    const size_t o = (size_t)b * fh + (size_t)j * L;
+                    int off = 0;
+                    for (int i = 0; i < L; i++)
+                        off |= (std::fabs(bx[o + i] - (gx0 + gxj * j + gxi * i)) > tolx) |
+                               (std::fabs(by[o + i] - (gy0 + gyb * b + gyj * j + gyi * i)) > toly) |
+                               (std::fabs(frac[o + i] - (f0 + fj * j + fi * i)) > tol);
+                    ok = !off;
                 }
             if (ok) {
                 g.affine = 1;
