@@ -692,11 +692,24 @@ __device__ __forceinline__ Aff aff_sub(const Aff &a, const Aff &b) {
 struct RedEq {  // reduced (interface) equation, general 2x2 blocks
     M2 A, B, C;
     double2 d, x;
+    double pad;  // neighbouring equations start in different LDS banks
 };
 
 struct InteriorRow {  // forward-eliminated interior row: Bh^{-1} and rhs
     M2 Bi;
     Aff R;
+};
+
+// The solve kernel's LDS besides the equations: the interface system, before
+// it the first interiors' affine forms, after it the filter's partial scans.
+struct SolveLds {
+    union {
+        RedEq red[kSolveWG];
+        Aff first[kSolveWG];
+        double scan[kSolveWG][4];
+    };
+    int hasInt[kSolveWG];
+    __device__ SolveLds() {}
 };
 
 // Solver id 0 (SolverCuSparse::solve, cusparsesolver.cu:41-174): incomplete
@@ -816,14 +829,14 @@ __device__ __forceinline__ bool knot_used(const double *__restrict__ S, const in
 }
 
 // Level-0 equations of knots tid, tid + kSolveWG, ... (d_fillDiagonals /
-// d_fillJTr entries, lambda extension), and the usage flags of the same
-// knots into `used`.  Each knot takes its own and its neighbours' usage from
-// the column counts, so that no pass over the flags has to come first.  The
-// pointers do not alias, so the next knot's loads may be issued before this
-// knot's equation is stored.  E may point to LDS.
-__device__ __forceinline__ void level0_equations(const double *__restrict__ S, const int *__restrict__ minPts,
-                                                 uint8_t *__restrict__ used, Eq0 *__restrict__ E, int n, int nb,
-                                                 double lambda, int fracUniform, int tid) {
+// d_fillJTr entries, lambda extension) into put(k, equation, used).  Each
+// knot takes its own and its neighbours' usage from the column counts, so
+// that no pass over the flags has to come first.  The pointers do not alias,
+// so the next knot's loads may be issued before this knot's equation is
+// stored.
+template <typename Put>
+__device__ __forceinline__ void level0_equations(const double *__restrict__ S, const int *__restrict__ minPts, int n,
+                                                 int nb, double lambda, int fracUniform, int tid, Put &&put) {
 #pragma unroll 4
     for (int k = tid; k < n; k += kSolveWG) {
         Eq0 e;
@@ -831,7 +844,6 @@ __device__ __forceinline__ void level0_equations(const double *__restrict__ S, c
         const bool u = knot_used(S, minPts, k, n, nb);
         const bool up = k > 0 && knot_used(S, minPts, k - 1, n, nb);
         const bool un = (k + 1 < n) && knot_used(S, minPts, k + 1, n, nb);
-        used[k] = u ? 1 : 0;
         if (!u) {
             e = Eq0{1, 0, 1, 0, 0, 0, 0, 0};
         } else {
@@ -860,29 +872,81 @@ __device__ __forceinline__ void level0_equations(const double *__restrict__ S, c
             e.d0 = jx;
             e.d1 = jy;
         }
-        E[k] = e;
+        put(k, e, u);
     }
 }
+
+// Where the equations of a group lie.  Few enough: in LDS, in order.  More:
+// in memory as 16-byte pieces [row of the partition][piece][thread], so that
+// the threads, each walking the rows of its own partition, load and store
+// consecutive addresses.
+struct LdsRows {
+    Eq0 *E;
+    int m;
+    __device__ __forceinline__ Eq0 load(int t, int r) const { return E[t * m + r]; }
+    __device__ __forceinline__ Eq0 knot(int k) const { return E[k]; }
+    __device__ __forceinline__ void put(int k, const Eq0 &e) const { E[k] = e; }
+    __device__ __forceinline__ void put_rhs(int k, double d0, double d1) const {
+        E[k].d0 = d0;
+        E[k].d1 = d1;
+    }
+};
+struct MemRows {
+    SS_GLOBAL d2v *E;
+    int m;
+    __device__ __forceinline__ SS_GLOBAL d2v *at(int t, int r) const { return E + (size_t)r * 4 * kSolveWG + t; }
+    __device__ __forceinline__ Eq0 load(int t, int r) const {
+        const SS_GLOBAL d2v *q = at(t, r);
+        const d2v a = q[0], b = q[kSolveWG], c = q[2 * kSolveWG], d = q[3 * kSolveWG];
+        return Eq0{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+    }
+    __device__ __forceinline__ Eq0 knot(int k) const { return load(k / m, k % m); }
+    __device__ __forceinline__ void put(int k, const Eq0 &e) const {
+        SS_GLOBAL d2v *q = at(k / m, k % m);
+        q[0] = d2v{e.b0, e.b1};
+        q[kSolveWG] = d2v{e.b2, e.c0};
+        q[2 * kSolveWG] = d2v{e.c1, e.c2};
+        q[3 * kSolveWG] = d2v{e.d0, e.d1};
+    }
+    __device__ __forceinline__ void put_rhs(int k, double d0, double d1) const {
+        at(k / m, k % m)[3 * kSolveWG] = d2v{d0, d1};
+    }
+};
+// The solution, in LDS or in memory.
+struct Solution {
+    double2 *lds;
+    SS_GLOBAL d2v *mem;
+    bool inLds;
+    __device__ __forceinline__ double2 get(int k) const {
+        if (inLds) return lds[k];
+        const d2v v = mem[k];
+        return make_double2(v.x, v.y);
+    }
+    __device__ __forceinline__ void set(int k, double2 v) const {
+        if (inLds) lds[k] = v;
+        else mem[k] = d2v{v.x, v.y};
+    }
+};
 
 // Interface system of the partitioned solve: thread t < P contributes the
 // equation of its partition's last knot z_t in terms of z_{t-1} and z_{t+1}
 // (its last interior row as lastA, the next partition's first interior row
 // as firstAff[t + 1]); cyclic reduction solves it.  Called by all threads;
 // returns z_t and z_{t-1} (0 for t = 0).
-__device__ void solve_interfaces(bool interior, const Aff &first, const Aff &lastA, const Eq0 &q, const M2 &A,
-                                 Aff *firstAff, int P, int tid, double2 &zo, double2 &zp) {
-    __shared__ RedEq red[kSolveWG];
-    __shared__ int hasInt[kSolveWG];
+__device__ __forceinline__ void solve_interfaces(bool interior, const Aff &first, const Aff &lastA, const Eq0 &q,
+                                                 const M2 &A, SolveLds &S, int P, int tid, double2 &zo, double2 &zp) {
+    RedEq *red = S.red;
     if (tid < P) {
-        hasInt[tid] = interior ? 1 : 0;
-        firstAff[tid] = first;
+        S.hasInt[tid] = interior ? 1 : 0;
+        S.first[tid] = first;
     }
     __syncthreads();
+    // x_{j+1}: first interior of partition t+1, or z_{t+1}
+    Aff F{make_double2(0, 0), zero2(), eye2()};
+    if (tid + 1 < P && S.hasInt[tid + 1]) F = S.first[tid + 1];
+    __syncthreads();  // the interface system takes the affine forms' memory
     if (tid < P) {
         const M2 C = sym(q.c0, q.c1, q.c2);
-        // x_{j+1}: first interior of partition t+1, or z_{t+1}
-        Aff F{make_double2(0, 0), zero2(), eye2()};
-        if (tid + 1 < P && hasInt[tid + 1]) F = firstAff[tid + 1];
         RedEq r;
         r.A = mul(A, lastA.V);
         r.B = add(add(sym(q.b0, q.b1, q.b2), mul(A, lastA.W)), mul(C, F.V));
@@ -963,100 +1027,62 @@ __device__ void solve_interfaces(bool interior, const Aff &first, const Aff &las
 // into X: partitioned block Thomas + cyclic reduction of the interface
 // system.  Thread t owns knots [s, e); its interior rows s..e-2 are
 // eliminated in terms of the interfaces z_{t-1} = x_{s-1} and z_t = x_{e-1}.
+// Called by all threads of the workgroup.
+//
 // Partitions of at most M knots keep their rows and eliminated rows in
-// registers (one round of loads); longer ones (M = 0) go through IR in
-// memory.  Both do the same arithmetic in the same order.  Called by all
-// threads of the workgroup; IR and firstAff are workspace.
-template <int M>
-__device__ void exact_solve_t(const Eq0 *__restrict__ E, InteriorRow *__restrict__ IR, double2 *__restrict__ X,
-                              Aff *firstAff, int n, int tid) {
+// registers (one round of loads).
+template <int M, typename Rows>
+__device__ __forceinline__ void exact_solve_reg(const Rows &E, const Solution &X, SolveLds &S, int n, int tid) {
     const int m = (n + kSolveWG - 1) / kSolveWG;
     const int P = (n + m - 1) / m;
     const int s0 = tid * m, e0 = min(n, s0 + m);
     const int len = e0 - s0;
-    constexpr int MR = M > 0 ? M : 1;
-    Eq0 q[MR];
-    InteriorRow ir[MR];
+    Eq0 q[M];
+    InteriorRow ir[M];
     Eq0 qm{};  // row s0 - 1
     Aff lastA, first;
     Eq0 qj{};  // row e0 - 1
     M2 A = zero2();
     const bool interior = len >= 2;
     if (tid < P) {
-        if constexpr (M > 0) {
 #pragma unroll
-            for (int r = 0; r < M; r++)
-                if (r < len) q[r] = E[s0 + r];
-            if (s0 > 0) qm = E[s0 - 1];
-        }
+        for (int r = 0; r < M; r++)
+            if (r < len) q[r] = E.load(tid, r);
+        if (s0 > 0) qm = E.load(tid - 1, m - 1);
         if (interior) {
             // forward elimination
             M2 BiPrev = zero2();
             Aff Rprev;
-            if constexpr (M > 0) {
 #pragma unroll
-                for (int r = 0; r < M - 1; r++) {
-                    if (r > len - 2) continue;
-                    const Eq0 &qq = q[r];
-                    M2 Bh = sym(qq.b0, qq.b1, qq.b2);
-                    Aff R{make_double2(qq.d0, qq.d1), zero2(), zero2()};
-                    if (r == 0) {
-                        if (tid > 0) R.V = neg(sym(qm.c0, qm.c1, qm.c2));
-                    } else {
-                        const Eq0 &qp = q[r - 1];
-                        const M2 Ap = sym(qp.c0, qp.c1, qp.c2);  // A_i = O_{i-1}
-                        const M2 Lm = mul(Ap, BiPrev);
-                        Bh = sub(Bh, mul(Lm, Ap));
-                        R = aff_sub(R, aff_apply(Lm, Rprev));
-                    }
-                    if (r == len - 2) R.W = neg(sym(qq.c0, qq.c1, qq.c2));
-                    const M2 Bi = inv(Bh);
-                    ir[r] = InteriorRow{Bi, R};
-                    BiPrev = Bi;
-                    Rprev = R;
+            for (int r = 0; r < M - 1; r++) {
+                if (r > len - 2) continue;
+                const Eq0 &qq = q[r];
+                M2 Bh = sym(qq.b0, qq.b1, qq.b2);
+                Aff R{make_double2(qq.d0, qq.d1), zero2(), zero2()};
+                if (r == 0) {
+                    if (tid > 0) R.V = neg(sym(qm.c0, qm.c1, qm.c2));
+                } else {
+                    const Eq0 &qp = q[r - 1];
+                    const M2 Ap = sym(qp.c0, qp.c1, qp.c2);  // A_i = O_{i-1}
+                    const M2 Lm = mul(Ap, BiPrev);
+                    Bh = sub(Bh, mul(Lm, Ap));
+                    R = aff_sub(R, aff_apply(Lm, Rprev));
                 }
-            } else {
-                for (int i = s0; i <= e0 - 2; i++) {
-                    const Eq0 qq = E[i];
-                    M2 Bh = sym(qq.b0, qq.b1, qq.b2);
-                    Aff R{make_double2(qq.d0, qq.d1), zero2(), zero2()};
-                    if (i == s0) {
-                        if (tid > 0) {
-                            const Eq0 qp = E[i - 1];
-                            R.V = neg(sym(qp.c0, qp.c1, qp.c2));
-                        }
-                    } else {
-                        const Eq0 qp = E[i - 1];
-                        const M2 Ap = sym(qp.c0, qp.c1, qp.c2);  // A_i = O_{i-1}
-                        const M2 Lm = mul(Ap, BiPrev);
-                        Bh = sub(Bh, mul(Lm, Ap));
-                        R = aff_sub(R, aff_apply(Lm, Rprev));
-                    }
-                    if (i == e0 - 2) R.W = neg(sym(qq.c0, qq.c1, qq.c2));
-                    const M2 Bi = inv(Bh);
-                    IR[i] = InteriorRow{Bi, R};
-                    BiPrev = Bi;
-                    Rprev = R;
-                }
+                if (r == len - 2) R.W = neg(sym(qq.c0, qq.c1, qq.c2));
+                const M2 Bi = inv(Bh);
+                ir[r] = InteriorRow{Bi, R};
+                BiPrev = Bi;
+                Rprev = R;
             }
             // back substitution of the affine forms
             Aff Xa = aff_apply(BiPrev, Rprev);
             lastA = Xa;
-            if constexpr (M > 0) {
 #pragma unroll
-                for (int r = M - 3; r >= 0; r--) {
-                    if (r > len - 3) continue;
-                    const Eq0 &qq = q[r];
-                    const Aff t = aff_sub(ir[r].R, aff_apply(sym(qq.c0, qq.c1, qq.c2), Xa));
-                    Xa = aff_apply(ir[r].Bi, t);
-                }
-            } else {
-                for (int i = e0 - 3; i >= s0; i--) {
-                    const InteriorRow iri = IR[i];
-                    const Eq0 qq = E[i];
-                    const Aff t = aff_sub(iri.R, aff_apply(sym(qq.c0, qq.c1, qq.c2), Xa));
-                    Xa = aff_apply(iri.Bi, t);
-                }
+            for (int r = M - 3; r >= 0; r--) {
+                if (r > len - 3) continue;
+                const Eq0 &qq = q[r];
+                const Aff t = aff_sub(ir[r].R, aff_apply(sym(qq.c0, qq.c1, qq.c2), Xa));
+                Xa = aff_apply(ir[r].Bi, t);
             }
             first = Xa;
         } else {
@@ -1065,61 +1091,178 @@ __device__ void exact_solve_t(const Eq0 *__restrict__ E, InteriorRow *__restrict
         }
         // the interface row j = e0 - 1 and its coupling A = O_{j-1}
         const int j = e0 - 1;
-        if constexpr (M > 0) {
 #pragma unroll
-            for (int r = 0; r < M; r++)
-                if (r == len - 1) qj = q[r];
-            if (len >= 2) {
+        for (int r = 0; r < M; r++)
+            if (r == len - 1) qj = q[r];
+        if (len >= 2) {
 #pragma unroll
-                for (int r = 0; r < M - 1; r++)
-                    if (r == len - 2) A = sym(q[r].c0, q[r].c1, q[r].c2);
-            } else if (j > 0) {
-                A = sym(qm.c0, qm.c1, qm.c2);
-            }
-        } else {
-            qj = E[j];
-            if (j > 0) {
-                const Eq0 qp = E[j - 1];
-                A = sym(qp.c0, qp.c1, qp.c2);
-            }
+            for (int r = 0; r < M - 1; r++)
+                if (r == len - 2) A = sym(q[r].c0, q[r].c1, q[r].c2);
+        } else if (j > 0) {
+            A = sym(qm.c0, qm.c1, qm.c2);
         }
     }
     double2 zo, zp;
-    solve_interfaces(interior, first, lastA, qj, A, firstAff, P, tid, zo, zp);
+    solve_interfaces(interior, first, lastA, qj, A, S, P, tid, zo, zp);
     // interior reconstruction: x_i = Bi_i (R_i(z) - O_i x_{i+1})
     if (tid < P) {
-        X[e0 - 1] = zo;
+        X.set(e0 - 1, zo);
         double2 xn = zo;
-        if constexpr (M > 0) {
 #pragma unroll
-            for (int r = M - 2; r >= 0; r--) {
-                if (r > len - 2) continue;
-                const InteriorRow &iri = ir[r];
-                const double2 v = mulv(iri.R.V, zp), w = mulv(iri.R.W, zo);
-                double2 rr = make_double2(iri.R.y.x + v.x + w.x, iri.R.y.y + v.y + w.y);
-                if (r < len - 2) {
-                    const double2 t = mulv(sym(q[r].c0, q[r].c1, q[r].c2), xn);
-                    rr.x -= t.x;
-                    rr.y -= t.y;
-                }
-                xn = mulv(iri.Bi, rr);
-                X[s0 + r] = xn;
+        for (int r = M - 2; r >= 0; r--) {
+            if (r > len - 2) continue;
+            const InteriorRow &iri = ir[r];
+            const double2 v = mulv(iri.R.V, zp), w = mulv(iri.R.W, zo);
+            double2 rr = make_double2(iri.R.y.x + v.x + w.x, iri.R.y.y + v.y + w.y);
+            if (r < len - 2) {
+                const double2 t = mulv(sym(q[r].c0, q[r].c1, q[r].c2), xn);
+                rr.x -= t.x;
+                rr.y -= t.y;
             }
-        } else {
-            for (int i = e0 - 2; i >= s0; i--) {
-                const InteriorRow iri = IR[i];
-                const double2 v = mulv(iri.R.V, zp), w = mulv(iri.R.W, zo);
-                double2 rr = make_double2(iri.R.y.x + v.x + w.x, iri.R.y.y + v.y + w.y);
-                if (i < e0 - 2) {
-                    const Eq0 qq = E[i];
-                    const double2 t = mulv(sym(qq.c0, qq.c1, qq.c2), xn);
-                    rr.x -= t.x;
-                    rr.y -= t.y;
-                }
-                xn = mulv(iri.Bi, rr);
-                X[i] = xn;
-            }
+            xn = mulv(iri.Bi, rr);
+            X.set(s0 + r, xn);
         }
+    }
+    __threadfence_block();
+    __syncthreads();
+}
+
+// 2x2 products with the rounding fixed: the second product rounded, the first
+// fused to it, as the compiler contracts the plain forms above in straight
+// code (elsewhere it may pick the other one).
+__device__ __forceinline__ M2 mul_f(const M2 &x, const M2 &y) {
+    return M2{fma(x.a, y.a, x.b * y.c), fma(x.a, y.b, x.b * y.d), fma(x.c, y.a, x.d * y.c), fma(x.c, y.b, x.d * y.d)};
+}
+__device__ __forceinline__ double2 mulv_f(const M2 &m, double2 v) {
+    return make_double2(fma(m.a, v.x, m.b * v.y), fma(m.c, v.x, m.d * v.y));
+}
+__device__ __forceinline__ M2 inv_f(const M2 &m) {
+    const double id = 1.0 / fma(m.a, m.d, -(m.b * m.c));
+    return M2{m.d * id, -m.b * id, -m.c * id, m.a * id};
+}
+__device__ __forceinline__ Aff aff_apply_f(const M2 &m, const Aff &a) {
+    return Aff{mulv_f(m, a.y), mul_f(m, a.V), mul_f(m, a.W)};
+}
+
+// Longer partitions walk their rows, the next ones loaded while these are
+// eliminated, and keep the eliminated rows in IR (workspace, laid out like
+// MemRows).  The same arithmetic in the same order.
+template <typename Rows>
+__device__ __forceinline__ void exact_solve_mem(const Rows &E, SS_GLOBAL d2v *IR, const Solution &X, SolveLds &S, int n,
+                                                int tid) {
+#pragma clang fp contract(off)
+    const int m = (n + kSolveWG - 1) / kSolveWG;
+    const int P = (n + m - 1) / m;
+    const int s0 = tid * m, e0 = min(n, s0 + m);
+    const int len = e0 - s0;
+    constexpr int kAhead = 4;
+    Aff lastA, first;
+    Eq0 qj{};  // row e0 - 1
+    M2 A = zero2();
+    const bool interior = len >= 2;
+    constexpr int kPieces = 7;  // 16-byte pieces of an InteriorRow
+    auto irow = [&](int r) { return IR + (size_t)r * kPieces * kSolveWG + tid; };
+    struct Row {
+        Eq0 q;
+        InteriorRow ir;
+    };
+    auto load_row = [&](int r) {
+        const SS_GLOBAL d2v *p = irow(r);
+        d2v v[kPieces];
+#pragma unroll
+        for (int u = 0; u < kPieces; u++) v[u] = p[u * kSolveWG];
+        return Row{E.load(tid, r),
+                   InteriorRow{M2{v[0].x, v[0].y, v[1].x, v[1].y},
+                               Aff{make_double2(v[2].x, v[2].y), M2{v[3].x, v[3].y, v[4].x, v[4].y},
+                                   M2{v[5].x, v[5].y, v[6].x, v[6].y}}}};
+    };
+    // rows top .. 0 in turn, the next ones loaded ahead
+    auto rows_down = [&](int top, auto &&body) {
+        Row ahead[2];
+        ahead[0] = load_row(max(top, 0));
+        ahead[1] = load_row(max(top - 1, 0));
+        for (int r = top; r >= 0; r--) {
+            const Row w = ahead[0];
+            ahead[0] = ahead[1];
+            ahead[1] = load_row(max(r - 2, 0));
+            body(r, w);
+        }
+    };
+    if (tid < P) {
+        if (interior) {
+            // forward elimination
+            M2 BiPrev = zero2();
+            Aff Rprev;
+            Eq0 qp{}, ahead[kAhead];
+            if (tid > 0) qp = E.load(tid - 1, m - 1);
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) ahead[u] = E.load(tid, min(u, len - 1));
+            for (int r = 0; r <= len - 2; r++) {
+                const Eq0 qq = ahead[0];
+#pragma unroll
+                for (int u = 0; u + 1 < kAhead; u++) ahead[u] = ahead[u + 1];
+                ahead[kAhead - 1] = E.load(tid, min(r + kAhead, len - 1));
+                M2 Bh = sym(qq.b0, qq.b1, qq.b2);
+                Aff R{make_double2(qq.d0, qq.d1), zero2(), zero2()};
+                if (r == 0) {
+                    if (tid > 0) R.V = neg(sym(qp.c0, qp.c1, qp.c2));
+                } else {
+                    const M2 Ap = sym(qp.c0, qp.c1, qp.c2);  // A_i = O_{i-1}
+                    const M2 Lm = mul_f(Ap, BiPrev);
+                    Bh = sub(Bh, mul_f(Lm, Ap));
+                    R = aff_sub(R, aff_apply_f(Lm, Rprev));
+                }
+                if (r == len - 2) R.W = neg(sym(qq.c0, qq.c1, qq.c2));
+                const M2 Bi = inv_f(Bh);
+                SS_GLOBAL d2v *p = irow(r);
+                p[0] = d2v{Bi.a, Bi.b};
+                p[kSolveWG] = d2v{Bi.c, Bi.d};
+                p[2 * kSolveWG] = d2v{R.y.x, R.y.y};
+                p[3 * kSolveWG] = d2v{R.V.a, R.V.b};
+                p[4 * kSolveWG] = d2v{R.V.c, R.V.d};
+                p[5 * kSolveWG] = d2v{R.W.a, R.W.b};
+                p[6 * kSolveWG] = d2v{R.W.c, R.W.d};
+                BiPrev = Bi;
+                Rprev = R;
+                qp = qq;
+            }
+            // back substitution of the affine forms
+            Aff Xa = aff_apply_f(BiPrev, Rprev);
+            lastA = Xa;
+            rows_down(len - 3, [&](int, const Row &w) {
+                const Aff t = aff_sub(w.ir.R, aff_apply_f(sym(w.q.c0, w.q.c1, w.q.c2), Xa));
+                Xa = aff_apply_f(w.ir.Bi, t);
+            });
+            first = Xa;
+        } else {
+            lastA = Aff{make_double2(0, 0), eye2(), zero2()};      // x_{e-2} := z_prev
+            first = Aff{make_double2(0, 0), zero2(), eye2()};      // unused
+        }
+        // the interface row j = e0 - 1 and its coupling A = O_{j-1}
+        qj = E.load(tid, len - 1);
+        if (e0 - 1 > 0) {
+            const Eq0 qp = len >= 2 ? E.load(tid, len - 2) : E.load(tid - 1, m - 1);
+            A = sym(qp.c0, qp.c1, qp.c2);
+        }
+    }
+    double2 zo, zp;
+    solve_interfaces(interior, first, lastA, qj, A, S, P, tid, zo, zp);
+    // interior reconstruction: x_i = Bi_i (R_i(z) - O_i x_{i+1})
+    if (tid < P) {
+        X.set(e0 - 1, zo);
+        double2 xn = zo;
+        if (interior)
+            rows_down(len - 2, [&](int r, const Row &w) {
+                const double2 v = mulv_f(w.ir.R.V, zp), z = mulv_f(w.ir.R.W, zo);
+                double2 rr = make_double2(w.ir.R.y.x + v.x + z.x, w.ir.R.y.y + v.y + z.y);
+                if (r < len - 2) {
+                    const double2 t = mulv_f(sym(w.q.c0, w.q.c1, w.q.c2), xn);
+                    rr.x -= t.x;
+                    rr.y -= t.y;
+                }
+                xn = mulv_f(w.ir.Bi, rr);
+                X.set(s0 + r, xn);
+            });
     }
     __threadfence_block();
     __syncthreads();
@@ -1127,17 +1270,80 @@ __device__ void exact_solve_t(const Eq0 *__restrict__ E, InteriorRow *__restrict
 
 // knots per partition that stay in registers
 constexpr int kSolveRegRows = 8;
-// knots whose level-0 equations the solve keeps in LDS (112 KiB; with the
-// kernel's other arrays within the 160 KiB of a workgroup)
-constexpr int kSolveLdsRows = 1792;
+// Knots whose level-0 equations the solve keeps in LDS (114 KiB).  Groups of
+// more knots keep their solution there instead (four times as many), and the
+// knots' usage beside it.  The rest of the 160 KiB holds the interface system.
+// One workgroup walks a group's rows, 16 per thread at 4096 knots, so latency
+// bounds the launch: with equations and eliminated rows one after the other
+// per thread in memory, a launch over groups of up to 4096 knots (10 groups,
+// FP32 with refinement) took 199 us; in pieces that a wave loads side by side,
+// the next rows ahead, and the solution in LDS, 122 us; 4096 knots without
+// neighbours 131 -> 82 us; with the equations in LDS (1600 knots, FP64)
+// 45 -> 40 us.
+constexpr int kSolveLdsRows = 1824, kSolveLdsKnots = 4 * kSolveLdsRows;
 
 // Inlined into the solve kernel: as a called function it would save and
 // restore the callee-saved registers it uses (over 200 per call).
-__device__ __forceinline__ void exact_solve(const Eq0 *E, InteriorRow *IR, double2 *X, Aff *firstAff, int n, int tid) {
+template <typename Rows>
+__device__ __forceinline__ void exact_solve(const Rows &E, SS_GLOBAL d2v *IR, const Solution &X, SolveLds &S, int n,
+                                            int tid) {
     if ((n + kSolveWG - 1) / kSolveWG <= kSolveRegRows)
-        exact_solve_t<kSolveRegRows>(E, IR, X, firstAff, n, tid);
+        exact_solve_reg<kSolveRegRows>(E, X, S, n, tid);
     else
-        exact_solve_t<0>(E, IR, X, firstAff, n, tid);
+        exact_solve_mem(E, IR, X, S, n, tid);
+}
+
+// The exact solve with, in mixed precision, one step of iterative refinement
+// in FP64: r = g - H x, H e = r, x += e (the matrix entries stay; each knot's
+// right-hand side is replaced by its residual; Xs keeps x).
+template <typename Rows>
+__device__ __forceinline__ void solve_refined(const Rows &E, SS_GLOBAL d2v *IR, const Solution &X, SS_GLOBAL d2v *Xs,
+                                              SolveLds &S, int n, int refine, int tid) {
+#pragma clang fp contract(off)
+    exact_solve(E, IR, X, S, n, tid);
+    if (!refine) return;
+    // each thread its partition's rows, loaded four at a time
+    const int m = (n + kSolveWG - 1) / kSolveWG;
+    const int s0 = tid * m, len = min(n, s0 + m) - s0;
+    Eq0 qp{};  // the row before
+    if (len > 0 && s0 > 0) qp = E.load(tid - 1, m - 1);
+    for (int r0 = 0; r0 < len; r0 += 4) {
+        Eq0 q4[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) q4[u] = E.load(tid, min(r0 + u, len - 1));
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int k = s0 + r0 + u;
+            if (r0 + u >= len) break;
+            const Eq0 q = q4[u];
+            const double2 x = X.get(k);
+            double r0_ = q.d0 - fma(q.b0, x.x, q.b1 * x.y);
+            double r1_ = q.d1 - fma(q.b1, x.x, q.b2 * x.y);
+            if (k > 0) {
+                const double2 xp = X.get(k - 1);
+                r0_ -= fma(qp.c0, xp.x, qp.c1 * xp.y);
+                r1_ -= fma(qp.c1, xp.x, qp.c2 * xp.y);
+            }
+            if (k + 1 < n) {
+                const double2 xn = X.get(k + 1);
+                r0_ -= fma(q.c0, xn.x, q.c1 * xn.y);
+                r1_ -= fma(q.c1, xn.x, q.c2 * xn.y);
+            }
+            Xs[k] = d2v{x.x, x.y};
+            E.put_rhs(k, r0_, r1_);
+            qp = q;
+        }
+    }
+    __threadfence_block();
+    __syncthreads();
+    exact_solve(E, IR, X, S, n, tid);
+    for (int k = tid; k < n; k += kSolveWG) {
+        const double2 e = X.get(k);
+        const d2v x = Xs[k];
+        X.set(k, make_double2(x.x + e.x, x.y + e.y));
+    }
+    __threadfence_block();
+    __syncthreads();
 }
 
 // Output 10: the device time since the group's last stage end goes to slot
@@ -1178,7 +1384,6 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
     }
     const double *S = g.colsum;
     const int *minPts = g.minPts;
-    uint8_t *used = g.used;
     // The loops below load a batch of entries before they use any of it:
     // one thread per frame or knot would otherwise wait out a memory latency
     // per entry.  The additions keep their order.
@@ -1209,80 +1414,77 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
     }
     // 2. knot usage (d_createParameterMask) and level-0 equations
     //    (d_fillDiagonals / d_fillJTr entries, lambda extension); the knots
-    //    from n on are never used.  The equations stay in LDS when they fit.
-    __shared__ Eq0 sE[kSolveLdsRows];
-    Eq0 *E = n <= kSolveLdsRows ? sE : reinterpret_cast<Eq0 *>(g.ws);
-    level0_equations(S, minPts, used, E, n, nb, g.lambda, g.fracUniform, tid);
-    for (int k = n + tid; k < N; k += kSolveWG) used[k] = 0;
-    __threadfence_block();
-    __syncthreads();
-    InteriorRow *IR = reinterpret_cast<InteriorRow *>(g.ws + (size_t)n * 8);
-    double2 *X = reinterpret_cast<double2 *>(IR + n);
-    Aff *firstAff = reinterpret_cast<Aff *>(X + n);
-    // The exact solve without refinement, its partitions in registers, has
-    // read every equation before its first barrier and writes the solution
-    // after the last: the solution then takes the equations' LDS.
-    if (E == sE && g.solverId != 0 && !g.refine && (n + kSolveWG - 1) / kSolveWG <= kSolveRegRows)
-        X = reinterpret_cast<double2 *>(sE);
+    //    from n on are never used.
+    __shared__ __align__(16) Eq0 sE[kSolveLdsRows];
+    __shared__ uint8_t sUsed[kSolveLdsKnots];
+    __shared__ SolveLds sS;
+    const int m = (n + kSolveWG - 1) / kSolveWG;
+    const bool rowsInLds = n <= kSolveLdsRows, usedInLds = n <= kSolveLdsKnots;
+    SS_GLOBAL uint8_t *gUsed = (SS_GLOBAL uint8_t *)g.used;
+    auto set_used = [&](int k, bool u) {
+        if (usedInLds) sUsed[k] = u;
+        else gUsed[k] = u;
+    };
+    auto used = [&](int k) {
+        uint8_t u;
+        if (usedInLds) u = sUsed[k];
+        else u = gUsed[k];
+        return u != 0;
+    };
+    // workspace: [equations][eliminated rows][solution][saved solution]
+    const size_t rows = (size_t)n + kSolveWG;
+    double *ws = g.ws;
+    SS_GLOBAL d2v *IR = (SS_GLOBAL d2v *)(ws + rows * 8);
+    double2 *Xmem = reinterpret_cast<double2 *>(ws + rows * (8 + sizeof(InteriorRow) / sizeof(double)));
+    SS_GLOBAL d2v *Xs = (SS_GLOBAL d2v *)(Xmem + rows);
+    // The solution takes the equations' LDS where they are in memory, and
+    // where the exact solve without refinement, its partitions in registers,
+    // has read every equation before its first barrier and writes the
+    // solution after the last.
+    const bool xInLds = rowsInLds ? g.solverId != 0 && !g.refine && m <= kSolveRegRows
+                                  : g.solverId != 0 && n <= kSolveLdsKnots;
+    const Solution X{reinterpret_cast<double2 *>(sE), (SS_GLOBAL d2v *)Xmem, xInLds};
+    auto equations = [&](auto &&put) {
+        level0_equations(S, minPts, n, nb, g.lambda, g.fracUniform, tid, [&](int k, const Eq0 &e, bool u) {
+            put(k, e);
+            set_used(k, u);
+        });
+        __threadfence_block();
+        __syncthreads();
+    };
     if (g.solverId == 0) {
         // 4a. solver id 0: ILU(0) in x-then-y order (one thread, the
         //     reference's recurrence order)
-        if (tid == 0) ilu0_solve(E, reinterpret_cast<IluRow *>(IR), X, n);
+        Eq0 *E = rowsInLds ? sE : reinterpret_cast<Eq0 *>(ws);
+        equations([&](int k, const Eq0 &e) { E[k] = e; });
+        if (tid == 0) ilu0_solve(E, (IluRow *)(ws + rows * 8), Xmem, n);
         __threadfence_block();
         __syncthreads();
+    } else if (rowsInLds) {
+        const LdsRows E{sE, m};
+        equations([&](int k, const Eq0 &e) { E.put(k, e); });
+        solve_refined(E, IR, X, Xs, sS, n, g.refine, tid);
     } else {
-        exact_solve(E, IR, X, firstAff, n, tid);
-        if (g.refine) {
-            // one step of iterative refinement in FP64: r = g - H x, H e = r,
-            // x += e (the matrix entries stay; each knot's right-hand side is
-            // replaced by its residual)
-            double2 *Xs = reinterpret_cast<double2 *>(firstAff + kSolveWG);
-            for (int k = tid; k < n; k += kSolveWG) {
-                const Eq0 q = E[k];
-                const double2 x = X[k];
-                double r0 = q.d0 - (q.b0 * x.x + q.b1 * x.y);
-                double r1 = q.d1 - (q.b1 * x.x + q.b2 * x.y);
-                if (k > 0) {
-                    const Eq0 qp = E[k - 1];
-                    const double2 xp = X[k - 1];
-                    r0 -= qp.c0 * xp.x + qp.c1 * xp.y;
-                    r1 -= qp.c1 * xp.x + qp.c2 * xp.y;
-                }
-                if (k + 1 < n) {
-                    const double2 xn = X[k + 1];
-                    r0 -= q.c0 * xn.x + q.c1 * xn.y;
-                    r1 -= q.c1 * xn.x + q.c2 * xn.y;
-                }
-                Xs[k] = x;
-                E[k].d0 = r0;
-                E[k].d1 = r1;
-            }
-            __threadfence_block();
-            __syncthreads();
-            exact_solve(E, IR, X, firstAff, n, tid);
-            for (int k = tid; k < n; k += kSolveWG) {
-                const double2 e = X[k], x = Xs[k];
-                X[k] = make_double2(x.x + e.x, x.y + e.y);
-            }
-            __threadfence_block();
-            __syncthreads();
-        }
+        const MemRows E{(SS_GLOBAL d2v *)ws, m};
+        equations([&](int k, const Eq0 &e) { E.put(k, e); });
+        solve_refined(E, IR, X, Xs, sS, n, g.refine, tid);
     }
     // 5. step filter over the used knots, x sequence then y sequence
     //    (SmearingFilter::apply / RangeFilter::apply on the compacted halves)
     const int filterKind = s_filter;
     const double strength = g.strength;
     if (filterKind == 1) {
-        __shared__ double sa[kSolveWG][4];
+        double (*sa)[4] = sS.scan;
         const int chunk = (n + kSolveWG - 1) / kSolveWG;
         const int c0 = min(n, tid * chunk), c1 = min(n, c0 + chunk);
         double ax = 1, bx = 0, ay = 1, by = 0;
         for (int k = c0; k < c1; k++) {
-            if (!g.used[k]) continue;
+            if (!used(k)) continue;
             ax *= strength;
-            bx = strength * bx + (1 - strength) * X[k].x;
+            const double2 x = X.get(k);
+            bx = strength * bx + (1 - strength) * x.x;
             ay *= strength;
-            by = strength * by + (1 - strength) * X[k].y;
+            by = strength * by + (1 - strength) * x.y;
         }
         sa[tid][0] = ax;
         sa[tid][1] = bx;
@@ -1311,10 +1513,11 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
         double yx = tid > 0 ? sa[tid - 1][1] : 0.0;
         double yy = tid > 0 ? sa[tid - 1][3] : 0.0;
         for (int k = c0; k < c1; k++) {
-            if (!g.used[k]) continue;
-            yx = yx * strength + X[k].x * (1 - strength);
-            yy = yy * strength + X[k].y * (1 - strength);
-            X[k] = make_double2(yx, yy);
+            if (!used(k)) continue;
+            const double2 x = X.get(k);
+            yx = yx * strength + x.x * (1 - strength);
+            yy = yy * strength + x.y * (1 - strength);
+            X.set(k, make_double2(yx, yy));
         }
         __threadfence_block();
         __syncthreads();
@@ -1323,19 +1526,22 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
             for (int axis = 0; axis < 2; axis++) {
                 int pv = -1, cu = -1;
                 for (int k = 0; k < n; k++) {
-                    if (!g.used[k]) continue;
+                    if (!used(k)) continue;
                     if (pv >= 0 && cu >= 0) {
-                        const double vm = axis ? X[pv].y : X[pv].x;
-                        const double vi = axis ? X[cu].y : X[cu].x;
-                        const double vp = axis ? X[k].y : X[k].x;
+                        const double2 xm = X.get(pv), xp = X.get(k);
+                        double2 xc = X.get(cu);
+                        const double vm = axis ? xm.y : xm.x;
+                        const double vi = axis ? xc.y : xc.x;
+                        const double vp = axis ? xp.y : xp.x;
                         const double tc = (vm + vp) / 2;
                         const double diff = (tc - vm) * strength;
                         bool rep;
                         if (vm < vp) rep = vi > vp + diff || vi < vm - diff;
                         else rep = vi < vp + diff || vi > vm - diff;
                         if (rep) {
-                            if (axis) X[cu].y = tc;
-                            else X[cu].x = tc;
+                            if (axis) xc.y = tc;
+                            else xc.x = tc;
+                            X.set(cu, xc);
                         }
                     }
                     pv = cu;
@@ -1360,8 +1566,10 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
             const bool fixed = ((((idx + 1) - (shift * (G >> 1))) % G) == 0);
             dv[u] = deltaP[idx];
             pv[u] = p[idx];
-            const bool uj = j < n && used[j];
-            xv[u] = uj ? (idx >= N ? X[j].y : X[j].x) : 0.0;
+            const int jj = min(j, n - 1);
+            const bool uj = j < n && used(jj);
+            const double2 x = X.get(jj);
+            xv[u] = uj ? (idx >= N ? x.y : x.x) : 0.0;
             keep[u] = fixed;
         }
 #pragma unroll
@@ -2155,9 +2363,9 @@ hipError_t launch_stage(const LaunchBatch &L, int entry, hipStream_t s) {
 }
 
 size_t solve_workspace_bytes(int n) {
-    // Eq0 + InteriorRow + solution per knot, first-interior forms per
-    // partition, the refinement's saved solution per knot
-    return (size_t)n * (sizeof(Eq0) + sizeof(InteriorRow) + 2 * sizeof(double2)) + kSolveWG * sizeof(Aff) + 256;
+    // Eq0 + InteriorRow + solution + the refinement's saved solution per knot
+    // and, the last partition's unused rows, per thread
+    return ((size_t)n + kSolveWG) * (sizeof(Eq0) + sizeof(InteriorRow) + 2 * sizeof(double2)) + 256;
 }
 
 }  // namespace ss
