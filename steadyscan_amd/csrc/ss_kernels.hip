@@ -689,8 +689,8 @@ __device__ __forceinline__ Aff aff_sub(const Aff &a, const Aff &b) {
     return Aff{make_double2(a.y.x - b.y.x, a.y.y - b.y.y), sub(a.V, b.V), sub(a.W, b.W)};
 }
 
-struct RedEq {  // reduced (interface) equation, general 2x2 blocks
-    M2 A, B, C;
+struct RedEq {  // reduced (interface) equation, general 2x2 blocks, B inverted
+    M2 A, Bi, C;
     double2 d, x;
     double pad;  // neighbouring equations start in different LDS banks
 };
@@ -817,61 +817,53 @@ __device__ void ilu0_solve(const Eq0 *E, IluRow *F, double2 *X, int n) {
     }
 }
 
-// Knot usage (d_createParameterMask): knot k < n is used when block column
-// k or k - 1 reaches its block's minimum point count; knots from n on never
-// are.
-__device__ __forceinline__ bool knot_used(const double *__restrict__ S, const int *__restrict__ minPts, int k,
-                                          int n, int nb) {
-    if (k < 0 || k >= n) return false;
-    const bool pc = S[(size_t)k * CS_N + CS_CNT] >= (double)minPts[k % nb];
-    const bool pp = k > 0 && S[(size_t)(k - 1) * CS_N + CS_CNT] >= (double)minPts[(k - 1) % nb];
-    return pc || pp;
-}
-
 // Level-0 equations of knots tid, tid + kSolveWG, ... (d_fillDiagonals /
-// d_fillJTr entries, lambda extension) into put(k, equation, used).  Each
-// knot takes its own and its neighbours' usage from the column counts, so
-// that no pass over the flags has to come first.  The pointers do not alias,
-// so the next knot's loads may be issued before this knot's equation is
-// stored.
+// d_fillJTr entries, lambda extension) into put(k, equation, used).  Knot
+// usage (d_createParameterMask): knot k < n is used when block column k or
+// k - 1 reaches its block's minimum point count; knots from n on never are.
+// Each knot takes its own and its neighbours' usage from the column counts,
+// so that no pass over the flags has to come first, and every load is issued
+// before any is used, at clamped indices instead of under a condition: one
+// memory latency per knot, and the pointers do not alias, so that the next
+// knots' loads overlap it.
 template <typename Put>
-__device__ __forceinline__ void level0_equations(const double *__restrict__ S, const int *__restrict__ minPts, int n,
-                                                 int nb, double lambda, int fracUniform, int tid, Put &&put) {
+__device__ __forceinline__ void level0_equations(const SS_GLOBAL double *__restrict__ S,
+                                                 const SS_GLOBAL int *__restrict__ minPts, int n, int nb,
+                                                 double lambda, int fracUniform, int tid, Put &&put) {
+    const int q = fracUniform ? CS_BXX : CS_QXX;
 #pragma unroll 4
     for (int k = tid; k < n; k += kSolveWG) {
-        Eq0 e;
-        const double *s = S + (size_t)k * CS_N;
-        const bool u = knot_used(S, minPts, k, n, nb);
-        const bool up = k > 0 && knot_used(S, minPts, k - 1, n, nb);
-        const bool un = (k + 1 < n) && knot_used(S, minPts, k + 1, n, nb);
-        if (!u) {
-            e = Eq0{1, 0, 1, 0, 0, 0, 0, 0};
-        } else {
-            double dxx = s[CS_AXX], dyy = s[CS_AYY], dxy = s[CS_AXY];
-            double jx = s[CS_JXA], jy = s[CS_JYA];
-            if (k > 0) {
-                const double *sp = s - CS_N;
-                const int q = fracUniform ? CS_BXX : CS_QXX;
-                dxx += sp[q];
-                dyy += sp[q + 1];
-                dxy += sp[q + 2];
-                jx += sp[CS_JXB];
-                jy += sp[CS_JYB];
-            }
-            const double nl = (double)(up ? 1 : 0) + (double)(un ? 1 : 0);
-            e.b0 = dxx + lambda * nl;
-            e.b1 = dxy;
-            e.b2 = dyy + lambda * nl;
-            if (un) {
-                e.c0 = s[CS_CXX] - lambda;
-                e.c1 = s[CS_CXY];
-                e.c2 = s[CS_CYY] - lambda;
-            } else {
-                e.c0 = e.c1 = e.c2 = 0;
-            }
-            e.d0 = jx;
-            e.d1 = jy;
+        const SS_GLOBAL double *s = S + (size_t)k * CS_N;
+        const SS_GLOBAL double *sp = k > 0 ? s - CS_N : s, *sn = k + 1 < n ? s + CS_N : s;
+        const SS_GLOBAL double *spp = k > 1 ? sp - CS_N : sp;
+        // block column of k - 2 .. k + 1
+        const int b = k % nb, bp = b > 0 ? b - 1 : nb - 1, bpp = bp > 0 ? bp - 1 : nb - 1, bn = b + 1 < nb ? b + 1 : 0;
+        double dxx = s[CS_AXX], dyy = s[CS_AYY], dxy = s[CS_AXY];
+        double jx = s[CS_JXA], jy = s[CS_JYA];
+        const double cxx = s[CS_CXX], cxy = s[CS_CXY], cyy = s[CS_CYY];
+        const double pxx = sp[q], pyy = sp[q + 1], pxy = sp[q + 2], pjx = sp[CS_JXB], pjy = sp[CS_JYB];
+        const double cnt = s[CS_CNT], cntP = sp[CS_CNT], cntPP = spp[CS_CNT], cntN = sn[CS_CNT];
+        const int mp = minPts[b], mpP = minPts[bp], mpPP = minPts[bpp], mpN = minPts[bn];
+        const bool c = cnt >= (double)mp, cP = k > 0 && cntP >= (double)mpP;
+        const bool cPP = k > 1 && cntPP >= (double)mpPP, cN = k + 1 < n && cntN >= (double)mpN;
+        const bool u = c || cP, up = k > 0 && (cP || cPP), un = k + 1 < n && (cN || c);
+        if (k > 0) {
+            dxx += pxx;
+            dyy += pyy;
+            dxy += pxy;
+            jx += pjx;
+            jy += pjy;
         }
+        const double nl = (double)(up ? 1 : 0) + (double)(un ? 1 : 0);
+        Eq0 e;
+        e.b0 = u ? dxx + lambda * nl : 1.0;
+        e.b1 = u ? dxy : 0.0;
+        e.b2 = u ? dyy + lambda * nl : 1.0;
+        e.c0 = u && un ? cxx - lambda : 0.0;
+        e.c1 = u && un ? cxy : 0.0;
+        e.c2 = u && un ? cyy - lambda : 0.0;
+        e.d0 = u ? jx : 0.0;
+        e.d1 = u ? jy : 0.0;
         put(k, e, u);
     }
 }
@@ -928,6 +920,34 @@ struct Solution {
     }
 };
 
+// 2x2 products with the rounding fixed: the second product rounded, the first
+// fused to it, as the compiler contracts the plain forms above in straight
+// code (elsewhere it may pick the other one).
+__device__ __forceinline__ M2 mul_f(const M2 &x, const M2 &y) {
+    return M2{fma(x.a, y.a, x.b * y.c), fma(x.a, y.b, x.b * y.d), fma(x.c, y.a, x.d * y.c), fma(x.c, y.b, x.d * y.d)};
+}
+__device__ __forceinline__ double2 mulv_f(const M2 &m, double2 v) {
+    return make_double2(fma(m.a, v.x, m.b * v.y), fma(m.c, v.x, m.d * v.y));
+}
+// ... the first product rounded, the second fused to it
+__device__ __forceinline__ M2 mul_s(const M2 &x, const M2 &y) {
+    return M2{fma(x.b, y.c, x.a * y.a), fma(x.b, y.d, x.a * y.b), fma(x.d, y.c, x.c * y.a), fma(x.d, y.d, x.c * y.b)};
+}
+__device__ __forceinline__ double2 mulv_s(const M2 &m, double2 v) {
+    return make_double2(fma(m.b, v.y, m.a * v.x), fma(m.d, v.y, m.c * v.x));
+}
+// ... of an inverse: the off-diagonal product rounded
+__device__ __forceinline__ double2 mulv_i(const M2 &m, double2 v) {
+    return make_double2(fma(m.a, v.x, m.b * v.y), fma(m.d, v.y, m.c * v.x));
+}
+__device__ __forceinline__ M2 inv_f(const M2 &m) {
+    const double id = 1.0 / fma(m.a, m.d, -(m.b * m.c));
+    return M2{m.d * id, -m.b * id, -m.c * id, m.a * id};
+}
+__device__ __forceinline__ Aff aff_apply_f(const M2 &m, const Aff &a) {
+    return Aff{mulv_f(m, a.y), mul_f(m, a.V), mul_f(m, a.W)};
+}
+
 // Interface system of the partitioned solve: thread t < P contributes the
 // equation of its partition's last knot z_t in terms of z_{t-1} and z_{t+1}
 // (its last interior row as lastA, the next partition's first interior row
@@ -935,6 +955,7 @@ struct Solution {
 // returns z_t and z_{t-1} (0 for t = 0).
 __device__ __forceinline__ void solve_interfaces(bool interior, const Aff &first, const Aff &lastA, const Eq0 &q,
                                                  const M2 &A, SolveLds &S, int P, int tid, double2 &zo, double2 &zp) {
+#pragma clang fp contract(off)
     RedEq *red = S.red;
     if (tid < P) {
         S.hasInt[tid] = interior ? 1 : 0;
@@ -945,82 +966,78 @@ __device__ __forceinline__ void solve_interfaces(bool interior, const Aff &first
     Aff F{make_double2(0, 0), zero2(), eye2()};
     if (tid + 1 < P && S.hasInt[tid + 1]) F = S.first[tid + 1];
     __syncthreads();  // the interface system takes the affine forms' memory
+    // Cyclic reduction, in place: level l's equation k is that of thread
+    // k * 2^l + 2^l - 1.  A thread keeps its own equation in registers and
+    // leaves the others what they read of it: the inverse of B, which its
+    // back substitution takes too, A, C and d.
+    M2 B = zero2(), Bi = zero2(), Ai = zero2(), C = zero2();
+    double2 d = make_double2(0, 0);
+    auto publish = [&]() {
+        Bi = inv_f(B);
+        red[tid].A = Ai;
+        red[tid].Bi = Bi;
+        red[tid].C = C;
+        red[tid].d = d;
+    };
     if (tid < P) {
-        const M2 C = sym(q.c0, q.c1, q.c2);
-        RedEq r;
-        r.A = mul(A, lastA.V);
-        r.B = add(add(sym(q.b0, q.b1, q.b2), mul(A, lastA.W)), mul(C, F.V));
-        r.C = mul(C, F.W);
-        const double2 ay = mulv(A, lastA.y), cy = mulv(C, F.y);
-        r.d = make_double2(q.d0 - ay.x - cy.x, q.d1 - ay.y - cy.y);
-        r.x = make_double2(0, 0);
-        if (tid == 0) r.A = zero2();
-        red[tid] = r;
+        const M2 Cn = sym(q.c0, q.c1, q.c2);
+        Ai = mul_f(A, lastA.V);
+        B = add(add(sym(q.b0, q.b1, q.b2), mul_f(A, lastA.W)), mul_f(Cn, F.V));
+        C = mul_f(Cn, F.W);
+        const double2 ay = mulv_f(A, lastA.y), cy = mulv_f(Cn, F.y);
+        d = make_double2(q.d0 - ay.x - cy.x, q.d1 - ay.y - cy.y);
+        if (tid == 0) Ai = zero2();
+        publish();
     }
     __syncthreads();
-    // cyclic reduction, in place: level-l equation k lives at k*2^l + 2^l - 1
     int nlev = 0;
     for (int mm = P; mm > 1; mm >>= 1) nlev++;
     for (int l = 0; l < nlev; l++) {
-        const int st = 1 << l, mm = P >> l;
-        for (int jj = tid; jj < (mm >> 1); jj += kSolveWG) {
-            const int i = (2 * jj + 1) * st + st - 1;
-            const int im = i - st, ip = i + st;
-            RedEq e = red[i];
-            const RedEq em = red[im];
-            const M2 al = neg(mul(e.A, inv(em.B)));
-            RedEq o;
-            o.A = mul(al, em.A);
-            o.B = add(e.B, mul(al, em.C));
-            double2 t = mulv(al, em.d);
-            o.d = make_double2(e.d.x + t.x, e.d.y + t.y);
-            if (2 * jj + 2 < mm) {
-                const RedEq ep = red[ip];
-                const M2 ga = neg(mul(e.C, inv(ep.B)));
-                o.B = add(o.B, mul(ga, ep.A));
-                o.C = mul(ga, ep.C);
-                t = mulv(ga, ep.d);
-                o.d = make_double2(o.d.x + t.x, o.d.y + t.y);
+        const int st = 1 << l;
+        if (tid < P && ((tid + 1) & (2 * st - 1)) == 0) {
+            const RedEq em = red[tid - st];
+            const M2 al = neg(mul_f(Ai, em.Bi));
+            Ai = mul_s(al, em.A);
+            B = add(B, mul_s(al, em.C));
+            double2 t = mulv_s(al, em.d);
+            double2 o = make_double2(d.x + t.x, d.y + t.y);
+            if (tid + st < P) {
+                const RedEq ep = red[tid + st];
+                const M2 ga = neg(mul_f(C, ep.Bi));
+                B = add(B, mul_s(ga, ep.A));
+                C = mul_s(ga, ep.C);
+                t = mulv_s(ga, ep.d);
+                o = make_double2(o.x + t.x, o.y + t.y);
             } else {
-                o.C = zero2();
+                C = zero2();
             }
-            o.x = make_double2(0, 0);
-            red[i] = o;
-        }
-        __syncthreads();
-    }
-    if (tid == 0 && P > 0) {
-        const int i = (1 << nlev) - 1;
-        red[i].x = mulv(inv(red[i].B), red[i].d);
-    }
-    __syncthreads();
-    for (int l = nlev - 1; l >= 0; l--) {
-        const int st = 1 << l, mm = P >> l;
-        for (int kk = tid; kk < (mm + 1) / 2; kk += kSolveWG) {
-            const int k = 2 * kk;  // even equations of level l
-            const int i = k * st + st - 1;
-            const RedEq e = red[i];
-            double2 r = e.d;
-            if (k > 0) {
-                const double2 t = mulv(e.A, red[i - st].x);
-                r.x -= t.x;
-                r.y -= t.y;
-            }
-            if (k + 1 < mm) {
-                const double2 t = mulv(e.C, red[i + st].x);
-                r.x -= t.x;
-                r.y -= t.y;
-            }
-            red[i].x = mulv(inv(e.B), r);
+            d = o;
+            publish();
         }
         __syncthreads();
     }
     zo = make_double2(0, 0);
     zp = make_double2(0, 0);
-    if (tid < P) {
-        zo = red[tid].x;
-        if (tid > 0) zp = red[tid - 1].x;
+    for (int l = nlev; l >= 0; l--) {
+        const int st = 1 << l;
+        if (tid < P && ((tid + 1) & (2 * st - 1)) == st) {  // eliminated at level l
+            double2 r = d;
+            if (tid >= st) {
+                const double2 t = mulv_f(Ai, red[tid - st].x);
+                r.x -= t.x;
+                r.y -= t.y;
+            }
+            if (tid + st < P) {
+                const double2 t = mulv_f(C, red[tid + st].x);
+                r.x -= t.x;
+                r.y -= t.y;
+            }
+            zo = mulv_i(Bi, r);
+            red[tid].x = zo;
+        }
+        __syncthreads();
     }
+    if (tid < P && tid > 0) zp = red[tid - 1].x;
 }
 
 // Exact FP64 solve of the level-0 block-tridiagonal system E (knots 0..n-1)
@@ -1112,36 +1129,19 @@ __device__ __forceinline__ void exact_solve_reg(const Rows &E, const Solution &X
         for (int r = M - 2; r >= 0; r--) {
             if (r > len - 2) continue;
             const InteriorRow &iri = ir[r];
-            const double2 v = mulv(iri.R.V, zp), w = mulv(iri.R.W, zo);
+            const double2 v = mulv_s(iri.R.V, zp), w = mulv_f(iri.R.W, zo);
             double2 rr = make_double2(iri.R.y.x + v.x + w.x, iri.R.y.y + v.y + w.y);
             if (r < len - 2) {
-                const double2 t = mulv(sym(q[r].c0, q[r].c1, q[r].c2), xn);
+                const double2 t = mulv_f(sym(q[r].c0, q[r].c1, q[r].c2), xn);
                 rr.x -= t.x;
                 rr.y -= t.y;
             }
-            xn = mulv(iri.Bi, rr);
+            xn = mulv_f(iri.Bi, rr);
             X.set(s0 + r, xn);
         }
     }
     __threadfence_block();
     __syncthreads();
-}
-
-// 2x2 products with the rounding fixed: the second product rounded, the first
-// fused to it, as the compiler contracts the plain forms above in straight
-// code (elsewhere it may pick the other one).
-__device__ __forceinline__ M2 mul_f(const M2 &x, const M2 &y) {
-    return M2{fma(x.a, y.a, x.b * y.c), fma(x.a, y.b, x.b * y.d), fma(x.c, y.a, x.d * y.c), fma(x.c, y.b, x.d * y.d)};
-}
-__device__ __forceinline__ double2 mulv_f(const M2 &m, double2 v) {
-    return make_double2(fma(m.a, v.x, m.b * v.y), fma(m.c, v.x, m.d * v.y));
-}
-__device__ __forceinline__ M2 inv_f(const M2 &m) {
-    const double id = 1.0 / fma(m.a, m.d, -(m.b * m.c));
-    return M2{m.d * id, -m.b * id, -m.c * id, m.a * id};
-}
-__device__ __forceinline__ Aff aff_apply_f(const M2 &m, const Aff &a) {
-    return Aff{mulv_f(m, a.y), mul_f(m, a.V), mul_f(m, a.W)};
 }
 
 // Longer partitions walk their rows, the next ones loaded while these are
@@ -1348,14 +1348,15 @@ __device__ __forceinline__ void solve_refined(const Rows &E, SS_GLOBAL d2v *IR, 
 
 // Output 10: the device time since the group's last stage end goes to slot
 // `slot`.  Called by one thread of a per-group kernel.
-__device__ __forceinline__ void stage_time(const GroupDev &g, GroupCtl &ctl, int slot) {
+template <typename G>
+__device__ __forceinline__ void stage_time(G &g, GroupCtl &ctl, int slot) {
     if (!g.funcTimes) return;
     const unsigned long long now = wall_clock64();
     if (ctl.tStage) g.funcTimes[slot] += (double)(now - ctl.tStage) / g.clockHz;
     ctl.tStage = now;
 }
 
-__device__ void final_finish(const GroupDev &g, GroupCtl &ctl);
+__device__ void final_finish(GroupRef g, GroupCtl &ctl);
 
 // The solve launch also ends the groups whose final pass ran in the
 // assembly launch before it (phase PH_FINAL).
@@ -1363,14 +1364,17 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
     if (ctl.phase == PH_FINAL) {
-        final_finish(B.groups[gi], ctl);
+        final_finish(group_of(B, gi), ctl);
         return;
     }
     if (ctl.phase != PH_ASSEMBLE) return;
-    const GroupDev &g = B.groups[gi];
+    GroupRef g = group_of(B, gi);
     const int tid = threadIdx.x;
-    const int nF = g.nF, nb = g.nb, N = g.N, n = g.fframeW;
+    const int nF = g.nF, nb = g.nb, N = g.N, n = g.fframeW, G = g.groupSize;
     const int shift = ctl.shift;
+    SS_GLOBAL double *deltaP = (SS_GLOBAL double *)g.deltaP, *d0 = (SS_GLOBAL double *)g.d0,
+                     *p0 = (SS_GLOBAL double *)g.p0;
+    const SS_GLOBAL double *p = as_global(g.p);
     // filter deactivation after max_filter_iterations (mainiteration.cpp:80-90)
     __shared__ int s_filter;
     if (tid == 0) {
@@ -1382,17 +1386,20 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
         s_filter = ctl.solverFilter;
         stage_time(g, ctl, FT_ASSEMBLY);
     }
-    const double *S = g.colsum;
-    const int *minPts = g.minPts;
+    const SS_GLOBAL double *S = as_global(g.colsum);
+    const SS_GLOBAL int *minPts = as_global(g.minPts);
     // The loops below load a batch of entries before they use any of it:
     // one thread per frame or knot would otherwise wait out a memory latency
     // per entry.  The additions keep their order.
     constexpr int kBatch = 8;
     // 1. per-frame errval of this shift (d_calcAllGroupErrval): a frame's
-    //    columns in batches of 32 (one round of loads for 512x512 frames)
+    //    columns in batches of 32 (one round of loads for 512x512 frames).
+    //    From the last thread on: a small group's equations are the first
+    //    waves' work, and the two run beside each other.
     constexpr int kEvBatch = 32;
-    for (int f = tid; f < nF; f += kSolveWG) {
-        const double *col = S + (size_t)f * nb * CS_N;
+    SS_GLOBAL double *errval = (SS_GLOBAL double *)g.errval + shift * nF;
+    for (int f = kSolveWG - 1 - tid; f < nF; f += kSolveWG) {
+        const SS_GLOBAL double *col = S + (size_t)f * nb * CS_N;
         double s = 0.0, c = 0.0;
         for (int b0 = 0; b0 < nb; b0 += kEvBatch) {
             double vs[kEvBatch], vc[kEvBatch];
@@ -1410,8 +1417,20 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
                 }
             }
         }
-        g.errval[shift * nF + f] = s / c;
+        errval[f] = s / c;
     }
+    // The knots' state that step 6 starts from, a batch per thread, ahead of
+    // the solve.
+    double dv0[kBatch], pv0[kBatch];
+    auto load_state = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) {
+            const int idx = min(i0 + u * kSolveWG + tid, 2 * N - 1);
+            dv0[u] = deltaP[idx];
+            pv0[u] = p[idx];
+        }
+    };
+    load_state(0);
     // 2. knot usage (d_createParameterMask) and level-0 equations
     //    (d_fillDiagonals / d_fillJTr entries, lambda extension); the knots
     //    from n on are never used.
@@ -1553,33 +1572,26 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
         __syncthreads();
     }
     // 6. d_expandResults (task_expandresults.cu:10-41) and line-search set-up
-    const int G = g.groupSize;
-    double *deltaP = g.deltaP, *d0 = g.d0, *p0 = g.p0;
-    const double *p = g.p;
-    for (int i0 = tid * kBatch; i0 < 2 * N; i0 += kSolveWG * kBatch) {
-        double dv[kBatch], pv[kBatch], xv[kBatch];
-        bool keep[kBatch];
+    for (int i0 = 0; i0 < 2 * N; i0 += kSolveWG * kBatch) {
+        if (i0 > 0) load_state(i0);
+        double xv[kBatch];
 #pragma unroll
         for (int u = 0; u < kBatch; u++) {
-            const int idx = min(i0 + u, 2 * N - 1);
-            const int j = idx >= N ? idx - N : idx;
-            const bool fixed = ((((idx + 1) - (shift * (G >> 1))) % G) == 0);
-            dv[u] = deltaP[idx];
-            pv[u] = p[idx];
-            const int jj = min(j, n - 1);
+            const int idx = min(i0 + u * kSolveWG + tid, 2 * N - 1);
+            const int j = idx >= N ? idx - N : idx, jj = min(j, n - 1);
             const bool uj = j < n && used(jj);
             const double2 x = X.get(jj);
             xv[u] = uj ? (idx >= N ? x.y : x.x) : 0.0;
-            keep[u] = fixed;
         }
 #pragma unroll
         for (int u = 0; u < kBatch; u++) {
-            const int idx = i0 + u;
+            const int idx = i0 + u * kSolveWG + tid;
             if (idx < 2 * N) {
-                const double v = keep[u] ? dv[u] : xv[u];
+                const bool fixed = ((((idx + 1) - (shift * (G >> 1))) % G) == 0);
+                const double v = fixed ? dv0[u] : xv[u];
                 deltaP[idx] = v;
                 d0[idx] = v;
-                p0[idx] = pv[u];
+                p0[idx] = pv0[u];
             }
         }
     }
@@ -1740,6 +1752,11 @@ __device__ __forceinline__ double wave_max(double x) {
     for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off, 64));
     return x;
 }
+// lane u's value, u the same in all lanes
+__device__ __forceinline__ double lane_value(double x, int u) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(x), u), hi = __builtin_amdgcn_readlane(__double2hiint(x), u);
+    return __hiloint2double(hi, lo);
+}
 __device__ __forceinline__ int wave_or(int x) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) x |= __shfl_xor(x, off, 64);
@@ -1749,25 +1766,43 @@ __device__ __forceinline__ int wave_or(int x) {
 // Sequential resolution of the candidates of frame f (reproduces the
 // reference's try / reduce / movement-threshold order) and commit.  One
 // wave per frame.
-__device__ void ls_decide_frame(const GroupDev &g, GroupCtl &ctl, int f, int K, int slot) {
+__device__ __forceinline__ void ls_decide_frame(GroupRef g, const SS_CONST GroupCtl &ctl, GroupCtl &out, int f, int K,
+                                                int slot) {
     const int nb = g.nb, N = g.N, nF = g.nF;
     const int lane = threadIdx.x;
+    const SS_GLOBAL double *d0 = as_global(g.d0) + (size_t)f * nb, *p0 = as_global(g.p0) + (size_t)f * nb;
+    const SS_GLOBAL int *minPts = as_global(g.minPts);
+    SS_GLOBAL double *errval = (SS_GLOBAL double *)g.errval + ctl.shift * nF;
+    // all that the decision and the commit read, before any of it is used
+    const int k0 = as_global(g.lsNextK)[f];
+    const double ev = errval[f];
+    const double r = g.rmult, thr = g.thr;
+    double d0x = 0.0, d0y = 0.0, p0x = 0.0, p0y = 0.0;  // the lane's first block column
     double se[kMaxCand], sn[kMaxCand];
 #pragma unroll
     for (int k = 0; k < kMaxCand; k++) se[k] = sn[k] = 0.0;
     int pres = 0;  // bit k: some column of candidate k reaches its block's min points
     double dmax = 0.0;
     for (int bb = lane; bb < nb; bb += 64) {
-        const double *ls = g.lssum + (size_t)(f * nb + bb) * 2 * kMaxCand;
+        const SS_GLOBAL d2v *ls = (const SS_GLOBAL d2v *)g.lssum + (size_t)(f * nb + bb) * kMaxCand;
+        const double dx = d0[bb], dy = d0[bb + N];
+        const double mp = (double)minPts[bb];
+        if (bb < 64) {
+            d0x = dx;
+            d0y = dy;
+            p0x = p0[bb];
+            p0y = p0[bb + N];
+        }
 #pragma unroll
         for (int k = 0; k < kMaxCand; k++) {
             if (k < K) {
-                se[k] += ls[2 * k];
-                sn[k] += ls[2 * k + 1];
-                if (ls[2 * k + 1] >= (double)g.minPts[bb]) pres |= 1 << k;
+                const d2v v = ls[k];
+                se[k] += v.x;
+                sn[k] += v.y;
+                if (v.y >= mp) pres |= 1 << k;
             }
         }
-        dmax = fmax(dmax, fmax(fabs(g.d0[f * nb + bb]), fabs(g.d0[f * nb + bb + N])));
+        dmax = fmax(dmax, fmax(fabs(dx), fabs(dy)));
     }
 #pragma unroll
     for (int k = 0; k < kMaxCand; k++) {
@@ -1780,9 +1815,6 @@ __device__ void ls_decide_frame(const GroupDev &g, GroupCtl &ctl, int f, int K, 
     dmax = wave_max(dmax);
     int fin = -1, acc = -1;
     if (lane == 0) {
-        const int shift = ctl.shift;
-        const double r = g.rmult, thr = g.thr;
-        const int k0 = g.lsNextK[f];
         double dm = reduce_pow(dmax, r, k0);
         int mk = -1, tries = 0;
         for (int kk = 0; kk < K && fin < 0; kk++) {
@@ -1803,10 +1835,10 @@ __device__ void ls_decide_frame(const GroupDev &g, GroupCtl &ctl, int f, int K, 
                         c = sn[q];
                     }
                 e /= c;
-                if (e < g.errval[shift * nF + f]) {
+                if (e < ev) {
                     acc = k;
                     fin = k;
-                    if (f == 0) g.errval[shift * nF] = e;
+                    if (f == 0) errval[0] = e;
                 } else if (!(dm > thr)) {
                     fin = k;
                 } else {
@@ -1815,35 +1847,44 @@ __device__ void ls_decide_frame(const GroupDev &g, GroupCtl &ctl, int f, int K, 
             }
         }
         g.lsMk[f] = mk;
-        atomicAdd(&ctl.tries, tries);
-        atomicAdd(&ctl.lsFramePasses, 1);
-        atomicMax(&ctl.slotRounds, slot + 1);
+        atomicAdd(&out.tries, tries);
+        atomicAdd(&out.lsFramePasses, 1);
+        atomicMax(&out.slotRounds, slot + 1);
         if (fin < 0) g.lsNextK[f] = k0 + K;
         else g.lsActive[f] = 0;
     }
     fin = __shfl(fin, 0, 64);
     acc = __shfl(acc, 0, 64);
     if (fin >= 0) {
-        const double r = g.rmult;
-        for (int t = lane; t < 2 * nb; t += 64) {
-            const int i = f * nb + (t % nb) + (t >= nb ? N : 0);
-            const double d0 = g.d0[i];
-            g.deltaP[i] = reduce_pow(d0, r, fin);
-            if (acc >= 0) g.p[i] = g.p0[i] + reduce_pow(d0, r, acc);
+        SS_GLOBAL double *deltaP = (SS_GLOBAL double *)g.deltaP + (size_t)f * nb, *p = (SS_GLOBAL double *)g.p + (size_t)f * nb;
+        for (int bb = lane; bb < nb; bb += 64) {
+            if (bb >= 64) {
+                d0x = d0[bb];
+                d0y = d0[bb + N];
+                p0x = p0[bb];
+                p0y = p0[bb + N];
+            }
+            deltaP[bb] = reduce_pow(d0x, r, fin);
+            deltaP[bb + N] = reduce_pow(d0y, r, fin);
+            if (acc >= 0) {
+                p[bb] = p0x + reduce_pow(d0x, r, acc);
+                p[bb + N] = p0y + reduce_pow(d0y, r, acc);
+            }
         }
     }
 }
 
 __global__ __launch_bounds__(64) void k_ls_decide(Batch B, int slot) {
     for (int fi = blockIdx.x; fi < B.nFrames; fi += gridDim.x) {
-        const int gi = B.frameGroup[fi];
-        GroupCtl &ctl = B.ctl[gi];
+        const int gi = as_const(B.frameGroup)[fi];
+        // the sums and flags that the decisions change are not read here
+        const SS_CONST GroupCtl &ctl = as_const(B.ctl)[gi];
         if (ctl.phase != PH_LS) continue;
-        const GroupDev &g = B.groups[gi];
+        GroupRef g = group_of(B, gi);
         if (!ls_round_runs(g, ctl, slot)) continue;
         const int f = fi - g.frameStart;
-        if (!g.lsActive[f]) continue;
-        ls_decide_frame(g, ctl, f, ls_round_k(g, ctl, slot), slot);
+        if (!as_global(g.lsActive)[f]) continue;
+        ls_decide_frame(g, ctl, B.ctl[gi], f, ls_round_k(g, ctl, slot), slot);
     }
 }
 
@@ -1856,11 +1897,24 @@ __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
     if (ctl.phase != PH_LS) return;
-    const GroupDev &g = B.groups[gi];
+    GroupRef g = group_of(B, gi);
     const int nF = g.nF;
     const int shift0 = ctl.shift, it0 = ctl.iteration;
+    // the frames' error values, 64 at a time, each added in the frames' order
+    const SS_GLOBAL double *ev = as_global(g.errval);
     int active = 0;
-    for (int f = threadIdx.x; f < nF; f += 64) active += g.lsActive[f];
+    double e0 = 0.0, e1 = 0.0;
+    for (int f0 = 0; f0 < nF; f0 += 64) {
+        const int f = min(f0 + (int)threadIdx.x, nF - 1), in = f0 + (int)threadIdx.x < nF;
+        const double v0 = ev[f], v1 = ev[f + nF];
+        active += in ? as_global(g.lsActive)[f] : 0;
+        const int m = min(64, nF - f0);
+#pragma unroll 4
+        for (int u = 0; u < m; u++) {
+            e0 += lane_value(v0, u);
+            e1 += lane_value(v1, u);
+        }
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) active += __shfl_xor(active, off, 64);
     if (active == 0 && g.rgParams && it0 <= g.maxIter) {  // output 14 (timedmainiteration.cpp:124)
@@ -1882,11 +1936,6 @@ __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
         return;
     }
     // half-iteration complete
-    double e0 = 0.0, e1 = 0.0;
-    for (int ff = 0; ff < nF; ff++) {
-        e0 += g.errval[ff];
-        e1 += g.errval[ff + nF];
-    }
     const int shift = ctl.shift;
     const int imp = (shift && e0 > e1) || (!shift && e0 < e1);
     ctl.improved &= imp;
@@ -2099,15 +2148,15 @@ __global__ __launch_bounds__(kSolveWG) void k_corr_finish(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
     if (ctl.phase != PH_CORR) return;
-    const GroupDev &g = B.groups[gi];
+    GroupRef g = group_of(B, gi);
     // read before the barriers below: thread 0 advances it afterwards
     const int it = ctl.iteration;
     double v[CR_N + 1];
 #pragma unroll
     for (int i = 0; i <= CR_N; i++) v[i] = 0.0;
     for (int c = threadIdx.x; c < g.fframeW; c += kSolveWG) {
-        for (int i = 0; i < CR_N; i++) v[i] += g.corrsum[(size_t)c * CR_N + i];
-        v[CR_N] += g.colsum[(size_t)c * CS_N + CS_SUMI];  // image over all pixels
+        for (int i = 0; i < CR_N; i++) v[i] += as_global(g.corrsum)[(size_t)c * CR_N + i];
+        v[CR_N] += as_global(g.colsum)[(size_t)c * CS_N + CS_SUMI];  // image over all pixels
     }
     __shared__ double tot[CR_N + 1];
     block_sum<CR_N + 1>(v, tot);
@@ -2267,7 +2316,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
 
 // Residual RMS and frame correlations of the final state, and the end of
 // the group.  Called by every thread of a kSolveWG workgroup.
-__device__ void final_finish(const GroupDev &g, GroupCtl &ctl) {
+__device__ void final_finish(GroupRef g, GroupCtl &ctl) {
     for (int f = threadIdx.x; f < g.nF; f += kSolveWG) {
         double s[FS_N];
         for (int i = 0; i < FS_N; i++) s[i] = 0.0;
@@ -2293,7 +2342,7 @@ __global__ __launch_bounds__(kSolveWG) void k_final_finish(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
     if (ctl.phase != PH_FINAL) return;
-    final_finish(B.groups[gi], ctl);
+    final_finish(group_of(B, gi), ctl);
 }
 
 // ---------------------------------------------------------------------------
