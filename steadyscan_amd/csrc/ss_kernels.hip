@@ -104,6 +104,20 @@ __device__ __forceinline__ const SS_CONST T *as_const(const T *p) {
 }
 __device__ __forceinline__ GroupRef group_of(const Batch &B, int gi) { return as_const(B.groups)[gi]; }
 
+// The group of frame item i; a batch of one group has no table to wait for.
+__device__ __forceinline__ int group_index(const Batch &B, const int *table, int i) {
+    return B.nGroups == 1 ? 0 : as_const(table)[i];
+}
+// The values are loaded by here, in one round: ahead of the conditions on
+// some of them that the compiler would wait for first.  (Not in the pixel
+// kernels: the registers that hold them cost the FP64 line search 5 to 10% at
+// 512x512, and the table's shortcut above as much.)
+__device__ __forceinline__ void loaded() {}
+template <typename T, typename... Rest>
+__device__ __forceinline__ void loaded(T x, Rest... rest) {
+    asm volatile("" ::"s"(x));
+    loaded(rest...);
+}
 // native vectors: their loads keep the pointer's address space
 using f2v = float __attribute__((ext_vector_type(2)));
 using f4v = float __attribute__((ext_vector_type(4)));
@@ -1363,15 +1377,17 @@ __device__ void final_finish(GroupRef g, GroupCtl &ctl);
 __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
-    if (ctl.phase == PH_FINAL) {
-        final_finish(group_of(B, gi), ctl);
+    GroupRef g = group_of(B, gi);
+    const int phase = as_const(B.ctl)[gi].phase, shift = as_const(B.ctl)[gi].shift;
+    const int nF = g.nF, nb = g.nb, N = g.N, n = g.fframeW, G = g.groupSize;
+    loaded(phase, shift, nF, nb, N, n, G, g.colsum, g.minPts, g.deltaP, g.p, g.d0, g.p0, g.errval, g.ws, g.lambda,
+           g.fracUniform, g.solverId, g.refine, g.funcTimes);
+    if (phase == PH_FINAL) {
+        final_finish(g, ctl);
         return;
     }
-    if (ctl.phase != PH_ASSEMBLE) return;
-    GroupRef g = group_of(B, gi);
+    if (phase != PH_ASSEMBLE) return;
     const int tid = threadIdx.x;
-    const int nF = g.nF, nb = g.nb, N = g.N, n = g.fframeW, G = g.groupSize;
-    const int shift = ctl.shift;
     SS_GLOBAL double *deltaP = (SS_GLOBAL double *)g.deltaP, *d0 = (SS_GLOBAL double *)g.d0,
                      *p0 = (SS_GLOBAL double *)g.p0;
     const SS_GLOBAL double *p = as_global(g.p);
@@ -1621,9 +1637,8 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
 // candidates in slot 0 (K1 after the solve, Kn when the line search goes on
 // from the previous slots) and Kn after it; no round runs past maxRounds.
 // ---------------------------------------------------------------------------
-template <typename G, typename C>
-__device__ __forceinline__ bool ls_round_runs(G &g, C &ctl, int slot) {
-    return ctl.roundsThisLS + slot < g.maxRounds;
+__device__ __forceinline__ bool ls_round_runs(GroupRef g, int roundsThisLS, int slot) {
+    return roundsThisLS + slot < g.maxRounds;
 }
 template <typename G, typename C>
 __device__ __forceinline__ int ls_round_k(G &g, C &ctl, int slot) {
@@ -1723,7 +1738,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(tune_varian
         const SS_CONST GroupCtl &ctl = as_const(B.ctl)[gi];
         if (ctl.phase != PH_LS) continue;
         GroupRef g = group_of(B, gi);
-        if (!runs_here<TI, R>(g) || g.var[TK_LS] != V || !ls_round_runs(g, ctl, slot)) continue;
+        if (!runs_here<TI, R>(g) || g.var[TK_LS] != V || !ls_round_runs(g, ctl.roundsThisLS, slot)) continue;
         const int c = item - g.itemStart, f = c / g.nb, b = c % g.nb;
         if (!as_const(g.lsActive)[f]) continue;
         int K = ls_round_k(g, ctl, slot), k0 = as_const(g.lsNextK)[f], slot0 = 0;
@@ -1774,35 +1789,40 @@ __device__ __forceinline__ void ls_decide_frame(GroupRef g, const SS_CONST Group
     const SS_GLOBAL int *minPts = as_global(g.minPts);
     SS_GLOBAL double *errval = (SS_GLOBAL double *)g.errval + ctl.shift * nF;
     // all that the decision and the commit read, before any of it is used
-    const int k0 = as_global(g.lsNextK)[f];
+    const int active = as_global(g.lsActive)[f], k0 = as_global(g.lsNextK)[f];
     const double ev = errval[f];
     const double r = g.rmult, thr = g.thr;
-    double d0x = 0.0, d0y = 0.0, p0x = 0.0, p0y = 0.0;  // the lane's first block column
+    struct Column {
+        double d0x, d0y, p0x, p0y;
+        int minPts;
+        d2v ls[kMaxCand];
+    };
+    auto column = [&](int bb) {
+        const SS_GLOBAL d2v *ls = (const SS_GLOBAL d2v *)g.lssum + (size_t)(f * nb + bb) * kMaxCand;
+        Column q{d0[bb], d0[bb + N], p0[bb], p0[bb + N], minPts[bb], {}};
+#pragma unroll
+        for (int k = 0; k < kMaxCand; k++) q.ls[k] = ls[k];
+        return q;
+    };
+    const Column q0 = column(min(lane, nb - 1));
+    asm volatile("" ::"v"(active), "v"(k0), "v"(ev), "v"(q0.p0y), "v"(q0.minPts), "v"(q0.ls[kMaxCand - 1].x));
+    if (!active) return;
     double se[kMaxCand], sn[kMaxCand];
 #pragma unroll
     for (int k = 0; k < kMaxCand; k++) se[k] = sn[k] = 0.0;
     int pres = 0;  // bit k: some column of candidate k reaches its block's min points
     double dmax = 0.0;
     for (int bb = lane; bb < nb; bb += 64) {
-        const SS_GLOBAL d2v *ls = (const SS_GLOBAL d2v *)g.lssum + (size_t)(f * nb + bb) * kMaxCand;
-        const double dx = d0[bb], dy = d0[bb + N];
-        const double mp = (double)minPts[bb];
-        if (bb < 64) {
-            d0x = dx;
-            d0y = dy;
-            p0x = p0[bb];
-            p0y = p0[bb + N];
-        }
+        const Column q = bb < 64 ? q0 : column(bb);
 #pragma unroll
         for (int k = 0; k < kMaxCand; k++) {
             if (k < K) {
-                const d2v v = ls[k];
-                se[k] += v.x;
-                sn[k] += v.y;
-                if (v.y >= mp) pres |= 1 << k;
+                se[k] += q.ls[k].x;
+                sn[k] += q.ls[k].y;
+                if (q.ls[k].y >= (double)q.minPts) pres |= 1 << k;
             }
         }
-        dmax = fmax(dmax, fmax(fabs(dx), fabs(dy)));
+        dmax = fmax(dmax, fmax(fabs(q.d0x), fabs(q.d0y)));
     }
 #pragma unroll
     for (int k = 0; k < kMaxCand; k++) {
@@ -1858,6 +1878,7 @@ __device__ __forceinline__ void ls_decide_frame(GroupRef g, const SS_CONST Group
     if (fin >= 0) {
         SS_GLOBAL double *deltaP = (SS_GLOBAL double *)g.deltaP + (size_t)f * nb, *p = (SS_GLOBAL double *)g.p + (size_t)f * nb;
         for (int bb = lane; bb < nb; bb += 64) {
+            double d0x = q0.d0x, d0y = q0.d0y, p0x = q0.p0x, p0y = q0.p0y;
             if (bb >= 64) {
                 d0x = d0[bb];
                 d0y = d0[bb + N];
@@ -1876,15 +1897,15 @@ __device__ __forceinline__ void ls_decide_frame(GroupRef g, const SS_CONST Group
 
 __global__ __launch_bounds__(64) void k_ls_decide(Batch B, int slot) {
     for (int fi = blockIdx.x; fi < B.nFrames; fi += gridDim.x) {
-        const int gi = as_const(B.frameGroup)[fi];
+        const int gi = group_index(B, B.frameGroup, fi);
         // the sums and flags that the decisions change are not read here
         const SS_CONST GroupCtl &ctl = as_const(B.ctl)[gi];
-        if (ctl.phase != PH_LS) continue;
         GroupRef g = group_of(B, gi);
-        if (!ls_round_runs(g, ctl, slot)) continue;
-        const int f = fi - g.frameStart;
-        if (!as_global(g.lsActive)[f]) continue;
-        ls_decide_frame(g, ctl, B.ctl[gi], f, ls_round_k(g, ctl, slot), slot);
+        const int phase = ctl.phase, rounds = ctl.roundsThisLS, K = ls_round_k(g, ctl, slot);
+        loaded(phase, rounds, K, ctl.shift, g.maxRounds, g.frameStart, g.nb, g.N, g.nF, g.lsActive, g.lsNextK, g.lssum,
+               g.errval, g.d0, g.p0, g.minPts);
+        if (phase != PH_LS || !ls_round_runs(g, rounds, slot)) continue;
+        ls_decide_frame(g, ctl, B.ctl[gi], fi - g.frameStart, K, slot);
     }
 }
 
@@ -1896,10 +1917,15 @@ __global__ __launch_bounds__(64) void k_ls_decide(Batch B, int slot) {
 __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
-    if (ctl.phase != PH_LS) return;
     GroupRef g = group_of(B, gi);
-    const int nF = g.nF;
-    const int shift0 = ctl.shift, it0 = ctl.iteration;
+    const SS_CONST GroupCtl &was = as_const(B.ctl)[gi];  // before this launch
+    const int nF = g.nF, phase = was.phase, shift = was.shift, it0 = was.iteration;
+    const int improved = was.improved, nFilterIterations = was.nFilterIterations, slotRounds = was.slotRounds;
+    const int rounds = was.rounds + slotRounds, roundsThisLS = was.roundsThisLS + slotRounds;
+    const int halfIterations = was.halfIterations + 1;
+    loaded(nF, phase, shift, it0, improved, nFilterIterations, rounds, roundsThisLS, halfIterations, g.Kn, g.maxRounds,
+           g.errval, g.lsActive, g.rgParams, g.maxIter, g.funcTimes);
+    if (phase != PH_LS) return;
     // the frames' error values, 64 at a time, each added in the frames' order
     const SS_GLOBAL double *ev = as_global(g.errval);
     int active = 0;
@@ -1919,33 +1945,32 @@ __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
     for (int off = 32; off > 0; off >>= 1) active += __shfl_xor(active, off, 64);
     if (active == 0 && g.rgParams && it0 <= g.maxIter) {  // output 14 (timedmainiteration.cpp:124)
         const int P = 2 * g.N;
-        double *dst = g.rgParams + (size_t)P * (size_t)(shift0 + 2 * (it0 - 1));
+        double *dst = g.rgParams + (size_t)P * (size_t)(shift + 2 * (it0 - 1));
         for (int i = threadIdx.x; i < P; i += 64) dst[i] = g.p[i];
     }
     if (threadIdx.x != 0) return;
     stage_time(g, ctl, FT_LINESEARCH);
-    ctl.rounds += ctl.slotRounds;
-    ctl.roundsThisLS += ctl.slotRounds;
+    ctl.rounds = rounds;
+    ctl.roundsThisLS = roundsThisLS;
     ctl.slotRounds = 0;
     if (active > 0) {
         ctl.K = g.Kn;
-        if (ctl.roundsThisLS >= g.maxRounds) {
+        if (roundsThisLS >= g.maxRounds) {
             ctl.error = 4;  // SS_ERR_NUMERICAL
             ctl.phase = PH_ERROR;
         }
         return;
     }
     // half-iteration complete
-    const int shift = ctl.shift;
-    const int imp = (shift && e0 > e1) || (!shift && e0 < e1);
-    ctl.improved &= imp;
-    ctl.halfIterations++;
+    const int imp = improved & ((shift && e0 > e1) || (!shift && e0 < e1));
+    ctl.improved = imp;
+    ctl.halfIterations = halfIterations;
     if (shift == 0) {
         ctl.shift = 1;
         ctl.phase = PH_ASSEMBLE;
         return;
     }
-    if (!ctl.improved && ctl.nFilterIterations != 0) {
+    if (!imp && nFilterIterations != 0) {
         ctl.solverFilter = 0;
         ctl.nFilterIterations = 0;
         ctl.improved = 1;  // run this iteration again without the filter
@@ -1953,7 +1978,7 @@ __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
         ctl.phase = PH_ASSEMBLE;
         return;
     }
-    ctl.iterImproved = ctl.improved;
+    ctl.iterImproved = imp;
     ctl.phase = PH_CORR;
 }
 
@@ -2147,10 +2172,15 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
 __global__ __launch_bounds__(kSolveWG) void k_corr_finish(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
-    if (ctl.phase != PH_CORR) return;
     GroupRef g = group_of(B, gi);
-    // read before the barriers below: thread 0 advances it afterwards
-    const int it = ctl.iteration;
+    // read ahead: thread 0 advances them
+    const SS_CONST GroupCtl &was = as_const(B.ctl)[gi];
+    const int phase = was.phase, it = was.iteration, filterID = was.filterID, iterImproved = was.iterImproved;
+    const double correlation = was.correlation;
+    loaded(phase, it, filterID, iterImproved, g.fframeW, g.corrsum, g.colsum, g.N, g.nF, g.nb, g.fcIter, g.maxIter,
+           g.allParams, g.p, g.pLast, g.funcTimes, g.iterCorr, g.iterTimes, g.iterErr, correlation, g.cit, g.fct,
+           g.halt);
+    if (phase != PH_CORR) return;
     double v[CR_N + 1];
 #pragma unroll
     for (int i = 0; i <= CR_N; i++) v[i] = 0.0;
@@ -2191,12 +2221,11 @@ __global__ __launch_bounds__(kSolveWG) void k_corr_finish(Batch B) {
             if (it <= g.maxIter) g.iterTimes[it - 1] = (double)(now - ctl.tIter) / g.clockHz;
             ctl.tIter = now;
         }
-        const double correlation = ctl.correlation;
         int copy = 0, save = 0;
         if (corr - correlation < g.cit) {
             ctl.retv = 0;  // CorrelationIncreaseThreshold
             ctl.phase = PH_FINAL;
-        } else if (corr - correlation < g.fct && ctl.filterID != 0) {
+        } else if (corr - correlation < g.fct && filterID != 0) {
             ctl.solverFilter = 0;
             ctl.nFilterIterations = 0;
             ctl.filterID = 0;
@@ -2209,7 +2238,7 @@ __global__ __launch_bounds__(kSolveWG) void k_corr_finish(Batch B) {
                 ctl.shift = 0;
                 ctl.phase = PH_ASSEMBLE;
             }
-        } else if (!ctl.iterImproved) {
+        } else if (!iterImproved) {
             ctl.retv = 2;  // MovementThreshold
             ctl.phase = PH_FINAL;
         } else if (g.maxIter == it) {
