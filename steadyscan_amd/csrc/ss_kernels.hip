@@ -1987,7 +1987,7 @@ __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
 // task_correlation.cu:63-99) of every frame's last-tried state; the
 // statistic of a column covers its leading run of masked rows only.
 // ---------------------------------------------------------------------------
-template <typename TI, typename R, int V, bool FAST>
+template <typename TI, typename R, int V, bool FAST, bool ONE>
 __device__ __forceinline__ void corr_column_t(GroupRef g, int c) {
     const int f = c / g.nb, b = c % g.nb;
     const int mk = as_const(g.lsMk)[f], dk = as_const(g.lsDk)[f];
@@ -1998,30 +1998,46 @@ __device__ __forceinline__ void corr_column_t(GroupRef g, int c) {
     const Template<R, FAST> T(g);
     GeoRun<R, FAST> geo(g, b);
     const int last = g.frameH - 1;
-    // first row outside the mask of the last-tried state: the moments cover
-    // the rows before it
+    // First row outside the mask of the last-tried state: the moments cover
+    // the rows before it.  Where a thread has at most two runs of rows (ONE),
+    // it needs no pass of its own for it: it stops at its own first row
+    // outside, keeps the moments of its first run, and takes back what lies
+    // behind the column's first row outside once all threads are through.
+    // 20 groups of 50 512x512 frames, FP64: 166 -> 148 us a launch; FP32, 24
+    // uneven groups: 126 -> 121 us.
     int firstOut = g.frameH;
     constexpr int CH = chunk_rows<R>(1, tune_variant<TK_CORR, R, V>().samples);
-    for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
-        const int rend = min(run * g.runLen + g.runLen, g.frameH);
-        geo.start(run, run * g.runLen);
-        for (int r0 = run * g.runLen; r0 < rend && r0 < firstOut; r0 += CH) {
-            R bx[CH], by[CH], f1[CH];
-            bool m[CH];
-            geo.template rows<CH>(r0, last, bx, by, f1, m);
+    const int start2 = (threadIdx.x + kWG) * g.runLen;  // the second run's first row
+    if constexpr (!ONE) {
+        for (int run = threadIdx.x; run * g.runLen < g.frameH; run += kWG) {
+            const int rend = min(run * g.runLen + g.runLen, g.frameH);
+            geo.start(run, run * g.runLen);
+            for (int r0 = run * g.runLen; r0 < rend && r0 < firstOut; r0 += CH) {
+                R bx[CH], by[CH], f1[CH];
+                bool m[CH];
+                geo.template rows<CH>(r0, last, bx, by, f1, m);
 #pragma unroll
-            for (int q = 0; q < CH; q++) {
-                const R x = km.x(bx[q], f1[q]), y = km.y(by[q], f1[q]);
-                if ((FAST || r0 + q < rend) && !(m[q] && T.inside(x, y))) firstOut = min(firstOut, r0 + q);
+                for (int q = 0; q < CH; q++) {
+                    const R x = km.x(bx[q], f1[q]), y = km.y(by[q], f1[q]);
+                    if ((FAST || r0 + q < rend) && !(m[q] && T.inside(x, y))) firstOut = min(firstOut, r0 + q);
+                }
             }
         }
+        firstOut = block_min(firstOut);
     }
-    firstOut = block_min(firstOut);
+    double first[CR_N];  // the moments of the first run
     double v[CR_N];
 #pragma unroll
-    for (int i = 0; i < CR_N; i++) v[i] = 0.0;
+    for (int i = 0; i < CR_N; i++) v[i] = first[i] = 0.0;
     walk_rows<CH, FAST>(
-        g, img, [&](int run, int r0) { geo.start(run, r0); },
+        g, img,
+        [&](int run, int r0) {
+            geo.start(run, r0);
+            if (ONE && run >= kWG) {
+#pragma unroll
+                for (int i = CR_SA; i < CR_N; i++) first[i] = v[i];
+            }
+        },
         [&](int r, int n, const Rows8<TI> &I, int off) {
             R bx[CH], by[CH], f1[CH];
             bool m[CH], mm[CH], okd[CH];
@@ -2057,6 +2073,7 @@ __device__ __forceinline__ void corr_column_t(GroupRef g, int c) {
                 const double Id = FAST || q < n ? (double)Iq : 0.0;
                 v[CR_SUMD] += (double)(mm[q] ? w : dbuf);
                 v[CR_NMASK] += mm[q] ? 1.0 : 0.0;
+                if (ONE && (FAST || q < n) && !mm[q]) firstOut = min(firstOut, r + q);
                 const bool lead = r + q < firstOut;  // rows before it are all inside the mask
                 const double a = lead ? (double)w : 0.0, bb = lead ? Id : 0.0;
                 v[CR_SA] += a;
@@ -2067,6 +2084,12 @@ __device__ __forceinline__ void corr_column_t(GroupRef g, int c) {
                 v[CR_NS] += lead ? 1.0 : 0.0;
             }
         });
+    if constexpr (ONE) {
+        firstOut = block_min(firstOut);
+        const bool none = firstOut <= (int)threadIdx.x * g.runLen, one = start2 < g.frameH && firstOut <= start2;
+#pragma unroll
+        for (int i = CR_SA; i < CR_N; i++) v[i] = none ? 0.0 : one ? first[i] : v[i];
+    }
     __shared__ double out[CR_N];
     block_sum<CR_N>(v, out);
     if (threadIdx.x < CR_N) g.corrsum[(size_t)c * CR_N + threadIdx.x] = out[threadIdx.x];
@@ -2074,8 +2097,11 @@ __device__ __forceinline__ void corr_column_t(GroupRef g, int c) {
 
 template <typename TI, typename R, int V>
 __device__ __forceinline__ void corr_column(GroupRef g, int c) {
-    if (g.fast) corr_column_t<TI, R, V, true>(g, c);
-    else corr_column_t<TI, R, V, false>(g, c);
+    const bool one = g.frameH <= 2 * kWG * g.runLen;
+    if (g.fast && one) corr_column_t<TI, R, V, true, true>(g, c);
+    else if (g.fast) corr_column_t<TI, R, V, true, false>(g, c);
+    else if (one) corr_column_t<TI, R, V, false, true>(g, c);
+    else corr_column_t<TI, R, V, false, false>(g, c);
 }
 
 template <typename TI, typename R, int V>
