@@ -218,13 +218,10 @@ ss_status ss_profile_read(ss_handle *h, int64_t *launches, double *ms, double *f
  * No reference counterpart (the reference fixes THREADS_PER_BLOCK 256,
  * cudaincludes.h:36).  The assembly, line-search and correlation kernels are
  * built in three launch variants each: (template samples a thread keeps in
- * flight, minimum waves per SIMD).  By default each batch picks them by its
- * size: variant 0, measured fastest on batches of 512x512 groups, for a
- * batch of more than 8 block columns per CU; for a smaller one (a single
- * group, say) the variants measured fastest there (more waves per SIMD for
- * the FP64 assembly and correlation, more samples in flight for the FP32
- * line search).  With tuning on, the first time a
- * handle sees a group shape (precision, mixed precision, frame element type,
+ * flight, minimum waves per SIMD).  By default every batch runs variant 0,
+ * the fastest on batches of 512x512 groups and on a single one.  With tuning
+ * on, the first time a handle sees a group shape (precision, mixed precision,
+ * frame element type,
  * frame_h, n_blocks, lines per run, geometry form, gradient form, frame-count
  * class floor(log2(n_frames))), it runs that group's first tick twice per
  * variant from the group's initial state (a warm-up pass, then a pass timed
