@@ -983,7 +983,9 @@ __device__ __forceinline__ void solve_interfaces(bool interior, const Aff &first
     // Cyclic reduction, in place: level l's equation k is that of thread
     // k * 2^l + 2^l - 1.  A thread keeps its own equation in registers and
     // leaves the others what they read of it: the inverse of B, which its
-    // back substitution takes too, A, C and d.
+    // back substitution takes too, A, C and d.  (With whole equations read
+    // from LDS and both neighbours' B inverted by every reader, the system of
+    // 96 knots took 17,000 cycles of a launch's 30,000.)
     M2 B = zero2(), Bi = zero2(), Ai = zero2(), C = zero2();
     double2 d = make_double2(0, 0);
     auto publish = [&]() {
@@ -1291,9 +1293,10 @@ constexpr int kSolveRegRows = 8;
 // bounds the launch: with equations and eliminated rows one after the other
 // per thread in memory, a launch over groups of up to 4096 knots (10 groups,
 // FP32 with refinement) took 199 us; in pieces that a wave loads side by side,
-// the next rows ahead, and the solution in LDS, 122 us; 4096 knots without
-// neighbours 131 -> 82 us; with the equations in LDS (1600 knots, FP64)
-// 45 -> 40 us.
+// the next rows ahead, and the solution in LDS, 122 us, and 105 with the
+// equations' loads in one round and the reduction in registers.  4096 knots
+// without neighbours 131 -> 82 -> 70 us; with the equations in LDS (1600
+// knots, FP64) 45 -> 40 -> 33 us; 96 knots 16.8 -> 16 -> 11 us.
 constexpr int kSolveLdsRows = 1824, kSolveLdsKnots = 4 * kSolveLdsRows;
 
 // Inlined into the solve kernel: as a called function it would save and

@@ -10,7 +10,7 @@
 // Variant 0 is the default: the values measured fastest on MI355X for batches
 // of 512x512 groups (1000 x 512x512 uint16 in FP64: line search 36.6 ms with
 // 4 samples at 5 waves against 46.0 at 4 waves and 40.0 with 8 samples at 3;
-// correlation 10.4 against 11.8 with 8 samples at 3 waves; assembly 20.6
+// correlation, then in two passes, 10.4 against 11.8 with 8 samples at 3 waves; assembly 20.6
 // against 21.2 at 3 waves.  24 uneven groups in FP32: line search 36.3 ms with
 // 4 samples at 5 waves against 37.9 with 8 at 4, correlation 8.7 against 9.4).
 // One 512x512 group of 50 frames measures the same order, so a batch of at
