@@ -144,6 +144,7 @@ struct ss_handle {
     size_t harenaBytes = 0;
     void *scratch = nullptr;  // work memory of the reconstruction
     size_t scratchBytes = 0;
+    void *hostFlag = nullptr;  // a word of pinned host memory that kernels set
     void *stack = nullptr;    // the driver's frame stack
     size_t stackBytes = 0;
     Profile prof;
@@ -1677,6 +1678,16 @@ void *handle_scratch(ss_handle *h, size_t bytes, ss_status *st) {
 
 size_t handle_scratch_held(const ss_handle *h) { return h->scratchBytes; }
 
+int *handle_host_flag(ss_handle *h, ss_status *st) {
+    *st = SS_OK;
+    if (!h->hostFlag && hipHostMalloc(&h->hostFlag, sizeof(int), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        h->hostFlag = nullptr;
+        *st = fail(h, SS_ERR_OUT_OF_MEMORY, "unable to allocate pinned host memory");
+    }
+    return (int *)h->hostFlag;
+}
+
 void *handle_raw_stream(const ss_handle *h) { return (void *)h->stream; }
 
 void *handle_stack(ss_handle *h, size_t bytes, ss_status *st) {
@@ -1794,6 +1805,7 @@ void ss_destroy(ss_handle *h) {
     if (h->arena) e = hipFree(h->arena);
     if (h->harena) e = hipHostFree(h->harena);
     if (h->scratch) e = hipFree(h->scratch);
+    if (h->hostFlag) e = hipHostFree(h->hostFlag);
     if (h->stack) e = hipFree(h->stack);
     if (h->trialTable) e = hipFree(h->trialTable);
     if (h->trialStage) e = hipHostFree(h->trialStage);

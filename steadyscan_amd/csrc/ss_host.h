@@ -20,6 +20,9 @@ hipStream_t handle_stream(const ss_handle *h);
 void *handle_scratch(ss_handle *h, size_t bytes, ss_status *st);
 // Bytes of work memory the handle holds now.
 size_t handle_scratch_held(const ss_handle *h);
+// A word of page-locked host memory, for a kernel to report to the host that
+// waits for it; nullptr on failure (st set).
+int *handle_host_flag(ss_handle *h, ss_status *st);
 // Looks up the device address of ss_resample_noalloc's static work area on
 // `device` (which must be current), once per device; later calls return the
 // first result.

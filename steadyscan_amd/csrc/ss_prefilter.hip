@@ -42,6 +42,9 @@
 namespace {
 
 constexpr int TM = 64, TN = 64, TK = 16;
+// FP64 planes of the frames that the sweep hands to the GEMMs: 32 frames of
+// 512x512, 2048 workgroups a launch
+constexpr size_t kPlaneBytes = (size_t)128 << 20;
 constexpr int kCgThreads = 1024;
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -64,6 +67,13 @@ template <> __device__ inline int16_t to_class<int16_t>(double v) {
 // ---------------------------------------------------------------------------
 // blur: both factors of the separable circular convolution in one sweep
 // ---------------------------------------------------------------------------
+constexpr int kBadNan = 1, kBadInf = 2;
+// A value's magnitude in an order of unsigned integers, NaN past infinity (of
+// doubles the upper half: a NaN with bits only in the lower one counts as an
+// infinity).
+__device__ __forceinline__ unsigned magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+__device__ __forceinline__ unsigned magnitude(double v) { return (unsigned)__double2hiint(v) & 0x7fffffffu; }
+
 constexpr int kBlurRadius = 64;  // most taps on each side of the centre
 constexpr int kBlurRows = 64, kBlurCols = 32, kBlurOut = 8;
 constexpr int kBlurMid = kBlurRows + 1;  // doubles per ring column: neighbouring columns in different banks
@@ -93,8 +103,9 @@ struct BlurAxis {
 // 8 multiply-adds (the LDS returns one wave's doubles in the time of four
 // multiply-adds per SIMD); the taps are wave-uniform and come through the
 // scalar cache.  A frame is read once, plus the halo rows of each strip
-// (through L2), and written once.  bad[f] reports a frame with an infinity
-// or a NaN, which the full convolution spreads over the whole frame.
+// (through L2), and written once.  bad[f] reports a frame with a NaN (kBadNan)
+// or an infinity (kBadInf), which the full convolution spreads over the whole
+// frame, and *anyBad, in host memory, that there is one.
 // Bound by the multiply-adds and LDS reads: 500 x 512x512 uint16 take 0.61 ms
 // at sigma 1 (10 taps a side; 1.06 ms without the loads a step ahead, 1.46
 // with the taps through vector loads) and 3.4 ms at 64 taps a side, where the
@@ -102,7 +113,8 @@ struct BlurAxis {
 // (132 KB at 64 taps a side) sets kBlurRadius.
 template <typename T>
 __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src, T *__restrict__ dst, BlurAxis Y,
-                                                       BlurAxis X, int segCols, int ring, int *__restrict__ bad) {
+                                                       BlurAxis X, int segCols, int ring, int *__restrict__ bad,
+                                                       int *__restrict__ anyBad) {
     extern __shared__ double lds[];
     const int rowsIn = kBlurRows - kBlurOut + Y.steps;  // rows of a loaded column, with the loop's padding
     const int strideIn = rowsIn | 1;                    // odd: columns start in different banks
@@ -118,7 +130,7 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src
     const int rowsUsed = kBlurRows + Y.dhi - Y.dlo;
     int next = x0 + X.dlo, slot = 0;  // next virtual column of the ring and where it goes
     int first = 0;                    // slot of virtual column x + X.dlo of the outputs at x
-    bool finite = true;
+    unsigned top = 0;       // the largest magnitude read
     // A step's columns are loaded into registers one step ahead, while the
     // step before is convolved: wave w holds columns w, w + 4, ..., rows lane,
     // lane + 64, ...  Virtual rows and columns wrap at the padded period; the
@@ -155,7 +167,7 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src
                 for (int m = 0; m < kBlurRowLoads; m++) {
                     const int r = lane + 64 * m;
                     const double v = (double)pre[k][m];
-                    if constexpr (std::is_floating_point<T>::value) finite = finite && isfinite(v);
+                    if constexpr (std::is_floating_point<T>::value) top = max(top, magnitude(pre[k][m]));
                     if (r < rowsIn) in[(wave + k * (kBlurThreads / 64)) * strideIn + r] = v;
                 }
             __syncthreads();
@@ -216,8 +228,13 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src
         first -= first >= ring ? ring : 0;
         __syncthreads();
     }
-    if constexpr (std::is_floating_point<T>::value)
-        if (!finite) atomicOr(&bad[blockIdx.y], 1);
+    if constexpr (std::is_floating_point<T>::value) {
+        const unsigned inf = magnitude((T)__builtin_inf());
+        if (top >= inf) {
+            atomicOr(&bad[blockIdx.y], top > inf ? kBadNan : kBadInf);
+            *anyBad = 1;
+        }
+    }
 }
 
 // The taps of one axis: g1[j] at circular distance j (0 <= j < S) of a period
@@ -299,16 +316,29 @@ __global__ __launch_bounds__(256) void k_circ_gemm(const double *__restrict__ sr
         }
 }
 
+// Frame blockIdx.y of a launch over frames, or over the listed ones.
+__device__ __forceinline__ size_t frame_of(const int *list, int k) { return list ? list[k] : k; }
+
+// the launch's frames, or the listed ones, as consecutive doubles
 template <typename T>
-__global__ __launch_bounds__(256) void k_to_double(const T *__restrict__ in, double *__restrict__ out, size_t n) {
+__global__ __launch_bounds__(256) void k_to_double(const T *__restrict__ in, const int *__restrict__ list,
+                                                   double *__restrict__ out, size_t np) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = (double)in[i];
+    if (i < np) out[blockIdx.y * np + i] = (double)in[frame_of(list, blockIdx.y) * np + i];
+}
+
+// ... and back
+template <typename T>
+__global__ __launch_bounds__(256) void k_from_double(const double *__restrict__ in, T *__restrict__ out,
+                                                     const int *__restrict__ list, size_t np) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < np) out[frame_of(list, blockIdx.y) * np + i] = to_class<T>(in[blockIdx.y * np + i]);
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_from_double(const double *__restrict__ in, T *__restrict__ out, size_t n) {
+__global__ __launch_bounds__(256) void k_set_nan(T *__restrict__ out, const int *__restrict__ list, size_t np) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = to_class<T>(in[i]);
+    if (i < np) out[list[blockIdx.y] * np + i] = (T)__builtin_nan("");
 }
 
 __device__ inline unsigned long long order_key(double v) {
@@ -357,11 +387,11 @@ __device__ double select_rank(const T *v, int np, int rank, int *hist, unsigned 
 // MATLAB median of each frame (NaN if the frame holds a NaN), then the
 // division data ./ median in the class's arithmetic.
 template <typename T>
-__global__ __launch_bounds__(1024) void k_median_divide(T *__restrict__ data, int np) {
+__global__ __launch_bounds__(1024) void k_median_divide(T *__restrict__ data, const int *__restrict__ list, int np) {
     __shared__ int hist[256];
     __shared__ unsigned long long s_prefix;
     __shared__ int s_rank, s_nan;
-    T *v = data + (size_t)blockIdx.x * np;
+    T *v = data + frame_of(list, blockIdx.x) * np;
     if (threadIdx.x == 0) s_nan = 0;
     __syncthreads();
     for (int i = threadIdx.x; i < np; i += blockDim.x)
@@ -828,9 +858,9 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     std::vector<double> taps1, taps2;
     const bool sweep = pregauss > 0 && blur_taps(g1, H, Y, taps1) && blur_taps(g2, W, X, taps2);
     const bool isFloat = type == SS_F64 || type == SS_F32;
-    // the GEMMs need two FP64 planes per frame (the sweep only of one frame at
-    // a time, for frames that it reports); the sweep reads and writes
-    // different buffers
+    // the GEMMs need two FP64 planes per frame (the sweep only for frames with
+    // an infinity, as many at a time as fill the chip); the sweep reads and
+    // writes different buffers
     const bool inPlace = on_device && in == out;
     const size_t planes = align256(np * 8) * 2;
     const size_t perFrame = (sweep || !(pregauss > 0) ? 0 : planes) + (on_device ? 0 : align256(np * es)) +
@@ -841,9 +871,10 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     PCHK(hipMemGetInfo(&freeB, &totalB));
     const size_t budget = std::max<size_t>((size_t)1 << 30, (freeB + ss::handle_scratch_held(h)) / 2);
     const int B = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_frames, budget / perFrame, (size_t)65535}));
+    const size_t G = !(pregauss > 0) ? 0 : !sweep ? B : !isFloat ? 0 : std::min<size_t>(B, std::max<size_t>(1, kPlaneBytes / planes));
     ss_status rc;
     const size_t tableBytes = align256(8 * (size_t)(S1 + S2)) + align256(8 * (taps1.size() + taps2.size())) +
-                              align256(4 * (size_t)B) + (sweep && isFloat ? planes : 0);
+                              align256(4 * (size_t)B) * 2 + (sweep ? planes * G : 0);
     char *base = (char *)ss::handle_scratch(h, tableBytes + perFrame * B, &rc);
     if (!base) return rc;
     hipStream_t s = ss::handle_stream(h);
@@ -855,13 +886,10 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     };
     double *dg = (double *)take(8 * (size_t)(S1 + S2));
     double *dt = (double *)take(8 * (taps1.size() + taps2.size()));
-    int *dbad = (int *)take(4 * (size_t)B);
-    double *dD = nullptr, *dT = nullptr;
-    if (pregauss > 0 && (!sweep || isFloat)) {
-        const size_t frames = sweep ? 1 : (size_t)B;
-        dD = (double *)take(np * 8 * frames);
-        dT = (double *)take(np * 8 * frames);
-    }
+    int *dbad = (int *)take(4 * (size_t)B), *dlist = (int *)take(4 * (size_t)B);
+    double *dD = G ? (double *)take(np * 8 * G) : nullptr, *dT = G ? (double *)take(np * 8 * G) : nullptr;
+    int *anyBad = nullptr;
+    if (sweep && isFloat && !(anyBad = ss::handle_host_flag(h, &rc))) return rc;
     char *dio = on_device ? nullptr : (char *)take(es * np * B);
     char *dcopy = sweep && (!on_device || inPlace) ? (char *)take(es * np * B) : nullptr;
     if (pregauss > 0) {
@@ -878,13 +906,13 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
         ring = X.dhi - X.dlo + kBlurCols;
         lds = 8 * ((size_t)kBlurCols * ((kBlurRows - kBlurOut + Y.steps) | 1) + (size_t)ring * kBlurMid);
     }
-    // nf frames of class values at work -> the same blurred, in place, by the GEMMs
-    auto gemms = [&](char *work, int nf) {
-        const size_t cnt = np * nf;
-        const dim3 g1d((unsigned)((cnt + 255) / 256));
+    const unsigned gx = (unsigned)((np + 255) / 256);
+    // nf frames of class values (or the listed ones) at `from`, blurred by the
+    // GEMMs to the same places at `work`
+    auto gemms = [&](const char *from, char *work, const int *list, int nf) {
         dispatch(type, [&](auto *tp) {
             using T = std::remove_pointer_t<decltype(tp)>;
-            hipLaunchKernelGGL(k_to_double<T>, g1d, dim3(256), 0, s, (const T *)work, dD, cnt);
+            hipLaunchKernelGGL(k_to_double<T>, dim3(gx, nf), dim3(256), 0, s, (const T *)from, list, dD, np);
         });
         hipLaunchKernelGGL(k_circ_gemm<0>, dim3((W * nf + TN - 1) / TN, (H + TM - 1) / TM, 1), dim3(256), 0, s, dD, dT,
                            dg, S1, H, W, W * nf);
@@ -892,14 +920,16 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
                            dg + S1, S2, H, W, 0);
         dispatch(type, [&](auto *tp) {
             using T = std::remove_pointer_t<decltype(tp)>;
-            hipLaunchKernelGGL(k_from_double<T>, g1d, dim3(256), 0, s, dD, (T *)work, cnt);
+            hipLaunchKernelGGL(k_from_double<T>, dim3(gx, nf), dim3(256), 0, s, dD, (T *)work, list, np);
         });
     };
-    auto median = [&](char *work, int nf) {
-        if (type == SS_F64) hipLaunchKernelGGL(k_median_divide<double>, dim3(nf), dim3(1024), 0, s, (double *)work, (int)np);
-        else hipLaunchKernelGGL(k_median_divide<float>, dim3(nf), dim3(1024), 0, s, (float *)work, (int)np);
+    auto median = [&](char *work, const int *list, int nf) {
+        if (type == SS_F64)
+            hipLaunchKernelGGL(k_median_divide<double>, dim3(nf), dim3(1024), 0, s, (double *)work, list, (int)np);
+        else
+            hipLaunchKernelGGL(k_median_divide<float>, dim3(nf), dim3(1024), 0, s, (float *)work, list, (int)np);
     };
-    std::vector<int> bad(sweep && isFloat ? B : 0);
+    std::vector<int> bad, list;
     for (int f0 = 0; f0 < n_frames; f0 += B) {
         const int nb = std::min(B, n_frames - f0);
         const size_t cnt = np * nb;
@@ -912,7 +942,10 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
                 PCHK(hipMemcpyAsync(dcopy, src, es * cnt, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
                 from = dcopy;
             }
-            if (isFloat) PCHK(hipMemsetAsync(dbad, 0, 4 * (size_t)nb, s));
+            if (isFloat) {
+                PCHK(hipMemsetAsync(dbad, 0, 4 * (size_t)nb, s));
+                *anyBad = 0;
+            }
             // one segment per strip of rows, or several (of whole column
             // blocks, each making the ring's columns before its own again)
             // where the strips do not fill the chip
@@ -925,25 +958,42 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
                 using T = std::remove_pointer_t<decltype(tp)>;
                 le = hipFuncSetAttribute((const void *)k_blur<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
                 hipLaunchKernelGGL(k_blur<T>, grid, dim3(kBlurThreads), lds, s, (const T *)from, (T *)work, Y, X, segCols,
-                                   ring, dbad);
+                                   ring, dbad, anyBad);
             });
             PCHK(le);
-            PCHK(hipGetLastError());
-            if (isFloat) {  // frames with an infinity or a NaN: the full convolution spreads it
-                PCHK(hipMemcpyAsync(bad.data(), dbad, 4 * (size_t)nb, hipMemcpyDeviceToHost, s));
-                PCHK(hipStreamSynchronize(s));
-                for (int f = 0; f < nb; f++) {
-                    if (!bad[f]) continue;
-                    PCHK(hipMemcpyAsync(work + es * np * f, from + es * np * f, es * np, hipMemcpyDeviceToDevice, s));
-                    gemms(work + es * np * f, 1);
-                }
-            }
         } else {
             if (!on_device) PCHK(hipMemcpyAsync(work, src, es * cnt, hipMemcpyHostToDevice, s));
             else if (src != dst) PCHK(hipMemcpyAsync(work, src, es * cnt, hipMemcpyDeviceToDevice, s));
-            if (pregauss > 0) gemms(work, nb);
+            if (pregauss > 0) gemms(work, work, nullptr, nb);
         }
-        if (mednorm) median(work, nb);
+        if (mednorm) median(work, nullptr, nb);
+        PCHK(hipGetLastError());
+        if (!on_device) PCHK(hipMemcpyAsync(dst, work, es * cnt, hipMemcpyDeviceToHost, s));
+        PCHK(hipStreamSynchronize(s));
+        if (!anyBad || !*(volatile int *)anyBad) continue;
+        // Frames with a NaN become NaN throughout: every output of the full
+        // convolution has it as a term.  Frames with an infinity go through the GEMMs.
+        // 500 x 512x512 float32 frames with a NaN each take 0.78 ms, with an
+        // infinity each 7.7 ms; blurred by the GEMMs one by one, 106 ms.
+        bad.resize(nb);
+        PCHK(hipMemcpy(bad.data(), dbad, 4 * (size_t)nb, hipMemcpyDeviceToHost));
+        list.clear();
+        for (int f = 0; f < nb; f++)
+            if (bad[f] & kBadNan) list.push_back(f);
+        const size_t nans = list.size();
+        for (int f = 0; f < nb; f++)
+            if (bad[f] == kBadInf) list.push_back(f);
+        PCHK(hipMemcpyAsync(dlist, list.data(), 4 * list.size(), hipMemcpyHostToDevice, s));
+        if (nans) {
+            const dim3 grid(gx, (unsigned)nans);
+            if (type == SS_F64) hipLaunchKernelGGL(k_set_nan<double>, grid, dim3(256), 0, s, (double *)work, dlist, np);
+            else hipLaunchKernelGGL(k_set_nan<float>, grid, dim3(256), 0, s, (float *)work, dlist, np);
+        }
+        for (size_t k = nans; k < list.size(); k += G) {
+            const int n = (int)std::min(G, list.size() - k);
+            gemms(from, work, dlist + k, n);
+            if (mednorm) median(work, dlist + k, n);
+        }
         PCHK(hipGetLastError());
         if (!on_device) PCHK(hipMemcpyAsync(dst, work, es * cnt, hipMemcpyDeviceToHost, s));
         PCHK(hipStreamSynchronize(s));
