@@ -45,6 +45,8 @@ constexpr int TM = 64, TN = 64, TK = 16;
 // FP64 planes of the frames that the sweep hands to the GEMMs: 32 frames of
 // 512x512, 2048 workgroups a launch
 constexpr size_t kPlaneBytes = (size_t)128 << 20;
+// most frames of a launch whose flags are cleared by the tables' upload
+constexpr int kFlagsInTab = 1024;
 constexpr int kCgThreads = 1024;
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -68,11 +70,6 @@ template <> __device__ inline int16_t to_class<int16_t>(double v) {
 // blur: both factors of the separable circular convolution in one sweep
 // ---------------------------------------------------------------------------
 constexpr int kBadNan = 1, kBadInf = 2;
-// A value's magnitude in an order of unsigned integers, NaN past infinity (of
-// doubles the upper half: a NaN with bits only in the lower one counts as an
-// infinity).
-__device__ __forceinline__ unsigned magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
-__device__ __forceinline__ unsigned magnitude(double v) { return (unsigned)__double2hiint(v) & 0x7fffffffu; }
 
 constexpr int kBlurRadius = 64;  // most taps on each side of the centre
 constexpr int kBlurRows = 64, kBlurCols = 32, kBlurOut = 8;
@@ -130,7 +127,7 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src
     const int rowsUsed = kBlurRows + Y.dhi - Y.dlo;
     int next = x0 + X.dlo, slot = 0;  // next virtual column of the ring and where it goes
     int first = 0;                    // slot of virtual column x + X.dlo of the outputs at x
-    unsigned top = 0;       // the largest magnitude read
+    bool finite = true;
     // A step's columns are loaded into registers one step ahead, while the
     // step before is convolved: wave w holds columns w, w + 4, ..., rows lane,
     // lane + 64, ...  Virtual rows and columns wrap at the padded period; the
@@ -167,7 +164,7 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src
                 for (int m = 0; m < kBlurRowLoads; m++) {
                     const int r = lane + 64 * m;
                     const double v = (double)pre[k][m];
-                    if constexpr (std::is_floating_point<T>::value) top = max(top, magnitude(pre[k][m]));
+                    if constexpr (std::is_floating_point<T>::value) finite = finite && isfinite(v);
                     if (r < rowsIn) in[(wave + k * (kBlurThreads / 64)) * strideIn + r] = v;
                 }
             __syncthreads();
@@ -228,11 +225,19 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src
         first -= first >= ring ? ring : 0;
         __syncthreads();
     }
+    // which kind, in a second look at the workgroup's own pixels: told apart in
+    // the loop, frames without any lose 10% at 56 taps a side
     if constexpr (std::is_floating_point<T>::value) {
-        const unsigned inf = magnitude((T)__builtin_inf());
-        if (top >= inf) {
-            atomicOr(&bad[blockIdx.y], top > inf ? kBadNan : kBadInf);
-            *anyBad = 1;
+        if (__syncthreads_or(!finite)) {
+            int kind = 0;
+            for (int x = x0 + wave; x < x1; x += kBlurThreads / 64) {
+                const double v = y0 + lane < H ? (double)s[(size_t)x * H + y0 + lane] : 0.0;
+                kind |= isnan(v) ? kBadNan : isinf(v) ? kBadInf : 0;
+            }
+            if (kind) {
+                atomicOr(&bad[blockIdx.y], kind);
+                *anyBad = 1;
+            }
         }
     }
 }
@@ -873,8 +878,22 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     const int B = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_frames, budget / perFrame, (size_t)65535}));
     const size_t G = !(pregauss > 0) ? 0 : !sweep ? B : !isFloat ? 0 : std::min<size_t>(B, std::max<size_t>(1, kPlaneBytes / planes));
     ss_status rc;
-    const size_t tableBytes = align256(8 * (size_t)(S1 + S2)) + align256(8 * (taps1.size() + taps2.size())) +
-                              align256(4 * (size_t)B) * 2 + (sweep ? planes * G : 0);
+    // the tables, in one upload: the sweep's taps, the whole kernels where the
+    // GEMMs may run, and the first launch's flags (0)
+    std::vector<double> tab;
+    if (sweep) {
+        tab = taps1;
+        tab.insert(tab.end(), taps2.begin(), taps2.end());
+    }
+    const size_t oG = tab.size();
+    if (G) {
+        tab.insert(tab.end(), g1.begin(), g1.end());
+        tab.insert(tab.end(), g2.begin(), g2.end());
+    }
+    const size_t oBad = tab.size();
+    const bool flagsInTab = sweep && isFloat && B <= kFlagsInTab;
+    if (flagsInTab) tab.resize(oBad + ((size_t)B + 1) / 2, 0.0);
+    const size_t tableBytes = align256(8 * tab.size()) + align256(4 * (size_t)B) * 2 + (sweep ? planes * G : 0);
     char *base = (char *)ss::handle_scratch(h, tableBytes + perFrame * B, &rc);
     if (!base) return rc;
     hipStream_t s = ss::handle_stream(h);
@@ -884,25 +903,20 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
         off += align256(bytes);
         return (void *)p;
     };
-    double *dg = (double *)take(8 * (size_t)(S1 + S2));
-    double *dt = (double *)take(8 * (taps1.size() + taps2.size()));
+    double *dtab = (double *)take(8 * tab.size()), *dg = dtab + oG;
     int *dbad = (int *)take(4 * (size_t)B), *dlist = (int *)take(4 * (size_t)B);
+    if (flagsInTab) dbad = (int *)(dtab + oBad);
     double *dD = G ? (double *)take(np * 8 * G) : nullptr, *dT = G ? (double *)take(np * 8 * G) : nullptr;
     int *anyBad = nullptr;
     if (sweep && isFloat && !(anyBad = ss::handle_host_flag(h, &rc))) return rc;
     char *dio = on_device ? nullptr : (char *)take(es * np * B);
     char *dcopy = sweep && (!on_device || inPlace) ? (char *)take(es * np * B) : nullptr;
-    if (pregauss > 0) {
-        PCHK(hipMemcpyAsync(dg, g1.data(), 8 * S1, hipMemcpyHostToDevice, s));
-        PCHK(hipMemcpyAsync(dg + S1, g2.data(), 8 * S2, hipMemcpyHostToDevice, s));
-    }
+    if (!tab.empty()) PCHK(hipMemcpyAsync(dtab, tab.data(), 8 * tab.size(), hipMemcpyHostToDevice, s));
     size_t lds = 0;
     int ring = 0;
     if (sweep) {
-        PCHK(hipMemcpyAsync(dt, taps1.data(), 8 * taps1.size(), hipMemcpyHostToDevice, s));
-        PCHK(hipMemcpyAsync(dt + taps1.size(), taps2.data(), 8 * taps2.size(), hipMemcpyHostToDevice, s));
-        Y.g = dt;
-        X.g = dt + taps1.size();
+        Y.g = dtab;
+        X.g = dtab + taps1.size();
         ring = X.dhi - X.dlo + kBlurCols;
         lds = 8 * ((size_t)kBlurCols * ((kBlurRows - kBlurOut + Y.steps) | 1) + (size_t)ring * kBlurMid);
     }
@@ -943,7 +957,7 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
                 from = dcopy;
             }
             if (isFloat) {
-                PCHK(hipMemsetAsync(dbad, 0, 4 * (size_t)nb, s));
+                if (f0 > 0 || !flagsInTab) PCHK(hipMemsetAsync(dbad, 0, 4 * (size_t)nb, s));
                 *anyBad = 0;
             }
             // one segment per strip of rows, or several (of whole column
