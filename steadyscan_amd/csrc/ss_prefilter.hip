@@ -44,7 +44,7 @@ namespace {
 constexpr int TM = 64, TN = 64, TK = 16;
 // FP64 planes of the frames that the sweep hands to the GEMMs: 32 frames of
 // 512x512, 2048 workgroups a launch
-constexpr size_t kPlaneBytes = (size_t)128 << 20;
+constexpr size_t kPlaneBytes = (size_t)64 << 20;
 // most frames of a launch whose flags are cleared by the tables' upload
 constexpr int kFlagsInTab = 1024;
 constexpr int kCgThreads = 1024;
@@ -267,24 +267,36 @@ bool blur_taps(const std::vector<double> &g1, int n, BlurAxis &A, std::vector<do
 // infinity or a NaN
 // ---------------------------------------------------------------------------
 // C(y, x) = sum_k A(y, k) B(k, x), 64 x 64 tile per workgroup, 4 x 4 per thread.
-// MODE 0: A(y, k) = g[(y - k) mod S] (generated), B = src (ld H, ncols columns),
-//         C = dst (ld H); the M = H, N = ncols, K = H.
-// MODE 1: frame f = blockIdx.z: A = src_f (H x W, ld H), B(k, x) = g[(x - k) mod S]
-//         (generated), C = dst_f; M = H, N = W, K = W.
-template <int MODE>
-__global__ __launch_bounds__(256) void k_circ_gemm(const double *__restrict__ src, double *__restrict__ dst,
-                                                   const double *__restrict__ g, int S, int H, int W,
-                                                   int ncols) {
+// MODE 0, the frames' columns side by side: A(y, k) = g[(y - k) mod S]
+//         (generated), B = src, the class's values (frame f's at listed
+//         place list[f]), C = dst, consecutive FP64 planes; M = H, N = W * nf,
+//         K = H.
+// MODE 1, frame blockIdx.z: A = src, its FP64 plane, B(k, x) = g[(x - k) mod S]
+//         (generated), C = dst, the class's values (at its listed place);
+//         M = H, N = W, K = W.
+// The frames are converted where they are read and written: 8 frames of
+// 48x48 take XX us a call in two launches, YY us in four.
+__device__ __forceinline__ size_t frame_of(const int *list, int f) { return list ? list[f] : f; }
+
+template <int MODE, typename TI, typename TO>
+__global__ __launch_bounds__(256) void k_circ_gemm(const TI *__restrict__ src, TO *__restrict__ dst,
+                                                   const int *__restrict__ list, const double *__restrict__ g, int S,
+                                                   int H, int W, int ncols) {
     __shared__ double As[TK][TM + 1];
     __shared__ double Bs[TK][TN + 1];
     const int M = H;
     const int N = MODE == 0 ? ncols : W;
     const int K = MODE == 0 ? H : W;
-    const size_t fo = MODE == 0 ? 0 : (size_t)blockIdx.z * H * W;
-    const double *s = src + fo;
-    double *d = dst + fo;
     const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
     const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
+    // the thread's columns of B (MODE 0) or the frame (MODE 1)
+    const TI *s[4];
+    for (int e = 0; e < 4; e++) {
+        const int x = min(n0 + (tid + 256 * e) / TK, N - 1), f = MODE == 0 ? x / W : (int)blockIdx.z;
+        s[e] = MODE == 0 ? src + (frame_of(list, f) * W + (x - f * W)) * H : src + (size_t)f * H * W;
+    }
+    TO *d = MODE == 0 ? dst : dst + frame_of(list, blockIdx.z) * H * W;
+    auto tap = [&](int at) { return g[at < 0 ? at + S : at]; };
     double acc[4][4] = {};
     for (int k0 = 0; k0 < K; k0 += TK) {
         for (int e = 0; e < 4; e++) {
@@ -292,7 +304,7 @@ __global__ __launch_bounds__(256) void k_circ_gemm(const double *__restrict__ sr
             const int m = idx % TM, kk = idx / TM;
             const int y = m0 + m, k = k0 + kk;
             double v = 0.0;
-            if (y < M && k < K) v = MODE == 0 ? g[(y - k + S) % S] : s[(size_t)k * H + y];
+            if (y < M && k < K) v = MODE == 0 ? tap(y - k) : (double)s[0][(size_t)k * H + y];
             As[kk][m] = v;
         }
         for (int e = 0; e < 4; e++) {
@@ -300,7 +312,7 @@ __global__ __launch_bounds__(256) void k_circ_gemm(const double *__restrict__ sr
             const int kk = idx % TK, n = idx / TK;
             const int k = k0 + kk, x = n0 + n;
             double v = 0.0;
-            if (k < K && x < N) v = MODE == 0 ? s[(size_t)x * H + k] : g[(x - k + S) % S];
+            if (k < K && x < N) v = MODE == 0 ? (double)s[e][k] : tap(x - k);
             Bs[kk][n] = v;
         }
         __syncthreads();
@@ -317,27 +329,11 @@ __global__ __launch_bounds__(256) void k_circ_gemm(const double *__restrict__ sr
     for (int i = 0; i < 4; i++)
         for (int j = 0; j < 4; j++) {
             const int y = m0 + ty + 16 * i, x = n0 + tx + 16 * j;
-            if (y < M && x < N) d[(size_t)x * H + y] = acc[i][j];
+            if (y < M && x < N) {
+                if constexpr (MODE == 0) d[(size_t)x * H + y] = acc[i][j];
+                else d[(size_t)x * H + y] = to_class<TO>(acc[i][j]);
+            }
         }
-}
-
-// Frame blockIdx.y of a launch over frames, or over the listed ones.
-__device__ __forceinline__ size_t frame_of(const int *list, int k) { return list ? list[k] : k; }
-
-// the launch's frames, or the listed ones, as consecutive doubles
-template <typename T>
-__global__ __launch_bounds__(256) void k_to_double(const T *__restrict__ in, const int *__restrict__ list,
-                                                   double *__restrict__ out, size_t np) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < np) out[blockIdx.y * np + i] = (double)in[frame_of(list, blockIdx.y) * np + i];
-}
-
-// ... and back
-template <typename T>
-__global__ __launch_bounds__(256) void k_from_double(const double *__restrict__ in, T *__restrict__ out,
-                                                     const int *__restrict__ list, size_t np) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < np) out[frame_of(list, blockIdx.y) * np + i] = to_class<T>(in[blockIdx.y * np + i]);
 }
 
 template <typename T>
@@ -863,12 +859,12 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     std::vector<double> taps1, taps2;
     const bool sweep = pregauss > 0 && blur_taps(g1, H, Y, taps1) && blur_taps(g2, W, X, taps2);
     const bool isFloat = type == SS_F64 || type == SS_F32;
-    // the GEMMs need two FP64 planes per frame (the sweep only for frames with
+    // the GEMMs need an FP64 plane per frame (the sweep only for frames with
     // an infinity, as many at a time as fill the chip); the sweep reads and
     // writes different buffers
     const bool inPlace = on_device && in == out;
-    const size_t planes = align256(np * 8) * 2;
-    const size_t perFrame = (sweep || !(pregauss > 0) ? 0 : planes) + (on_device ? 0 : align256(np * es)) +
+    const size_t plane = align256(np * 8);
+    const size_t perFrame = (sweep || !(pregauss > 0) ? 0 : plane) + (on_device ? 0 : align256(np * es)) +
                             (sweep && (!on_device || inPlace) ? align256(np * es) : 0) + 256;
     // work memory: half of what is free on the device or already held by the handle
     PCHK(hipSetDevice(ss::handle_device(h)));
@@ -876,7 +872,7 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     PCHK(hipMemGetInfo(&freeB, &totalB));
     const size_t budget = std::max<size_t>((size_t)1 << 30, (freeB + ss::handle_scratch_held(h)) / 2);
     const int B = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_frames, budget / perFrame, (size_t)65535}));
-    const size_t G = !(pregauss > 0) ? 0 : !sweep ? B : !isFloat ? 0 : std::min<size_t>(B, std::max<size_t>(1, kPlaneBytes / planes));
+    const size_t G = !(pregauss > 0) ? 0 : !sweep ? B : !isFloat ? 0 : std::min<size_t>(B, std::max<size_t>(1, kPlaneBytes / plane));
     ss_status rc;
     // the tables, in one upload: the sweep's taps, the whole kernels where the
     // GEMMs may run, and the first launch's flags (0)
@@ -893,7 +889,7 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     const size_t oBad = tab.size();
     const bool flagsInTab = sweep && isFloat && B <= kFlagsInTab;
     if (flagsInTab) tab.resize(oBad + ((size_t)B + 1) / 2, 0.0);
-    const size_t tableBytes = align256(8 * tab.size()) + align256(4 * (size_t)B) * 2 + (sweep ? planes * G : 0);
+    const size_t tableBytes = align256(8 * tab.size()) + align256(4 * (size_t)B) * 2 + (sweep ? plane * G : 0);
     char *base = (char *)ss::handle_scratch(h, tableBytes + perFrame * B, &rc);
     if (!base) return rc;
     hipStream_t s = ss::handle_stream(h);
@@ -906,7 +902,7 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     double *dtab = (double *)take(8 * tab.size()), *dg = dtab + oG;
     int *dbad = (int *)take(4 * (size_t)B), *dlist = (int *)take(4 * (size_t)B);
     if (flagsInTab) dbad = (int *)(dtab + oBad);
-    double *dD = G ? (double *)take(np * 8 * G) : nullptr, *dT = G ? (double *)take(np * 8 * G) : nullptr;
+    double *dT = G ? (double *)take(np * 8 * G) : nullptr;
     int *anyBad = nullptr;
     if (sweep && isFloat && !(anyBad = ss::handle_host_flag(h, &rc))) return rc;
     char *dio = on_device ? nullptr : (char *)take(es * np * B);
@@ -926,15 +922,10 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     auto gemms = [&](const char *from, char *work, const int *list, int nf) {
         dispatch(type, [&](auto *tp) {
             using T = std::remove_pointer_t<decltype(tp)>;
-            hipLaunchKernelGGL(k_to_double<T>, dim3(gx, nf), dim3(256), 0, s, (const T *)from, list, dD, np);
-        });
-        hipLaunchKernelGGL(k_circ_gemm<0>, dim3((W * nf + TN - 1) / TN, (H + TM - 1) / TM, 1), dim3(256), 0, s, dD, dT,
-                           dg, S1, H, W, W * nf);
-        hipLaunchKernelGGL(k_circ_gemm<1>, dim3((W + TN - 1) / TN, (H + TM - 1) / TM, nf), dim3(256), 0, s, dT, dD,
-                           dg + S1, S2, H, W, 0);
-        dispatch(type, [&](auto *tp) {
-            using T = std::remove_pointer_t<decltype(tp)>;
-            hipLaunchKernelGGL(k_from_double<T>, dim3(gx, nf), dim3(256), 0, s, dD, (T *)work, list, np);
+            hipLaunchKernelGGL((k_circ_gemm<0, T, double>), dim3((W * nf + TN - 1) / TN, (H + TM - 1) / TM, 1), dim3(256),
+                               0, s, (const T *)from, dT, list, dg, S1, H, W, W * nf);
+            hipLaunchKernelGGL((k_circ_gemm<1, double, T>), dim3((W + TN - 1) / TN, (H + TM - 1) / TM, nf), dim3(256), 0,
+                               s, dT, (T *)work, list, dg + S1, S2, H, W, 0);
         });
     };
     auto median = [&](char *work, const int *list, int nf) {
@@ -977,8 +968,9 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
             PCHK(le);
         } else {
             if (!on_device) PCHK(hipMemcpyAsync(work, src, es * cnt, hipMemcpyHostToDevice, s));
-            else if (src != dst) PCHK(hipMemcpyAsync(work, src, es * cnt, hipMemcpyDeviceToDevice, s));
-            if (pregauss > 0) gemms(work, work, nullptr, nb);
+            else if (src != dst && !(pregauss > 0))
+                PCHK(hipMemcpyAsync(work, src, es * cnt, hipMemcpyDeviceToDevice, s));
+            if (pregauss > 0) gemms(on_device ? src : work, work, nullptr, nb);
         }
         if (mednorm) median(work, nullptr, nb);
         PCHK(hipGetLastError());
