@@ -262,6 +262,39 @@ bool blur_taps(const std::vector<double> &g1, int n, BlurAxis &A, std::vector<do
     return true;
 }
 
+// The sweep's LDS, and the columns of its ring.
+size_t blur_lds(const BlurAxis &Y, const BlurAxis &X, int &ring) {
+    ring = X.dhi - X.dlo + kBlurCols;
+    return 8 * ((size_t)kBlurCols * ((kBlurRows - kBlurOut + Y.steps) | 1) + (size_t)ring * kBlurMid);
+}
+
+// Columns of a workgroup's segment, for `strips` strips of rows: a strip may
+// be cut into segments of whole column blocks, each of which makes the
+// ring's columns before its own again, where that fills the chip.  Taken is
+// the least of a segment's multiply-adds times the workgroups that a CU's LDS
+// has to take one after the other (and a fifth for those of a launch that
+// does not fill the chip).  Cut to 4 workgroups a CU whatever the LDS holds, wide kernels made
+// their columns several times: 8 x 512x512 uint16, sigma 6, 186 -> 113 us;
+// 64 x 160x160, 178 -> 114 us.
+int blur_segment(const BlurAxis &Y, const BlurAxis &X, size_t strips, size_t lds) {
+    constexpr size_t kCus = 256, kLdsOfCu = 160 << 10;
+    auto whole = [](size_t c) { return (c + kBlurCols - 1) / kBlurCols * kBlurCols; };
+    const size_t perCu = std::max<size_t>(1, std::min<size_t>(4, kLdsOfCu / lds));
+    const size_t blocks = whole(X.n) / kBlurCols, most = std::min(blocks, std::max<size_t>(1, 4 * kCus / strips));
+    size_t best = 0, bestCost = 0;
+    for (size_t q = 1; q <= most; q++) {
+        const size_t cols = (blocks + q - 1) / q * kBlurCols, used = std::min<size_t>(cols, X.n);
+        const size_t work = whole(used + X.dhi - X.dlo) * Y.steps + whole(used) * X.steps;
+        const size_t groups = strips * ((X.n + cols - 1) / cols), rounds = (groups + kCus * perCu - 1) / (kCus * perCu);
+        const size_t cost = work * (5 * rounds + 1);
+        if (!best || cost < bestCost) {
+            best = cols;
+            bestCost = cost;
+        }
+    }
+    return (int)best;
+}
+
 // ---------------------------------------------------------------------------
 // the same convolution as GEMMs, for wider kernels and frames with an
 // infinity or a NaN
@@ -275,7 +308,7 @@ bool blur_taps(const std::vector<double> &g1, int n, BlurAxis &A, std::vector<do
 //         (generated), C = dst, the class's values (at its listed place);
 //         M = H, N = W, K = W.
 // The frames are converted where they are read and written: 8 frames of
-// 48x48 take XX us a call in two launches, YY us in four.
+// 48x48 take 50 us a call in two launches, 57 us in four.
 __device__ __forceinline__ size_t frame_of(const int *list, int f) { return list ? list[f] : f; }
 
 template <int MODE, typename TI, typename TO>
@@ -913,8 +946,7 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     if (sweep) {
         Y.g = dtab;
         X.g = dtab + taps1.size();
-        ring = X.dhi - X.dlo + kBlurCols;
-        lds = 8 * ((size_t)kBlurCols * ((kBlurRows - kBlurOut + Y.steps) | 1) + (size_t)ring * kBlurMid);
+        lds = blur_lds(Y, X, ring);
     }
     const unsigned gx = (unsigned)((np + 255) / 256);
     // nf frames of class values (or the listed ones) at `from`, blurred by the
@@ -951,12 +983,7 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
                 if (f0 > 0 || !flagsInTab) PCHK(hipMemsetAsync(dbad, 0, 4 * (size_t)nb, s));
                 *anyBad = 0;
             }
-            // one segment per strip of rows, or several (of whole column
-            // blocks, each making the ring's columns before its own again)
-            // where the strips do not fill the chip
-            const int strips = (H + kBlurRows - 1) / kBlurRows, blocks = (W + kBlurCols - 1) / kBlurCols;
-            const int segs = (int)std::max<size_t>(1, std::min<size_t>((size_t)blocks, 1024 / ((size_t)strips * nb)));
-            const int segCols = (blocks + segs - 1) / segs * kBlurCols;
+            const int strips = (H + kBlurRows - 1) / kBlurRows, segCols = blur_segment(Y, X, (size_t)strips * nb, lds);
             const dim3 grid(strips, nb, (W + segCols - 1) / segCols);
             hipError_t le = hipSuccess;
             dispatch(type, [&](auto *tp) {
