@@ -297,7 +297,7 @@ int blur_segment(const BlurAxis &Y, const BlurAxis &X, size_t strips, size_t lds
 
 // ---------------------------------------------------------------------------
 // the same convolution as GEMMs, for wider kernels and frames with an
-// infinity or a NaN
+// infinity
 // ---------------------------------------------------------------------------
 // C(y, x) = sum_k A(y, k) B(k, x), 64 x 64 tile per workgroup, 4 x 4 per thread.
 // MODE 0, the frames' columns side by side: A(y, k) = g[(y - k) mod S]
@@ -330,25 +330,29 @@ __global__ __launch_bounds__(256) void k_circ_gemm(const TI *__restrict__ src, T
     }
     TO *d = MODE == 0 ? dst : dst + frame_of(list, blockIdx.z) * H * W;
     auto tap = [&](int at) { return g[at < 0 ? at + S : at]; };
-    double acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += TK) {
+    // a step's operands are loaded into registers while the step before is computed
+    double ra[4], rb[4];
+    auto fetch = [&](int k0) {
+#pragma unroll
         for (int e = 0; e < 4; e++) {
             const int idx = tid + 256 * e;
-            const int m = idx % TM, kk = idx / TM;
-            const int y = m0 + m, k = k0 + kk;
-            double v = 0.0;
-            if (y < M && k < K) v = MODE == 0 ? tap(y - k) : (double)s[0][(size_t)k * H + y];
-            As[kk][m] = v;
+            const int y = m0 + idx % TM, ka = k0 + idx / TM, x = n0 + idx / TK, kb = k0 + idx % TK;
+            ra[e] = rb[e] = 0.0;
+            if (y < M && ka < K) ra[e] = MODE == 0 ? tap(y - ka) : (double)s[0][(size_t)ka * H + y];
+            if (x < N && kb < K) rb[e] = MODE == 0 ? (double)s[e][kb] : tap(x - kb);
         }
+    };
+    double acc[4][4] = {};
+    fetch(0);
+    for (int k0 = 0; k0 < K; k0 += TK) {
+#pragma unroll
         for (int e = 0; e < 4; e++) {
             const int idx = tid + 256 * e;
-            const int kk = idx % TK, n = idx / TK;
-            const int k = k0 + kk, x = n0 + n;
-            double v = 0.0;
-            if (k < K && x < N) v = MODE == 0 ? (double)s[e][k] : tap(x - k);
-            Bs[kk][n] = v;
+            As[idx / TM][idx % TM] = ra[e];
+            Bs[idx % TK][idx / TK] = rb[e];
         }
         __syncthreads();
+        if (k0 + TK < K) fetch(k0 + TK);
 #pragma unroll
         for (int kk = 0; kk < TK; kk++) {
             double a[4], b[4];
