@@ -262,6 +262,23 @@ bool blur_taps(const std::vector<double> &g1, int n, BlurAxis &A, std::vector<do
     return true;
 }
 
+// Whether the sweep makes no more multiply-adds for a frame than the GEMMs,
+// the padding of both included: a wide kernel's taps go round a small frame's
+// padded period and outnumber its pixels.  512 uint16 frames, sweep and GEMMs
+// (ratio of the multiply-adds): 48x48 at sigma 2 (1.4) 53 and 55 us, at sigma 6
+// (2.9) 94 and 56; 100x100 at sigma 4 (1.1) 225 and 156; 129x129 at sigma 4
+// (0.7) 367 and 322; 256 of 256x256 at sigma 6.7 (0.7) 519 and 586.  Few
+// frames favour the sweep, which is one launch: 8 of 200x48 at sigma 4 (1.2) 53
+// and 66 us, 512 of them 239 and 159.  The number of frames is left out all
+// the same, so that a frame's result does not depend on its stack.
+bool blur_by_sweep(const BlurAxis &Y, const BlurAxis &X) {
+    auto whole = [](double n, double tile) { return std::ceil(n / tile) * tile; };
+    const double rows = whole(Y.n, kBlurRows);
+    const double sweep = rows * (whole(X.n + X.dhi - X.dlo, kBlurCols) * Y.steps + whole(X.n, kBlurCols) * X.steps);
+    const double gemms = rows * ((double)X.n * whole(Y.n, TK) + whole(X.n, TN) * whole(X.n, TK));
+    return sweep <= gemms;
+}
+
 // The sweep's LDS, and the columns of its ring.
 size_t blur_lds(const BlurAxis &Y, const BlurAxis &X, int &ring) {
     ring = X.dhi - X.dlo + kBlurCols;
@@ -296,8 +313,8 @@ int blur_segment(const BlurAxis &Y, const BlurAxis &X, size_t strips, size_t lds
 }
 
 // ---------------------------------------------------------------------------
-// the same convolution as GEMMs, for wider kernels and frames with an
-// infinity
+// the same convolution as GEMMs, for wider kernels, small frames and frames
+// with an infinity
 // ---------------------------------------------------------------------------
 // C(y, x) = sum_k A(y, k) B(k, x), 64 x 64 tile per workgroup, 4 x 4 per thread.
 // MODE 0, the frames' columns side by side: A(y, k) = g[(y - k) mod S]
@@ -894,7 +911,7 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     }
     BlurAxis Y{}, X{};
     std::vector<double> taps1, taps2;
-    const bool sweep = pregauss > 0 && blur_taps(g1, H, Y, taps1) && blur_taps(g2, W, X, taps2);
+    const bool sweep = pregauss > 0 && blur_taps(g1, H, Y, taps1) && blur_taps(g2, W, X, taps2) && blur_by_sweep(Y, X);
     const bool isFloat = type == SS_F64 || type == SS_F32;
     // the GEMMs need an FP64 plane per frame (the sweep only for frames with
     // an infinity, as many at a time as fill the chip); the sweep reads and
