@@ -44,7 +44,8 @@ constexpr int kCH = 8;         // pixels per unrolled chunk
 // 1) makes the pixel loads global loads; through the generic pointers of
 // GroupDev they would be flat loads, which also wait for LDS and cannot be
 // counted apart, so that every use waits for all loads in flight.  What no
-// kernel of the launch writes (address space 4) is read by scalar loads.
+// kernel of the launch writes (address space 4) is read by scalar loads; of the
+// control blocks, the fields that the kernel itself leaves alone.
 #define SS_GLOBAL __attribute__((address_space(1)))
 #define SS_CONST __attribute__((address_space(4)))
 // a group's description in the pixel kernels, which do not write it
@@ -1381,7 +1382,9 @@ __global__ __launch_bounds__(kSolveWG) void k_solve(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
     GroupRef g = group_of(B, gi);
-    const int phase = as_const(B.ctl)[gi].phase, shift = as_const(B.ctl)[gi].shift;
+    // read ahead; this launch writes the phase
+    const SS_GLOBAL GroupCtl &was = as_global(B.ctl)[gi];
+    const int phase = was.phase, shift = was.shift;
     const int nF = g.nF, nb = g.nb, N = g.N, n = g.fframeW, G = g.groupSize;
     loaded(phase, shift, nF, nb, N, n, G, g.colsum, g.minPts, g.deltaP, g.p, g.d0, g.p0, g.errval, g.ws, g.lambda,
            g.fracUniform, g.solverId, g.refine, g.funcTimes);
@@ -1921,7 +1924,7 @@ __global__ __launch_bounds__(64) void k_ls_finish(Batch B) {
     const int gi = blockIdx.x;
     GroupCtl &ctl = B.ctl[gi];
     GroupRef g = group_of(B, gi);
-    const SS_CONST GroupCtl &was = as_const(B.ctl)[gi];  // before this launch
+    const SS_GLOBAL GroupCtl &was = as_global(B.ctl)[gi];  // read ahead; this launch writes these fields
     const int nF = g.nF, phase = was.phase, shift = was.shift, it0 = was.iteration;
     const int improved = was.improved, nFilterIterations = was.nFilterIterations, slotRounds = was.slotRounds;
     const int rounds = was.rounds + slotRounds, roundsThisLS = was.roundsThisLS + slotRounds;
@@ -2203,7 +2206,7 @@ __global__ __launch_bounds__(kSolveWG) void k_corr_finish(Batch B) {
     GroupCtl &ctl = B.ctl[gi];
     GroupRef g = group_of(B, gi);
     // read ahead: thread 0 advances them
-    const SS_CONST GroupCtl &was = as_const(B.ctl)[gi];
+    const SS_GLOBAL GroupCtl &was = as_global(B.ctl)[gi];
     const int phase = was.phase, it = was.iteration, filterID = was.filterID, iterImproved = was.iterImproved;
     const double correlation = was.correlation;
     loaded(phase, it, filterID, iterImproved, g.fframeW, g.corrsum, g.colsum, g.N, g.nF, g.nb, g.fcIter, g.maxIter,
