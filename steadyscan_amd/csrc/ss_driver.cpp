@@ -103,6 +103,7 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
     if (st) return st;
     const int nk = geom->nknots, nb = nk - 1, th = geom->template_h, tw = geom->template_w;
     const size_t nbm = (size_t)fh * nb;
+    if (nbm > INT32_MAX) return SS_ERR_INVALID_ARGUMENT;  // no group holds such a frame
     // geometry block matrices and the template gradients (steady_scan.m:166-179)
     std::vector<double> frac(nbm), bx(nbm), by(nbm);
     std::vector<uint8_t> bm(nbm);
@@ -117,14 +118,18 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         for (int iy = 0; iy < th; iy++) xg[(size_t)ix * th + iy] = T(iy, ix + 1) - T(iy, ix);
     for (int ix = 0; ix < tw; ix++)
         for (int iy = 0; iy + 1 < th; iy++) yg[(size_t)ix * th + iy] = T(iy + 1, ix) - T(iy, ix);
-    int32_t tid = 0, gid = 0;
-    st = ss_upload_template(h, th, tw, template_image, xg.data(), yg.data(), &tid);
+    // the template and geometry of this call, given back however it ends
+    struct Resident {
+        ss_handle *h;
+        int32_t tid = 0, gid = 0;
+        ~Resident() {
+            if (tid) ss_release(h, tid);
+            if (gid) ss_release(h, gid);
+        }
+    } res{h};
+    st = ss_upload_template(h, th, tw, template_image, xg.data(), yg.data(), &res.tid);
+    if (!st) st = ss_upload_geometry(h, fh, nb, frac.data(), bx.data(), by.data(), bm.data(), &res.gid);
     if (st) return st;
-    st = ss_upload_geometry(h, fh, nb, frac.data(), bx.data(), by.data(), bm.data(), &gid);
-    if (st) {
-        ss_release(h, tid);
-        return st;
-    }
     // outputs start as "not estimated" (steady_scan.m:161-163)
     for (size_t i = 0; i < (size_t)nk * n_frames; i++) out->dx_knots[i] = out->dy_knots[i] = nan;
     for (int j = 0; j < n_frames; j++) {
@@ -150,17 +155,17 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         est_dx = est_dy = zeros.data();
     }
     const size_t esz = elem_size(type), rawPix = (size_t)geom->nlines * geom->linewidth, rawFrame = rawPix * esz;
-    // the raw pixel of every block-matrix element: a block lists its pixels
-    // column by column (steady_scan.m:229-234, 601-613) of the cropped image
-    // (steady_scan.m:830-834)
-    if (rawPix >= ss::kNoPixel) return SS_ERR_INVALID_ARGUMENT;
+    // the pixel of every block-matrix element, counted from the cropped
+    // image's first one (steady_scan.m:830-834): a block lists its pixels
+    // column by column (steady_scan.m:229-234, 601-613)
+    const size_t crop0 = (size_t)geom->cropping[0] * geom->nlines + geom->cropping[2];
     std::vector<uint32_t> at(nbm, ss::kNoPixel);
     {
         std::vector<size_t> fill(nb, 0);
         for (int j = 0; j < Wc; j++)
             for (int i = 0; i < Hc; i++) {
                 const int b = knot[(size_t)j * Hc + i] - 1;
-                at[(size_t)b * fh + fill[b]++] = (uint32_t)((size_t)(j + geom->cropping[0]) * geom->nlines + (i + geom->cropping[2]));
+                at[(size_t)b * fh + fill[b]++] = (uint32_t)((size_t)j * geom->nlines + i);
             }
     }
     // Device memory of the stack: the table, the used flags, the packed
@@ -173,12 +178,7 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
     const size_t oUsed = al(nbm * sizeof(uint32_t)), oPacked = oUsed + al(cols), oMask = oPacked + al(nbm * esz * n_frames),
                  oRaw = oMask + al(cols * fh);
     char *dev = (char *)ss::handle_stack(h, oRaw + rawFrame * piece, &st);
-    auto release = [&] {
-        ss_release(h, tid);
-        ss_release(h, gid);
-        return st;
-    };
-    if (st) return release();
+    if (st) return st;
     void *stream = ss::handle_raw_stream(h);
     st = ss::handle_upload(h, dev, at.data(), nbm * sizeof(uint32_t));
     for (int f0 = 0; f0 < n_frames && !st; f0 += piece) {
@@ -188,11 +188,11 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         // a frame's result does not depend on its set, so the stack is filtered once
         if (!st && (ds->pregauss > 0 || ds->mednorm))
             st = ss_prefilter(h, type, dev + oRaw, dev + oRaw, geom->nlines, geom->linewidth, n, ds->pregauss, ds->mednorm, 1);
-        if (!st && ss::pack_frames(stream, (const uint32_t *)dev, (int)nbm, (int)esz, dev + oRaw, rawPix, n,
+        if (!st && ss::pack_frames(stream, (const uint32_t *)dev, (int)nbm, (int)esz, dev + oRaw + crop0 * esz, rawPix, n,
                                    dev + oPacked + nbm * esz * f0))
             st = SS_ERR_DEVICE;
     }
-    if (st) return release();
+    if (st) return st;
     std::vector<ss_group_in> gin(nsets);
     std::vector<ss_settings> gs(nsets, *s);
     std::vector<ss_group_out> gout(nsets);
@@ -210,8 +210,8 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         g.group_size = nb * ds->frame_groupsize;
         g.template_h = th;
         g.template_w = tw;
-        g.template_id = tid;
-        g.geometry_id = gid;
+        g.template_id = res.tid;
+        g.geometry_id = res.gid;
         g.data_type = type;
         g.data = dev + oPacked + nbm * esz * start[i];
         g.data_on_device = 1;
@@ -236,7 +236,7 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
     std::vector<uint8_t> usedAll(cols);
     if (!st && ss::used_blocks(stream, (const uint8_t *)dev + oMask, fh, (int)cols, (uint8_t *)dev + oUsed)) st = SS_ERR_DEVICE;
     if (!st) st = ss::handle_download(h, usedAll.data(), dev + oUsed, cols);
-    if (release()) return st;
+    if (st) return st;
     // unpacking and success tests (steady_scan.m:246-284)
     for (int i = 0; i < nsets; i++) {
         for (int sj = 0; sj + 1 < nset[i]; sj++) {

@@ -11,8 +11,8 @@
 namespace ss {
 
 // n block matrices (nbm elements of esz bytes each) from raw frames of rawPix
-// elements, through the table `at` (the raw pixel of every element, kNoPixel
-// where the block is shorter: 0).
+// elements, through the table `at` (the pixel of every element, counted from
+// `frames`, kNoPixel where the block is shorter: 0).
 constexpr uint32_t kNoPixel = ~0u;
 int pack_frames(void *stream, const uint32_t *at, int nbm, int esz, const void *frames, size_t rawPix, int n, void *out);
 // used[c] = 1 when column c (fh bytes) of mask has a nonzero byte.
