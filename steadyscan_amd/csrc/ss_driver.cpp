@@ -118,13 +118,14 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         for (int iy = 0; iy < th; iy++) xg[(size_t)ix * th + iy] = T(iy, ix + 1) - T(iy, ix);
     for (int ix = 0; ix < tw; ix++)
         for (int iy = 0; iy + 1 < th; iy++) yg[(size_t)ix * th + iy] = T(iy + 1, ix) - T(iy, ix);
-    // the template and geometry of this call, given back however it ends
+    // the template, geometry and stack of this call, given back however it ends
     struct Resident {
         ss_handle *h;
         int32_t tid = 0, gid = 0;
         ~Resident() {
             if (tid) ss_release(h, tid);
             if (gid) ss_release(h, gid);
+            ss::handle_stack_done(h);
         }
     } res{h};
     st = ss_upload_template(h, th, tw, template_image, xg.data(), yg.data(), &res.tid);

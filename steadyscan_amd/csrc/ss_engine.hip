@@ -147,6 +147,7 @@ struct ss_handle {
     void *hostFlag = nullptr;  // a word of pinned host memory that kernels set
     void *stack = nullptr;    // the driver's frame stack
     size_t stackBytes = 0;
+    bool stackInUse = false;
     Profile prof;
     // the tick's launches, captured once per group table and replayed
     bool useGraph = true;
@@ -246,6 +247,25 @@ struct Arena {
     }
 };
 
+void free_idle(ss_handle *h, void *&mem, size_t &bytes) {
+    (void)hipStreamSynchronize(h->stream);
+    (void)hipFree(mem);
+    mem = nullptr;
+    bytes = 0;
+}
+
+// Device memory for a batch or for work.  The driver's stack, idle between its
+// calls, is given back where it is what is missing.
+hipError_t alloc_device(ss_handle *h, void **mem, size_t bytes) {
+    hipError_t e = hipMalloc(mem, bytes);
+    if (e != hipSuccess && h->stack && !h->stackInUse) {
+        (void)hipGetLastError();
+        free_idle(h, h->stack, h->stackBytes);
+        e = hipMalloc(mem, bytes);
+    }
+    return e;
+}
+
 ss_status ensure_arena(ss_handle *h, size_t bytes, size_t hostBytes) {
     if (h->arenaBytes < bytes) {
         if (h->arena) {
@@ -254,7 +274,7 @@ ss_status ensure_arena(ss_handle *h, size_t bytes, size_t hostBytes) {
             h->arena = nullptr;
             h->arenaBytes = 0;
         }
-        hipError_t e = hipMalloc(&h->arena, bytes);
+        hipError_t e = alloc_device(h, &h->arena, bytes);
         if (e != hipSuccess) return fail(h, SS_ERR_OUT_OF_MEMORY, "unable to allocate device memory");
         h->arenaBytes = bytes;
     }
@@ -1665,7 +1685,7 @@ void *handle_scratch(ss_handle *h, size_t bytes, ss_status *st) {
         h->scratch = nullptr;
         h->scratchBytes = 0;
     }
-    hipError_t e = hipMalloc(&h->scratch, bytes);
+    hipError_t e = alloc_device(h, &h->scratch, bytes);
     if (e != hipSuccess) {
         h->scratch = nullptr;
         *st = fail(h, e == hipErrorOutOfMemory ? SS_ERR_OUT_OF_MEMORY : SS_ERR_DEVICE,
@@ -1692,23 +1712,28 @@ void *handle_raw_stream(const ss_handle *h) { return (void *)h->stream; }
 
 void *handle_stack(ss_handle *h, size_t bytes, ss_status *st) {
     *st = SS_OK;
-    if (h->stackBytes >= bytes) return h->stack;
     (void)hipSetDevice(h->device);
-    if (h->stack) {
-        (void)hipStreamSynchronize(h->stream);
-        (void)hipFree(h->stack);
-        h->stack = nullptr;
-        h->stackBytes = 0;
+    if (h->stackBytes < bytes) {
+        if (h->stack) free_idle(h, h->stack, h->stackBytes);
+        hipError_t e = hipMalloc(&h->stack, bytes);
+        if (e != hipSuccess && h->arena) {  // no batch runs here: the last one's memory may be what is missing
+            (void)hipGetLastError();
+            free_idle(h, h->arena, h->arenaBytes);
+            e = hipMalloc(&h->stack, bytes);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            h->stack = nullptr;
+            *st = fail(h, SS_ERR_OUT_OF_MEMORY, "unable to allocate device memory for the frame stack");
+            return nullptr;
+        }
+        h->stackBytes = bytes;
     }
-    if (hipMalloc(&h->stack, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        h->stack = nullptr;
-        *st = fail(h, SS_ERR_OUT_OF_MEMORY, "unable to allocate device memory for the frame stack");
-        return nullptr;
-    }
-    h->stackBytes = bytes;
+    h->stackInUse = true;
     return h->stack;
 }
+
+void handle_stack_done(ss_handle *h) { h->stackInUse = false; }
 
 ss_status handle_upload(ss_handle *h, void *dst, const void *src, size_t bytes) {
     HIPCHK(hipSetDevice(h->device));

@@ -18,9 +18,12 @@ int pack_frames(void *stream, const uint32_t *at, int nbm, int esz, const void *
 // used[c] = 1 when column c (fh bytes) of mask has a nonzero byte.
 int used_blocks(void *stream, const uint8_t *mask, int fh, int cols, uint8_t *used);
 
-// The driver's device memory of at least `bytes`, kept by the handle across
-// calls (grown on demand, freed by ss_destroy); nullptr on failure (st set).
+// The driver's device memory of at least `bytes`, in use until
+// handle_stack_done; nullptr on failure (st set).  Kept by the handle across
+// calls (grown on demand, freed by ss_destroy) as the batches' memory is, but
+// either is given back for the other where the device does not hold both.
 void *handle_stack(ss_handle *h, size_t bytes, ss_status *st);
+void handle_stack_done(ss_handle *h);
 // The handle's stream, as pack_frames takes it.
 void *handle_raw_stream(const ss_handle *h);
 // Host memory to the device through the handle's page-locked staging, which

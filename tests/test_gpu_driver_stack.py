@@ -1,11 +1,16 @@
 """The driver's frame stack on the device: recordings longer than a piece of
 the upload (256 MiB) and than its staging (two halves of 32 MiB), and raw
-frames of more pixels than 32 bits count, of which the cropping leaves a few."""
+frames of more pixels than 32 bits count, of which the cropping leaves a few,
+and a device that holds the stack or a batch, not both."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import steadyscan_amd as ssa
 from steadyscan_amd import workloads as W
+
+from devbuf import DeviceBuffer
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +55,31 @@ def test_wide_raw_frames(handle):
     for out, k in ((got["dx_knots"], "knots_x"), (got["dy_knots"], "knots_y")):
         assert np.isfinite(out[:, 0]).all() and np.array_equal(out[:, 0], r[k].reshape(n, 2)[0])
     assert (got["dx_knots"][:, 0] > 0).all()
+
+
+def test_stack_and_batch_in_turn():
+    """A call of the driver and a batch of about 1.2 GiB each, with 2 GiB of
+    the device left: either runs after the other."""
+    h, n, per_set = 256, 6200, 310
+    T = W.make_template(h, h, 100, (2.0, 6.0), offset=10.0, seed=35)
+    dx, dy = W.make_motion(per_set, h, 0.05, 0.0, (1.5, 1.0), seed=36)
+    part = W.make_frames(T, dx, dy, h, h, np.uint16, True, seed=37)
+    fr = np.asfortranarray(np.broadcast_to(part[:, :, None, :], (h, h, n // per_set, per_set)).reshape((h, h, n)))
+    hd = ssa.Handle(0)
+    a = W.group_args(T, part, ssa.init_settings(h, h, T.shape, nknots=17), max_iter=2)
+    calls = [dict(a, bmData=np.asfortranarray(np.tile(a["bmData"], (1, 31))), nsetframes=31 * per_set,
+                  est_dx_knots=np.zeros((17, 31 * per_set)), est_dy_knots=np.zeros((17, 31 * per_set)))]
+    kw = dict(nknots=17, min_frames_per_set=2, handle=hd, max_iter=2)
+    ssa.estimate_displacements(fr[:, :, :8], T, frames_per_set=8, **kw)  # the kernels' own memory
+    hip = DeviceBuffer(1 << 20)._hip
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    ballast = DeviceBuffer(free.value - (2 << 30))
+    try:
+        for _ in range(2):
+            est = ssa.estimate_displacements(fr, T, frames_per_set=per_set, **kw)
+            assert np.isfinite(est["dx_knots"][:, :-1]).all()
+            assert np.isfinite(ssa.align_groups(calls, handle=hd, with_mask=False)[0]["frame_corr"]).all()
+    finally:
+        ballast.free()
+        hd.close()
