@@ -169,6 +169,10 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
                 at[(size_t)b * fh + fill[b]++] = (uint32_t)((size_t)j * geom->nlines + i);
             }
     }
+    // FP64 frames in precision 'S' are aligned as floats, as a group's host frames are
+    const bool toFloat = type == SS_F64 && s->precision == 'S';
+    const ss_dtype ptype = toFloat ? SS_F32 : type;
+    const size_t psz = elem_size(ptype);
     // Device memory of the stack: the table, the used flags, the packed
     // frames (a set's are consecutive, its last one the next set's first),
     // the sets' masks, and a piece of raw frames to upload, filter and pack.
@@ -176,7 +180,7 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
     for (int n : nset) cols += (size_t)n * nb;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const int piece = (int)std::max<size_t>(1, std::min<size_t>(n_frames, ((size_t)256 << 20) / rawFrame));
-    const size_t oUsed = al(nbm * sizeof(uint32_t)), oPacked = oUsed + al(cols), oMask = oPacked + al(nbm * esz * n_frames),
+    const size_t oUsed = al(nbm * sizeof(uint32_t)), oPacked = oUsed + al(cols), oMask = oPacked + al(nbm * psz * n_frames),
                  oRaw = oMask + al(cols * fh);
     char *dev = (char *)ss::handle_stack(h, oRaw + rawFrame * piece, &st);
     if (st) return st;
@@ -189,8 +193,8 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         // a frame's result does not depend on its set, so the stack is filtered once
         if (!st && (ds->pregauss > 0 || ds->mednorm))
             st = ss_prefilter(h, type, dev + oRaw, dev + oRaw, geom->nlines, geom->linewidth, n, ds->pregauss, ds->mednorm, 1);
-        if (!st && ss::pack_frames(stream, (const uint32_t *)dev, (int)nbm, (int)esz, dev + oRaw + crop0 * esz, rawPix, n,
-                                   dev + oPacked + nbm * esz * f0))
+        if (!st && ss::pack_frames(stream, (const uint32_t *)dev, (int)nbm, (int)esz, toFloat, dev + oRaw + crop0 * esz, rawPix, n,
+                                   dev + oPacked + nbm * psz * f0))
             st = SS_ERR_DEVICE;
     }
     if (st) return st;
@@ -213,8 +217,8 @@ extern "C" ss_status ss_estimate_displacements(ss_handle *h, const ss_geometry_d
         g.template_w = tw;
         g.template_id = res.tid;
         g.geometry_id = res.gid;
-        g.data_type = type;
-        g.data = dev + oPacked + nbm * esz * start[i];
+        g.data_type = ptype;
+        g.data = dev + oPacked + nbm * psz * start[i];
         g.data_on_device = 1;
         g.init_x = est_dx;
         g.init_y = est_dy;

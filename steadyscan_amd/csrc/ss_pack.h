@@ -12,9 +12,11 @@ namespace ss {
 
 // n block matrices (nbm elements of esz bytes each) from raw frames of rawPix
 // elements, through the table `at` (the pixel of every element, counted from
-// `frames`, kNoPixel where the block is shorter: 0).
+// `frames`, kNoPixel where the block is shorter: 0).  toFloat: the elements
+// are doubles, and floats in the block matrices.
 constexpr uint32_t kNoPixel = ~0u;
-int pack_frames(void *stream, const uint32_t *at, int nbm, int esz, const void *frames, size_t rawPix, int n, void *out);
+int pack_frames(void *stream, const uint32_t *at, int nbm, int esz, bool toFloat, const void *frames, size_t rawPix, int n,
+                void *out);
 // used[c] = 1 when column c (fh bytes) of mask has a nonzero byte.
 int used_blocks(void *stream, const uint8_t *mask, int fh, int cols, uint8_t *used);
 

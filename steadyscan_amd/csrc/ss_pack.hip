@@ -1,9 +1,10 @@
 // ss_pack.hip -- a frame stack's block matrices on the GPU: the packing of
 // estimate_displacements (steady_scan.m:229-234, image2blockmatrix,
 // steady_scan.m:601-613) and, after the alignment, which blocks of a frame
-// have a masked pixel (steady_scan.m:255).  Both only move or test bytes;
-// memory bound.
+// have a masked pixel (steady_scan.m:255).  Both only move, convert or test
+// values; memory bound.
 #include <algorithm>
+#include <type_traits>
 
 #include <hip/hip_runtime.h>
 
@@ -17,13 +18,13 @@ using ss::kNoPixel;
 // the raw pixel at[e], or 0 where the block is shorter (kNoPixel).  A block
 // lists its pixels column by column, so a wave reads runs of consecutive
 // lines and writes consecutive elements; the table stays in the L2s.
-template <typename T>
+template <typename T, typename TO>
 __global__ __launch_bounds__(256) void k_pack(const uint32_t *__restrict__ at, int nbm, const T *__restrict__ frames,
-                                              size_t rawPix, T *__restrict__ out) {
+                                              size_t rawPix, TO *__restrict__ out) {
     const size_t fo = (size_t)blockIdx.y;
     for (int e = blockIdx.x * 256 + threadIdx.x; e < nbm; e += gridDim.x * 256) {
         const uint32_t p = at[e];
-        out[fo * nbm + e] = p != kNoPixel ? frames[fo * rawPix + p] : (T)0;
+        out[fo * nbm + e] = p != kNoPixel ? (TO)frames[fo * rawPix + p] : (TO)0;
     }
 }
 
@@ -44,19 +45,23 @@ __global__ __launch_bounds__(256) void k_used(const uint8_t *__restrict__ mask, 
 
 namespace ss {
 
-int pack_frames(void *stream, const uint32_t *at, int nbm, int esz, const void *frames, size_t rawPix, int n, void *out) {
+int pack_frames(void *stream, const uint32_t *at, int nbm, int esz, bool toFloat, const void *frames, size_t rawPix, int n,
+                void *out) {
     const hipStream_t s = (hipStream_t)stream;
     const int gx = std::min((nbm + 255) / 256, 1024);
     for (int f = 0; f < n; f += 65535) {
         const dim3 grid(gx, std::min(n - f, 65535));
         const char *src = (const char *)frames + rawPix * esz * f;
-        char *dst = (char *)out + (size_t)nbm * esz * f;
-        if (esz == 8)
-            hipLaunchKernelGGL(k_pack<uint64_t>, grid, dim3(256), 0, s, at, nbm, (const uint64_t *)src, rawPix, (uint64_t *)dst);
-        else if (esz == 4)
-            hipLaunchKernelGGL(k_pack<uint32_t>, grid, dim3(256), 0, s, at, nbm, (const uint32_t *)src, rawPix, (uint32_t *)dst);
-        else
-            hipLaunchKernelGGL(k_pack<uint16_t>, grid, dim3(256), 0, s, at, nbm, (const uint16_t *)src, rawPix, (uint16_t *)dst);
+        char *dst = (char *)out + (size_t)nbm * (toFloat ? sizeof(float) : esz) * f;
+        auto launch = [&](auto *from, auto *to) {
+            using T = std::remove_pointer_t<decltype(from)>;
+            using TO = std::remove_pointer_t<decltype(to)>;
+            hipLaunchKernelGGL((k_pack<T, TO>), grid, dim3(256), 0, s, at, nbm, (const T *)src, rawPix, (TO *)dst);
+        };
+        if (toFloat) launch((double *)nullptr, (float *)nullptr);
+        else if (esz == 8) launch((uint64_t *)nullptr, (uint64_t *)nullptr);
+        else if (esz == 4) launch((uint32_t *)nullptr, (uint32_t *)nullptr);
+        else launch((uint16_t *)nullptr, (uint16_t *)nullptr);
     }
     return (int)hipGetLastError();
 }

@@ -83,3 +83,33 @@ def test_stack_and_batch_in_turn():
     finally:
         ballast.free()
         hd.close()
+
+
+def test_doubles_in_single_precision(handle):
+    """FP64 frames in precision 'S' are packed as floats, with the results of
+    the same sets as host frames, and no more than 6 bytes a pixel held."""
+    h, n = 256, 800
+    T = W.make_template(h, h, 100, (2.0, 6.0), offset=10.0, seed=45)
+    dx, dy = W.make_motion(9, h, 0.05, 0.0, (1.5, 1.0), seed=46)
+    part = W.make_frames(T, dx, dy, h, h, np.float64, True, seed=47) / 3
+    fr = np.asfortranarray(np.resize(part.transpose(2, 1, 0), (n, h, h)).transpose(2, 1, 0))
+    kw = dict(flags="S", nknots=17, frames_per_set=100, min_frames_per_set=10, max_iter=3)
+    hd = ssa.Handle(0)
+    ssa.estimate_displacements(fr[:, :, :8], T, handle=hd, **kw)
+    hip = DeviceBuffer(1 << 20)._hip
+    free = [ctypes.c_size_t(), ctypes.c_size_t()]
+    total = ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free[0]), ctypes.byref(total)) == 0
+    got = ssa.estimate_displacements(fr, T, handle=hd, **kw)
+    assert hip.hipMemGetInfo(ctypes.byref(free[1]), ctypes.byref(total)) == 0
+    hd.close()
+    held = free[0].value - free[1].value
+    print(f"{held / fr.size:.2f} bytes a pixel with the raw piece of 256 MiB", flush=True)
+    # floats and masks 5 bytes, the state of the batch (16 blocks of 4096 pixels a frame) below 1
+    assert held - (256 << 20) <= 6 * fr.size
+    geom = ssa.init_settings(h, h, T.shape, nknots=17)
+    a = W.group_args(T, fr, geom, flags="S", first=100, count=101, max_iter=3)
+    r = ssa.align_groups([dict(a, bmData=np.asfortranarray(a["bmData"]))], handle=handle)[0]
+    for out, k in (("dx_knots", "knots_x"), ("dy_knots", "knots_y")):
+        assert np.array_equal(got[out][:, 100:200].T, r[k].reshape(101, 17)[:100])
+    assert np.array_equal(got["corr"][100:200], r["frame_corr"][:100])
