@@ -241,9 +241,9 @@ typedef struct {
     int32_t samples[3][3];       /* [kernel][variant]: the variants' parameters      */
     int32_t waves[3][3];
 } ss_tuning_entry;
-/* -2 (default): variants by the size of each batch; 0, 1 or 2: use that
- * variant for every kernel, no tuning; -1: tune each new group shape.  A
- * group keeps the mode in force when it was submitted. */
+/* -2 (default) or 0: variant 0 for every kernel, no tuning; 1 or 2: that
+ * variant; -1: tune each new group shape.  A group keeps the mode in force
+ * when it was submitted. */
 ss_status ss_tuning_mode(ss_handle *h, int32_t mode);
 /* Copies up to cap of the handle's tuned shapes to out; returns how many
  * there are. */

@@ -13,9 +13,8 @@
 // correlation, then in two passes, 10.4 against 11.8 with 8 samples at 3 waves; assembly 20.6
 // against 21.2 at 3 waves.  24 uneven groups in FP32: line search 36.3 ms with
 // 4 samples at 5 waves against 37.9 with 8 at 4, correlation 8.7 against 9.4).
-// One 512x512 group of 50 frames measures the same order, so a batch of at
-// most 8 block columns per CU, whose group does not fill the chip, runs them
-// too (kSmallBatchVariant).
+// One 512x512 group of 50 frames, which does not fill the chip, measures the
+// same order.
 // The engine's autotuner (off unless asked for) times all variants on a
 // group shape's first tick and keeps the fastest per kernel.
 // A variant only changes how many rows a thread unrolls and how registers
@@ -41,9 +40,6 @@ constexpr TuneVariant kTuneTable[TK_COUNT][2][kVariants] = {
     // correlation (one sample per row; a chunk holds at most 8 rows)
     {{{4, 5}, {8, 4}, {4, 6}}, {{4, 4}, {8, 3}, {2, 4}}},
 };
-
-// [kernel][fp64]: the variant of batches of at most 8 block columns per CU
-constexpr int kSmallBatchVariant[TK_COUNT][2] = {{0, 0}, {0, 0}, {0, 0}};
 
 template <int KERNEL, typename R, int V>
 __host__ __device__ constexpr TuneVariant tune_variant() {
