@@ -925,7 +925,9 @@ extern "C" ss_status ss_prefilter(ss_handle *h, ss_dtype type, const void *in, v
     size_t freeB = 0, totalB = 0;
     PCHK(hipMemGetInfo(&freeB, &totalB));
     const size_t budget = std::max<size_t>((size_t)1 << 30, (freeB + ss::handle_scratch_held(h)) / 2);
-    const int B = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_frames, budget / perFrame, (size_t)65535}));
+    // frames of a launch: the grid's limit and, for the GEMMs, 31 bits of columns
+    const size_t most = sweep ? 65535 : std::min<size_t>(65535, (INT32_MAX - TN) / W);
+    const int B = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_frames, budget / perFrame, most}));
     const size_t G = !(pregauss > 0) ? 0 : !sweep ? B : !isFloat ? 0 : std::min<size_t>(B, std::max<size_t>(1, kPlaneBytes / plane));
     ss_status rc;
     // the tables, in one upload: the sweep's taps, the whole kernels where the
