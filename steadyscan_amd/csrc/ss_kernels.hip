@@ -23,7 +23,7 @@
 // unmasked samples, with a wait each.  Per-column partial sums are reduced
 // in registers, then across waves through LDS in FP64.  No floating-point
 // atomics: every result is run-to-run deterministic.
-// What bounds them (1000 x 512x512 uint16, FP64): VALU issue, 67-82% of the
+// What bounds them (1000 x 512x512 uint16, FP64): VALU issue, 61-80% of the
 // cycles, next to the L1's 64 bytes a cycle for the gathers.  Global instead
 // of flat loads, batched gathers, scalar loads of the group's description,
 // line-constant geometry and lane-swap reductions took the full batch's

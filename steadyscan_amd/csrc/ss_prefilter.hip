@@ -8,10 +8,13 @@
 // is separable, g2d(y, x) = g1(y) g2(x) with each factor normalised, so the
 // convolution is two circulant matrix products restricted to the H x W
 // output: T = C1 D over the rows and U = T C2^T over the columns, in FP64.
-// Up to kBlurRadius taps on each side (beyond them a tap is below 2^-64 of
-// the centre one) both run in one sweep over the frame (k_blur); a wider
-// kernel runs as FP64 tiled GEMMs whose circulant operand is generated from
-// g1/g2 on the fly.  Both agree with the FFT to FP64 rounding.
+// Up to kBlurRadius taps on each side both run in one sweep over the frame
+// (k_blur), which leaves out taps below 2^-64 of the centre one; wider kernels,
+// frames so small that a wide kernel's taps outnumber their pixels, and frames
+// with an infinity run as FP64 tiled GEMMs whose circulant operand is generated
+// from g1/g2 on the fly.  Both agree with the FFT to FP64 rounding of the
+// frame's largest value.  Of a pixel that lies a factor of 2^60 or more below
+// its neighbours only the GEMMs' result holds the far taps' terms.
 // The result takes the input's class (integer frames: rounded half away
 // from zero and saturated, NaN to 0).  Median normalisation divides each
 // frame by its median, found exactly by an 8-pass radix select on the
@@ -103,11 +106,11 @@ struct BlurAxis {
 // (through L2), and written once.  bad[f] reports a frame with a NaN (kBadNan)
 // or an infinity (kBadInf), which the full convolution spreads over the whole
 // frame, and *anyBad, in host memory, that there is one.
-// Bound by the multiply-adds and LDS reads: 500 x 512x512 uint16 take 0.61 ms
-// at sigma 1 (10 taps a side; 1.06 ms without the loads a step ahead, 1.46
-// with the taps through vector loads) and 3.4 ms at 64 taps a side, where the
-// two GEMM passes and their conversions take 10.4 ms for any sigma.  The LDS
-// (132 KB at 64 taps a side) sets kBlurRadius.
+// Bound by the multiply-adds and LDS reads: 500 x 512x512 uint16 take 0.60 ms
+// at sigma 1 (9 taps a side; 1.06 ms without the loads a step ahead, 1.46
+// with the taps through vector loads) and 3.4 ms at sigma 6.8 (64 taps a side), where
+// the two GEMMs take 8.6 ms for any sigma.  The LDS (132 KB at 64 taps a side)
+// sets kBlurRadius.
 template <typename T>
 __global__ __launch_bounds__(kBlurThreads) void k_blur(const T *__restrict__ src, T *__restrict__ dst, BlurAxis Y,
                                                        BlurAxis X, int segCols, int ring, int *__restrict__ bad,
@@ -588,8 +591,9 @@ __device__ __forceinline__ double block_sum(double v, double *sp) {
 // entries in order, then the threads as block_sum does.
 // Bound by the 10 LDS reads per entry and iteration and by the barriers of
 // the two reductions.  128 x 512x512 frames with up to 18300 missing pixels
-// and 546 iterations take 5.8 ms; with the residual in LDS too, which held
-// 8192 entries and left larger frames to a kernel in global memory, 25 ms.
+// and 546 iterations take 5.8 ms (6.0 with one loop for all lengths); with the
+// residual in LDS too, which held 8192 entries and left larger frames to a
+// kernel in global memory, 25 ms.
 constexpr int kFillK = 19;
 constexpr int kFillLds = kFillK * kCgThreads;
 constexpr unsigned kNoNbr = 0x7fffu, kHasN = 1u << 30, kHasS = 1u << 31;
@@ -728,10 +732,12 @@ __device__ __forceinline__ void fill_cg_lds(const FillChunk &C, T *__restrict__ 
 }
 
 // The same for larger regions: p of the first kFillLds entries in LDS, the
-// rest of it and the other vectors in global memory (57 bytes per entry and
-// iteration, at one CU's latency and bandwidth).  128 frames of which the
-// largest misses 20400 pixels take 14 ms; 29 ms through generic pointers with
-// p on the image grid.
+// rest of it and the other vectors in global memory, at one CU's latency and
+// bandwidth: 58 bytes per entry and iteration (neighbours, degree and flags
+// twice 9, the solution 16, the residual 24), 32 more for the direction of an
+// entry past the LDS, and its neighbours'.  128 frames of which the largest
+// misses 20400 pixels take 14 ms; 29 ms through generic pointers with p on the
+// image grid.
 template <typename T>
 __device__ __forceinline__ void fill_cg_stream(const FillChunk &C, T *__restrict__ data, Partials *sp, double *lp) {
 #pragma clang fp contract(off)

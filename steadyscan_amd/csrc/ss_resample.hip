@@ -21,14 +21,15 @@
 // gather 0.32 (its chain of dependent loads); 8.2 ms with an atomicMax per
 // corner, winners evaluated by each corner and a host-built geometry table.
 //
-// All frames of a launch share the pixel geometry; grid.y is the frame.
+// All frames of a launch share the pixel geometry; grid.y is the frame, or
+// kWinFrames of them in the winners' pass.
 // ss_resample tables each pixel's knot and fraction once per call on the GPU
 // (k_scan_table).  The work memory (tables, knots, winners and the staging of
 // host frames and host output) is the handle's, kept across calls, and
 // everything runs on the handle's stream with one synchronisation at the end
 // of the call.
 //
-// ss_resample_noalloc runs the same two passes with no allocation at all:
+// ss_resample_noalloc runs the same three passes with no allocation at all:
 // the kernels compute each pixel's geometry from the scan formulas
 // (ss_scan.h) instead of reading a table, and the knots and winner tables
 // live in a fixed static device array (kNoAllocBytes per device).
